@@ -49,7 +49,7 @@ namespace ca {
 
 // One thread per (row of the pass's query tiles, 8 elements): Dl = dY . y,
 // then the Q and dY/Z limbs of the 8 elements (one 16-byte store per plane)
-// and, per row, (-m, -Dl/Z).  The limb planes are tile-major: tile j of the
+// and, per row, (-(m + kShareShift), -Dl/Z).  The limb planes are tile-major: tile j of the
 // pass in slice bh is the block limbs[(bh * ntiles + j) * P * 32 * D ..] of
 // P planes [32 rows][D] (P = q_limb_planes<E>() + 3).  Rows past T (in the
 // last tile) are written as zeros, so the dK/dV kernel stages whole tiles
@@ -112,7 +112,8 @@ __global__ __launch_bounds__(256) void ca_bwd_prep_kernel(View Qv, const float* 
   put(QL, 3, dy, invz);
   if (c == 0) {
     // negated: the dK/dV kernel starts its S and dP' accumulators from them
-    qstat[(size_t)row * 2 + 0] = -m;
+    // (m an integer from the forward, so the sum with kShareShift is exact)
+    qstat[(size_t)row * 2 + 0] = -(m + kShareShift);
     qstat[(size_t)row * 2 + 1] = -(x * invz);
   }
 }

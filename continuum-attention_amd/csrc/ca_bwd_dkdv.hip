@@ -7,7 +7,8 @@
 // Score-tile layout: the 16x16 result of S / dP' puts slot j
 // (key 14*kb - 1 + j) in lane j of each 16-lane row and queries 4*(l/16) + r
 // in its registers, so the two neighbours of a segment sit in adjacent lanes
-// of one DPP row (row_shr / row_shl).  p = 2^(s - m) stays unnormalised and
+// of one DPP row (row_shr / row_shl).  p = 2^(s - m - kShareShift) stays
+// unnormalised (its shares come out four times as large, relative to m) and
 // dY arrives pre-scaled by 1/Z, so the weight gradient g = dY.v/Z - Dl/Z comes
 // straight out of the MFMA (its accumulator starts at -Dl/Z) and dV = W^T dY
 // is formed as w^T (dY/Z) with no per-row scaling in the kernel.
@@ -290,7 +291,7 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
           for (int r = 0; r < 4; ++r) {
             const int i = i0 + 16 * rb + 4 * g + r;
             const bool vis = !kGeneral || (key_j >= 0 && key_j <= i && i < T);
-            const float s = vis ? sacc[rb][r] : 0.f;   // s - m
+            const float s = vis ? sacc[rb][r] : 0.f;   // s - m - kShareShift
             const float gg = vis ? pacc[rb][r] : 0.f;  // g = dY.v/Z - Dl/Z
             const float p = fast_exp2(s);
             const float sl = row_shr1(s), pl = row_shr1(p), gl = row_shr1(gg);
@@ -312,7 +313,7 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
             float ds = dRv + row_shl1(dLv);
             if (kGeneral) {
               // half-token caps on the first key and the last visible key
-              const float cap = (vis && key_j == 0 ? 0.5f * p : 0.f) + (vis && key_j == i ? 0.5f * p : 0.f);
+              const float cap = (vis && key_j == 0 ? 2.0f * p : 0.f) + (vis && key_j == i ? 2.0f * p : 0.f);
               w += cap;
               ds = fmaf(cap, gg, ds);
             }

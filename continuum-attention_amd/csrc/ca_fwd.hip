@@ -180,16 +180,20 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
   }
 
   // ---- split-start state -------------------------------------------------
+  // The row shift m_ref is kept an integer, so that m_ref - kShareShift, the
+  // shift the shares' weights are relative to (seg_shares returns four times
+  // the shares of p), is exact and rescales are exact powers of two.
   float m_ref = 0.f, s_carry = 0.f, r_carry = 0.f, zsum = 0.f;
   if (wave_active) {
     if (t_b == 0) {
-      m_ref = halo_dot<D>(qreg, Ks, krs, rope_k, 0) * cl2;
-      s_carry = 0.0f;  // score of key 0 relative to m_ref
+      const float s0 = halo_dot<D>(qreg, Ks, krs, rope_k, 0) * cl2;
+      m_ref = rintf(s0);
+      s_carry = s0 - m_ref;  // score of key 0 relative to m_ref
     } else {
       const int k0 = 32 * t_b;  // <= first query of this wave, so both halo keys are visible
       s_carry = halo_dot<D>(qreg, Ks, krs, rope_k, k0) * cl2;
       const float s_prev = halo_dot<D>(qreg, Ks, krs, rope_k, k0 - 1) * cl2;
-      m_ref = fmaxf(s_carry, s_prev);
+      m_ref = rintf(fmaxf(s_carry, s_prev));
       float l_unused;
       seg_shares(s_prev, s_carry, fast_exp2(s_prev - m_ref), fast_exp2(s_carry - m_ref), l_unused,
                  r_carry);
@@ -389,7 +393,7 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
       // depends on other (possibly later) queries of the wave.
       const bool grow = mt > kLazyRescale;
       if (wave_any(grow)) {
-        const float shift = grow ? mt : 0.0f;
+        const float shift = grow ? rintf(mt) : 0.0f;
         const float alpha = grow ? fast_exp2(-shift) : 1.0f;
 #pragma unroll
         for (int mb = 0; mb < P::NMB; ++mb)
@@ -429,8 +433,8 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
         float x = Lv + r_prev;
         const int wk = kbase - 1 + r;  // weight key, its score is sl
         if constexpr (kGeneral) {
-          const float cap_last = (diag && wk == i) ? 0.5f * pl : 0.0f;  // last half-token cap
-          const float cap_first = wk == 0 ? 0.5f * pl : 0.0f;           // first half-token cap
+          const float cap_last = (diag && wk == i) ? 2.0f * pl : 0.0f;  // last half-token cap
+          const float cap_first = wk == 0 ? 2.0f * pl : 0.0f;           // first half-token cap
           x += cap_last + cap_first;
         }
         sacc[r] = x;
@@ -526,11 +530,11 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
   }
   if (h == 0) {
     if (single) {
-      stats[((size_t)bh * T + i) * 2 + 0] = m_ref;
+      stats[((size_t)bh * T + i) * 2 + 0] = m_ref - kShareShift;
       stats[((size_t)bh * T + i) * 2 + 1] = scl;
     } else {
       float* mz = part + (size_t)BH * smax * T * D + (((size_t)bh * smax + split) * T + i) * 2;
-      mz[0] = m_ref;
+      mz[0] = m_ref - kShareShift;
       mz[1] = ztot;
     }
   }
@@ -676,12 +680,14 @@ __global__ __launch_bounds__(512, (fwd16_waves_per_simd<D, E, ROPE>())) void ca_
   float m_ref = 0.f, s_carry = 0.f, r_carry = 0.f, zsum = 0.f;
   if (wave_active) {
     if (t_b == 0) {
-      m_ref = halo_dot16<D>(qv, Ks, krs, rope_k, 0) * cl2;
+      const float s0 = halo_dot16<D>(qv, Ks, krs, rope_k, 0) * cl2;
+      m_ref = rintf(s0);
+      s_carry = s0 - m_ref;
     } else {
       const int k0 = 32 * t_b;
       s_carry = halo_dot16<D>(qv, Ks, krs, rope_k, k0) * cl2;
       const float s_prev = halo_dot16<D>(qv, Ks, krs, rope_k, k0 - 1) * cl2;
-      m_ref = fmaxf(s_carry, s_prev);
+      m_ref = rintf(fmaxf(s_carry, s_prev));
       float l_unused;
       seg_shares(s_prev, s_carry, fast_exp2(s_prev - m_ref), fast_exp2(s_carry - m_ref), l_unused,
                  r_carry);
@@ -852,7 +858,7 @@ __global__ __launch_bounds__(512, (fwd16_waves_per_simd<D, E, ROPE>())) void ca_
       mt = fmaxf(mt, xhalf(mt));
       const bool grow = mt > kLazyRescale;
       if (wave_any(grow)) {
-        const float shift = grow ? mt : 0.0f;
+        const float shift = grow ? rintf(mt) : 0.0f;
         const float alpha = grow ? fast_exp2(-shift) : 1.0f;
 #pragma unroll
         for (int mb = 0; mb < P::NMB; ++mb) acc_o[mb] *= alpha;
@@ -889,8 +895,8 @@ __global__ __launch_bounds__(512, (fwd16_waves_per_simd<D, E, ROPE>())) void ca_
         float x = Lv + r_prev;
         const int wk = kbase - 1 + r;
         if constexpr (kGeneral) {
-          const float cap_last = (diag && wk == i) ? 0.5f * pl : 0.0f;
-          const float cap_first = wk == 0 ? 0.5f * pl : 0.0f;
+          const float cap_last = (diag && wk == i) ? 2.0f * pl : 0.0f;
+          const float cap_first = wk == 0 ? 2.0f * pl : 0.0f;
           x += cap_last + cap_first;
         }
         wt[r] = x;
@@ -979,11 +985,11 @@ __global__ __launch_bounds__(512, (fwd16_waves_per_simd<D, E, ROPE>())) void ca_
   }
   if (G4 == 0) {
     if (single) {
-      stats[((size_t)bh * T + i) * 2 + 0] = m_ref;
+      stats[((size_t)bh * T + i) * 2 + 0] = m_ref - kShareShift;
       stats[((size_t)bh * T + i) * 2 + 1] = scl;
     } else {
       float* mz = part + (size_t)BH * smax * T * D + (((size_t)bh * smax + split) * T + i) * 2;
-      mz[0] = m_ref;
+      mz[0] = m_ref - kShareShift;
       mz[1] = ztot;
     }
   }
