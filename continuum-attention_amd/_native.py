@@ -43,6 +43,12 @@ SIGNATURES = {
                         _i, _i, _i, _i, _vp]),
     "ca_bwd_f32_noalloc": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                 _i, _i, _i, _i, _vp]),
+    "ca_padded_head_dim": (_i, [_i]),
+    "ca_fwd_op_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
+    "ca_bwd_op_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
+    "ca_fwd_op": (_i, [_vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _sz, _i, _i, _i, _i, _vp]),
+    "ca_bwd_op": (_i, [_vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz,
+                       _i, _i, _i, _i, _vp]),
     "ca_weights_f32": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _vp]),
     "ca_weights_bwd_f32": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp]),
     "ca_fwd_qkv": (_i, [_vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _i, _i, _i, _i, _vp]),

@@ -285,18 +285,23 @@ bool plan_bwd(int B, int H, int T, int D, size_t bytes, bool kv_sums, BwdPlan* p
   return false;
 }
 
+// The workspace cap less `used` bytes (never 0; SIZE_MAX: no cap).
+size_t cap_less(size_t used) {
+  if (g_workspace_cap == 0) return SIZE_MAX;
+  return g_workspace_cap > used ? g_workspace_cap - used : 1;
+}
+
 // Workspace the backward asks for under the cap: the full one when it fits
 // (without kv_sums), else the need of the plan for the cap, or, when no plan
 // fits under the cap, the least any plan needs (sets of one head, one
 // 128-query group per pass).
-size_t bwd_capped_bytes(int B, int H, int T, int D, bool kv_sums) {
+size_t bwd_capped_bytes(int B, int H, int T, int D, bool kv_sums, size_t cap) {
   if (!kv_sums) {
     const size_t full = bwd_full_bytes(B, H, T, D);
-    if (g_workspace_cap == 0 || full <= g_workspace_cap) return full;
+    if (full <= cap) return full;
   }
   BwdPlan plan;
-  if (plan_bwd(B, H, T, D, g_workspace_cap ? g_workspace_cap : SIZE_MAX, kv_sums, &plan))
-    return plan.need;
+  if (plan_bwd(B, H, T, D, cap, kv_sums, &plan)) return plan.need;
   size_t need = 0;
   for (int g = 0; g < ca::dq_num_groups(T); ++g)
     need = std::max(need, bwd_layout(1, 1, T, D, ca::bwd_pass(T, g, g + 1)).total);
@@ -421,7 +426,7 @@ size_t ca_fwd_workspace_bytes(int B, int H, int T, int D) {
 
 size_t ca_bwd_workspace_bytes(int B, int H, int T, int D) {
   if (B <= 0 || H <= 0 || T <= 0 || D <= 0) return 0;
-  return bwd_capped_bytes(B, H, T, D, false);
+  return bwd_capped_bytes(B, H, T, D, false, cap_less(0));
 }
 
 // The token-major entry points add room for the keys rotated once when that
@@ -442,7 +447,7 @@ size_t ca_bwd_qkv_workspace_bytes(int B, int H, int T, int D) {
   const size_t with_keys = rotated_keys_bytes(B, H, T, D) + full;
   if (g_workspace_cap == 0 || with_keys <= g_workspace_cap) return with_keys;
   if (full <= g_workspace_cap) return full;
-  return std::min(full, bwd_capped_bytes(B, H, T, D, true));
+  return std::min(full, bwd_capped_bytes(B, H, T, D, true, cap_less(0)));
 }
 
 }  // extern "C"
@@ -610,7 +615,7 @@ int bwd_common(const ca::BwdIO& io, int dtype, void* workspace, size_t workspace
   BwdPlan plan;
   if (!workspace || !plan_bwd(B, H, T, D, workspace_bytes, kv_sums, &plan))
     return fail(CA_ERR_WORKSPACE, "backward workspace of %zu bytes required, %zu given",
-                bwd_capped_bytes(B, H, T, D, kv_sums), workspace ? workspace_bytes : 0);
+                bwd_capped_bytes(B, H, T, D, kv_sums, cap_less(0)), workspace ? workspace_bytes : 0);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
   if (plan.hc == 0) return run_set(io, dtype, ws, plan.passes, true, kv_sums, B, H, T, D, s);
@@ -660,7 +665,7 @@ int ca_fwd_f32(const float* q, const float* k, const float* v, const float* log_
   if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out))
     return fail(CA_ERR_INVALID, "q, k, v and out must be 16-byte aligned");
   ca::FwdIO io{heads_view(q, H, T, D), heads_view(k, H, T, D), heads_view(v, H, T, D), nullptr,
-               false, log_gain, out, ca::View{nullptr, 0, 0, 0}, stats};
+               false, log_gain, out, ca::View{nullptr, 0, 0, 0}, stats, D};
   return fwd_common(io, CA_DTYPE_F32, workspace, workspace_bytes, B, H, T, D, stream);
 }
 
@@ -678,7 +683,174 @@ int ca_bwd_f32(const float* q, const float* k, const float* v, const float* log_
   ca::BwdIO io{heads_view(q, H, T, D), heads_view(k, H, T, D), heads_view(v, H, T, D), nullptr,
                false, log_gain, out, stats, heads_view(dout, H, T, D), heads_view(dq, H, T, D),
                heads_view(dk, H, T, D), heads_view(dv, H, T, D), dlog_gain};
+  io.head_dim = D;
   return bwd_common(io, CA_DTYPE_F32, workspace, workspace_bytes, B, H, T, D, stream, false);
+}
+
+}  // extern "C"
+
+// ---- the operator on [B,H,T,D] tensors of any operand type and head dim -----
+// Head dims without kernels of their own run on zero-padded rows (pads at
+// the start of the workspace, the padded problem's own workspace after them).
+static size_t pad_bytes(int dtype, int B, int H, int T, int DP, int tensors) {
+  return tensors * align256((size_t)B * H * T * DP * dtype_size(dtype));
+}
+static size_t fwd_pads(int dtype, int B, int H, int T, int D) {
+  const int DP = ca::padded_head_dim(D);
+  // q, k, v and, when the caller keeps no y, the padded fp32 output
+  return DP == D ? 0 : pad_bytes(dtype, B, H, T, DP, 3) + pad_bytes(CA_DTYPE_F32, B, H, T, DP, 1);
+}
+static size_t bwd_pads(int dtype, int B, int H, int T, int D) {
+  const int DP = ca::padded_head_dim(D);
+  return DP == D ? 0 : pad_bytes(dtype, B, H, T, DP, 7);  // q, k, v, dout; dq, dk, dv
+}
+static int check_op(const char* fn, int dtype, int B, int H, int T, int D) {
+  if (dtype != CA_DTYPE_F32 && dtype != CA_DTYPE_BF16 && dtype != CA_DTYPE_F16)
+    return fail(CA_ERR_INVALID, "%s: unknown dtype code %d", fn, dtype);
+  if (B > 0 && H > 0 && T > 0 && D > 0 && !ca::padded_head_dim(D))
+    return fail(CA_ERR_UNSUPPORTED, "%s: head dim D=%d not supported (at most 128)", fn, D);
+  return check_shape(B, H, T, D > 0 ? ca::padded_head_dim(D) : D);
+}
+template <class E>
+static hipError_t pad_rows(const void* const* src, char* dst, size_t each, int count, long long rows,
+                           int D, int DP, hipStream_t s) {
+  ca::PadSet<E> set{};
+  for (int i = 0; i < count; ++i) {
+    set.src[i] = static_cast<const E*>(src[i]);
+    set.dst[i] = reinterpret_cast<E*>(dst + i * each);
+  }
+  return ca::launch_pad<E>(set, count, rows, D, DP, s);
+}
+static hipError_t pad_rows(int dtype, const void* const* src, char* dst, size_t each, int count,
+                           long long rows, int D, int DP, hipStream_t s) {
+  if (dtype == CA_DTYPE_BF16) return pad_rows<__bf16>(src, dst, each, count, rows, D, DP, s);
+  if (dtype == CA_DTYPE_F16) return pad_rows<_Float16>(src, dst, each, count, rows, D, DP, s);
+  return pad_rows<float>(src, dst, each, count, rows, D, DP, s);
+}
+template <class S, class E>
+static hipError_t unpad_rows(const char* src, size_t each, void* const* dst, int count,
+                             long long rows, int D, int DP, hipStream_t s) {
+  ca::UnpadSet<S, E> set{};
+  for (int i = 0; i < count; ++i) {
+    set.src[i] = reinterpret_cast<const S*>(src + i * each);
+    set.dst[i] = static_cast<E*>(dst[i]);
+  }
+  return ca::launch_unpad<S, E>(set, count, rows, D, DP, s);
+}
+
+extern "C" {
+
+int ca_padded_head_dim(int D) { return ca::padded_head_dim(D); }
+
+size_t ca_fwd_op_workspace_bytes(int dtype, int B, int H, int T, int D) {
+  const int DP = ca::padded_head_dim(D);
+  if (B <= 0 || H <= 0 || T <= 0 || !DP) return 0;
+  const size_t pads = fwd_pads(dtype, B, H, T, D);
+  return pads + ca::fwd_part_floats(B * H, T, fwd_split(B * H, T, DP, true, cap_less(pads)), DP) *
+                    sizeof(float);
+}
+
+int ca_fwd_op(const void* q, const void* k, const void* v, int dtype, const float* log_gain,
+              float* y, void* out, float* stats, void* workspace, size_t workspace_bytes, int B,
+              int H, int T, int D, void* stream) {
+  int rc = check_op("ca_fwd_op", dtype, B, H, T, D);
+  if (rc) return rc;
+  if (!q || !k || !v || !log_gain || !stats || (!y && !out))
+    return fail(CA_ERR_INVALID, "ca_fwd_op: null tensor pointer");
+  const size_t a = dtype == CA_DTYPE_F32 ? 16 : 8;
+  if (!aligned_to(q, a) || !aligned_to(k, a) || !aligned_to(v, a) || (out && !aligned_to(out, a)) ||
+      (y && !aligned16(y)))
+    return fail(CA_ERR_INVALID, "ca_fwd_op: misaligned tensor (q, k, v, out %zu-byte, y 16-byte)", a);
+  const int DP = ca::padded_head_dim(D);
+  if (DP == D) {
+    ca::FwdIO io{heads_view(q, H, T, D), heads_view(k, H, T, D), heads_view(v, H, T, D), nullptr,
+                 false, log_gain, y, out ? heads_view(out, H, T, D) : ca::View{nullptr, 0, 0, 0},
+                 stats, D};
+    return fwd_common(io, dtype, workspace, workspace_bytes, B, H, T, D, stream);
+  }
+  const size_t pads = fwd_pads(dtype, B, H, T, D);
+  if (!workspace || workspace_bytes < pads)
+    return fail(CA_ERR_WORKSPACE, "ca_fwd_op: workspace of %zu bytes required, %zu given",
+                ca_fwd_op_workspace_bytes(dtype, B, H, T, D), workspace ? workspace_bytes : 0);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  char* ws = static_cast<char*>(workspace);
+  const size_t each = pad_bytes(dtype, B, H, T, DP, 1);
+  const long long rows = (long long)B * H * T;
+  const void* src[3] = {q, k, v};
+  hipError_t e = pad_rows(dtype, src, ws, each, 3, rows, D, DP, s);
+  if (e != hipSuccess) return fail(CA_ERR_HIP, "ca_fwd_op: pad launch: %s", hipGetErrorString(e));
+  float* yp = y ? y : reinterpret_cast<float*>(ws + 3 * each);
+  ca::FwdIO io{heads_view(ws, H, T, DP), heads_view(ws + each, H, T, DP),
+               heads_view(ws + 2 * each, H, T, DP), nullptr, false, log_gain, yp,
+               ca::View{nullptr, 0, 0, 0}, stats, D};
+  rc = fwd_common(io, dtype, ws + pads, workspace_bytes - pads, B, H, T, DP, stream);
+  if (rc || !out) return rc;
+  const char* ysrc = reinterpret_cast<const char*>(yp);
+  if (dtype == CA_DTYPE_BF16) e = unpad_rows<float, __bf16>(ysrc, 0, &out, 1, rows, D, DP, s);
+  else if (dtype == CA_DTYPE_F16) e = unpad_rows<float, _Float16>(ysrc, 0, &out, 1, rows, D, DP, s);
+  else e = unpad_rows<float, float>(ysrc, 0, &out, 1, rows, D, DP, s);
+  if (e != hipSuccess) return fail(CA_ERR_HIP, "ca_fwd_op: unpad launch: %s", hipGetErrorString(e));
+  return CA_OK;
+}
+
+size_t ca_bwd_op_workspace_bytes(int dtype, int B, int H, int T, int D) {
+  const int DP = ca::padded_head_dim(D);
+  if (B <= 0 || H <= 0 || T <= 0 || !DP) return 0;
+  const size_t pads = bwd_pads(dtype, B, H, T, D), cap = cap_less(pads);
+  const size_t full = bwd_full_bytes(B, H, T, DP);
+  if (full <= cap) return pads + full;
+  // passes: 16-bit gradients are summed over them in fp32 (as ca_bwd_qkv)
+  const bool sums = dtype != CA_DTYPE_F32;
+  const size_t need = bwd_capped_bytes(B, H, T, DP, sums, cap);
+  return pads + (sums ? std::min(full, need) : need);
+}
+
+int ca_bwd_op(const void* q, const void* k, const void* v, int dtype, const float* log_gain,
+              const float* y, const float* stats, const void* dout, void* dq, void* dk, void* dv,
+              float* dlog_gain, void* workspace, size_t workspace_bytes, int B, int H, int T,
+              int D, void* stream) {
+  int rc = check_op("ca_bwd_op", dtype, B, H, T, D);
+  if (rc) return rc;
+  if (!q || !k || !v || !log_gain || !y || !stats || !dout || !dq || !dk || !dv || !dlog_gain)
+    return fail(CA_ERR_INVALID, "ca_bwd_op: null tensor pointer");
+  const size_t a = dtype == CA_DTYPE_F32 ? 16 : 8;
+  for (const void* p : {q, k, v, dout, (const void*)dq, (const void*)dk, (const void*)dv})
+    if (!aligned_to(p, a)) return fail(CA_ERR_INVALID, "ca_bwd_op: tensors must be %zu-byte aligned", a);
+  if (!aligned16(y)) return fail(CA_ERR_INVALID, "ca_bwd_op: y must be 16-byte aligned");
+  const int DP = ca::padded_head_dim(D);
+  const size_t pads = bwd_pads(dtype, B, H, T, D);
+  if (!workspace || workspace_bytes < pads)
+    return fail(CA_ERR_WORKSPACE, "ca_bwd_op: workspace of %zu bytes required, %zu given",
+                ca_bwd_op_workspace_bytes(dtype, B, H, T, D), workspace ? workspace_bytes : 0);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  char* ws = static_cast<char*>(workspace);
+  const size_t each = DP == D ? 0 : pad_bytes(dtype, B, H, T, DP, 1);
+  const long long rows = (long long)B * H * T;
+  const void* in[4] = {q, k, v, dout};
+  void* grads[3] = {dq, dk, dv};
+  const void *pin[4], *pgrad[3];
+  hipError_t e;
+  for (int i = 0; i < 4; ++i) pin[i] = DP == D ? in[i] : ws + i * each;
+  for (int i = 0; i < 3; ++i) pgrad[i] = DP == D ? grads[i] : ws + (4 + i) * each;
+  if (DP != D) {
+    e = pad_rows(dtype, in, ws, each, 4, rows, D, DP, s);
+    if (e != hipSuccess) return fail(CA_ERR_HIP, "ca_bwd_op: pad launch: %s", hipGetErrorString(e));
+  }
+  ca::BwdIO io{heads_view(pin[0], H, T, DP), heads_view(pin[1], H, T, DP),
+               heads_view(pin[2], H, T, DP), nullptr, false, log_gain, y, stats,
+               heads_view(pin[3], H, T, DP), heads_view(pgrad[0], H, T, DP),
+               heads_view(pgrad[1], H, T, DP), heads_view(pgrad[2], H, T, DP), dlog_gain};
+  io.head_dim = D;
+  const size_t core = workspace_bytes - pads;
+  const bool sums = dtype != CA_DTYPE_F32 && core < bwd_full_bytes(B, H, T, DP);
+  rc = bwd_common(io, dtype, ws + pads, core, B, H, T, DP, stream, sums);
+  if (rc || DP == D) return rc;
+  const char* gsrc = ws + 4 * each;
+  if (dtype == CA_DTYPE_BF16) e = unpad_rows<__bf16, __bf16>(gsrc, each, grads, 3, rows, D, DP, s);
+  else if (dtype == CA_DTYPE_F16) e = unpad_rows<_Float16, _Float16>(gsrc, each, grads, 3, rows, D, DP, s);
+  else e = unpad_rows<float, float>(gsrc, each, grads, 3, rows, D, DP, s);
+  if (e != hipSuccess) return fail(CA_ERR_HIP, "ca_bwd_op: unpad launch: %s", hipGetErrorString(e));
+  return CA_OK;
 }
 
 static int check_qkv(const char* fn, int dtype, const void* qkv, const float* rope_cs,
@@ -710,7 +882,7 @@ int ca_fwd_qkv(const void* qkv, int dtype, const float* rope_cs, const float* lo
   if (rc) return rc;
   ca::FwdIO io{tokens_view(qkv, dtype, 0, 3, T, H, D), tokens_view(qkv, dtype, 1, 3, T, H, D),
                tokens_view(qkv, dtype, 2, 3, T, H, D), rope_cs, false, log_gain, y,
-               tokens_view(out, dtype, 0, 1, T, H, D), stats};
+               tokens_view(out, dtype, 0, 1, T, H, D), stats, D};
   char* ws = static_cast<char*>(workspace);
   size_t bytes = workspace_bytes;
   if (workspace &&
@@ -738,6 +910,7 @@ int ca_bwd_qkv(const void* qkv, int dtype, const float* rope_cs, const float* lo
                tokens_view(dout, dtype, 0, 1, T, H, D), tokens_view(dqkv, dtype, 0, 3, T, H, D),
                tokens_view(dqkv, dtype, 1, 3, T, H, D), tokens_view(dqkv, dtype, 2, 3, T, H, D),
                dlog_gain};
+  io.head_dim = D;
   char* ws = static_cast<char*>(workspace);
   size_t bytes = workspace_bytes;
   const size_t full = bwd_full_bytes(B, H, T, D);

@@ -10,7 +10,7 @@
 //   ca_bwd_prep     per query row: Dl_i = dY_i . y_i (the reference forms the
 //                   same row mean at cuda/continuum_attention.py:268-269),
 //                   Q_i and dY_i / Z_i split into bf16 limb planes, and
-//                   (-m_i, -Dl_i / Z_i).
+//                   (-(m_i + kShareShift), Dl_i / Z_i).
 //   ca_bwd_dkdv     (ca_bwd_dkdv.hip) one work group per (slice, 56 keys); wave w owns 14 keys
 //                   (16 MFMA slots).  The 4 waves walk the query tiles
 //                   together: each 32-query tile of Q and dY/Z limbs is staged
@@ -49,7 +49,7 @@ namespace ca {
 
 // One thread per (row of the pass's query tiles, 8 elements): Dl = dY . y,
 // then the Q and dY/Z limbs of the 8 elements (one 16-byte store per plane)
-// and, per row, (-(m + kShareShift), -Dl/Z).  The limb planes are tile-major: tile j of the
+// and, per row, (-(m + kShareShift), Dl/Z).  The limb planes are tile-major: tile j of the
 // pass in slice bh is the block limbs[(bh * ntiles + j) * P * 32 * D ..] of
 // P planes [32 rows][D] (P = q_limb_planes<E>() + 3).  Rows past T (in the
 // last tile) are written as zeros, so the dK/dV kernel stages whole tiles
@@ -111,10 +111,10 @@ __global__ __launch_bounds__(256) void ca_bwd_prep_kernel(View Qv, const float* 
   put(0, QL, qq, 1.0f);  // bf16 operands: Q is bf16-valued, its h limb is exact
   put(QL, 3, dy, invz);
   if (c == 0) {
-    // negated: the dK/dV kernel starts its S and dP' accumulators from them
+    // as the dK/dV kernel's score shift and dP' accumulator start take them
     // (m an integer from the forward, so the sum with kShareShift is exact)
     qstat[(size_t)row * 2 + 0] = -(m + kShareShift);
-    qstat[(size_t)row * 2 + 1] = -(x * invz);
+    qstat[(size_t)row * 2 + 1] = x * invz;
   }
 }
 
@@ -223,7 +223,8 @@ __global__ __launch_bounds__(256, (std::is_same<E, __bf16>::value && D <= 64 ? 4
                                                         int n_items, int n_part, int n_kv_items,
                                                         const float* __restrict__ kv_part,
                                                         View dKv, View dVv, int kv_chunk,
-                                                        int kv_part_items, bool kv_f32) {
+                                                        int kv_part_items, bool kv_f32,
+                                                        int hd) {
   using P = DqP<D>;
   const int BH = B * H;
   if ((int)blockIdx.x >= n_items * BH) {
@@ -260,7 +261,7 @@ __global__ __launch_bounds__(256, (std::is_same<E, __bf16>::value && D <= 64 ? 4
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int qt = kDqTiles * qg + w;
   const bool wave_on = qt < nqt;
-  const float c = head_scale_log2(log_gain, bh % H, D) * kLn2;
+  const float c = head_scale_log2(log_gain, bh % H, hd) * kLn2;
   // stages of this chunk met by the wave's tile (stage s holds keys 32s .. 32s+31)
   const int my_end = wave_on ? min(qt + 1, st_hi) : 0;
   const int iters = st_hi > st_lo ? st_hi - st_lo : 0;
@@ -536,6 +537,83 @@ hipError_t launch_kv_cast(const float* dk_sum, const float* dv_sum, View dk, Vie
   return hipGetLastError();
 }
 
+// ---- head dims without kernels of their own --------------------------------
+// Zero columns change neither q.k nor any gradient of the real columns, so
+// a head dim D below the next kernel dim DP runs on rows padded with zeros.
+// One launch pads up to four [rows][D] tensors (grid y) to [rows][DP]; one
+// narrows up to three back.  Both are memory-bound copies: each thread
+// handles four consecutive padded (narrowed) elements, so the wide side is
+// accessed 16 (8) bytes at a time.
+template <class E>
+__global__ __launch_bounds__(256) void ca_pad_kernel(PadSet<E> set, long long n4, int D, int DP) {
+  const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (t >= n4) return;
+  const E* __restrict__ src = set.src[blockIdx.y];
+  const int c4 = DP / 4;
+  const long long row = t / c4;
+  const int d0 = 4 * (int)(t % c4);
+  E v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = d0 + e < D ? src[row * D + d0 + e] : (E)0.f;
+  typename Raw4<E>::type w;
+  __builtin_memcpy(&w, v, sizeof(w));
+  *reinterpret_cast<typename Raw4<E>::type*>(set.dst[blockIdx.y] + 4 * t) = w;
+}
+
+// narrowed element i of [rows][D] from row i / D of the padded tensor, which
+// holds fp32 (the forward's y) or E (gradients)
+template <class S, class E>
+__global__ __launch_bounds__(256) void ca_unpad_kernel(UnpadSet<S, E> set, long long n, int D,
+                                                       int DP) {
+  const long long i0 = ((long long)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i0 >= n) return;
+  const S* __restrict__ src = set.src[blockIdx.y];
+  E* __restrict__ dst = set.dst[blockIdx.y];
+  long long row = i0 / D;
+  int d = (int)(i0 - row * D);
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (i0 + e < n) v[e] = ld1(src + row * DP + d);
+    if (++d == D) {
+      d = 0;
+      ++row;
+    }
+  }
+  if (i0 + 4 <= n)
+    st4(dst + i0, v);
+  else
+    for (int e = 0; i0 + e < n; ++e) st1(dst + i0 + e, v[e]);
+}
+
+template <class E>
+hipError_t launch_pad(const PadSet<E>& set, int count, long long rows, int D, int DP,
+                      hipStream_t stream) {
+  const long long n4 = rows * (DP / 4);
+  hipLaunchKernelGGL((ca_pad_kernel<E>), dim3((unsigned)((n4 + 255) / 256), count), dim3(256), 0,
+                     stream, set, n4, D, DP);
+  return hipGetLastError();
+}
+template <class S, class E>
+hipError_t launch_unpad(const UnpadSet<S, E>& set, int count, long long rows, int D, int DP,
+                        hipStream_t stream) {
+  const long long n = rows * D;
+  hipLaunchKernelGGL((ca_unpad_kernel<S, E>), dim3((unsigned)((n + 1023) / 1024), count), dim3(256),
+                     0, stream, set, n, D, DP);
+  return hipGetLastError();
+}
+#define CA_INST_PAD(EE)                                                                        \
+  template hipError_t launch_pad<EE>(const PadSet<EE>&, int, long long, int, int, hipStream_t); \
+  template hipError_t launch_unpad<float, EE>(const UnpadSet<float, EE>&, int, long long, int,   \
+                                              int, hipStream_t);
+CA_INST_PAD(float)
+CA_INST_PAD(__bf16)
+CA_INST_PAD(_Float16)
+template hipError_t launch_unpad<__bf16, __bf16>(const UnpadSet<__bf16, __bf16>&, int, long long,
+                                                 int, int, hipStream_t);
+template hipError_t launch_unpad<_Float16, _Float16>(const UnpadSet<_Float16, _Float16>&, int,
+                                                     long long, int, int, hipStream_t);
+
 template <int D, class E>
 hipError_t launch_bwd(const BwdIO& io, const BwdWork& ws, const BwdPass& pass, const DqSplit& sp,
                       const DkdvSplit& kvs, int B, int H, int T, hipStream_t stream) {
@@ -562,12 +640,12 @@ hipError_t launch_bwd(const BwdIO& io, const BwdWork& ws, const BwdPass& pass, c
     hipLaunchKernelGGL((ca_bwd_dq_kernel<D, E, true>), dq_grid, dim3(256), 0, stream, ws.dsbuf,
                        io.k, io.rope, io.log_gain, io.dq, ws.dq_part, ws.gain_part, io.dlog_gain,
                        pass, B, H, T, sp.chunk, sp.items, sp.part_items, kvs.items, ws.kv_part,
-                       io.dk, io.dv, kvs.chunk, kvs.part_items, io.kv_f32);
+                       io.dk, io.dv, kvs.chunk, kvs.part_items, io.kv_f32, io.head_dim);
   else
     hipLaunchKernelGGL((ca_bwd_dq_kernel<D, E, false>), dq_grid, dim3(256), 0, stream, ws.dsbuf,
                        io.k, io.rope, io.log_gain, io.dq, ws.dq_part, ws.gain_part, io.dlog_gain,
                        pass, B, H, T, sp.chunk, sp.items, sp.part_items, kvs.items, ws.kv_part,
-                       io.dk, io.dv, kvs.chunk, kvs.part_items, io.kv_f32);
+                       io.dk, io.dv, kvs.chunk, kvs.part_items, io.kv_f32, io.head_dim);
   timer_end(kBwdDq, stream);
   e = hipGetLastError();
   if (e != hipSuccess) return e;

@@ -10,7 +10,7 @@
 // of one DPP row (row_shr / row_shl).  p = 2^(s - m - kShareShift) stays
 // unnormalised (its shares come out four times as large, relative to m) and
 // dY arrives pre-scaled by 1/Z, so the weight gradient g = dY.v/Z - Dl/Z comes
-// straight out of the MFMA (its accumulator starts at -Dl/Z) and dV = W^T dY
+// straight out of the MFMA (its accumulator starts at Dl/Z, see kDpFlip) and dV = W^T dY
 // is formed as w^T (dY/Z) with no per-row scaling in the kernel.
 #include <type_traits>
 
@@ -65,18 +65,18 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
     const __bf16* __restrict__ limbs,
     const float* __restrict__ qstat, const float* __restrict__ log_gain, View dKv, View dVv,
     float* __restrict__ dsbuf, float* __restrict__ kv_part, float* __restrict__ gain_part,
-    BwdPass pass, int BH, int H, int T, int chunk, int n_items, int n_part, bool kv_f32) {
+    BwdPass pass, int BH, int H, int T, int chunk, int n_items, int n_part, bool kv_f32,
+    int hd) {
   // bf16 operands: Q, K (rotated and rounded as the reference rounds them)
   // and V are bf16-valued, so the tile carries Q's h limb alone and the
   // products with Q or V skip their zero limb products (limb_step_used), with
-  // the same sums bit for bit; S is q.k of the h limbs, scaled after the
-  // product.  Other operand types: K enters S scaled by the head's gain, in
-  // three limbs.
+  // the same sums bit for bit.
   constexpr bool BF = q_limb_planes<E>() == 1;
   using P = Bwd<D, q_limb_planes<E>()>;
   constexpr int NBUF = SB ? 1 : 2;
   __shared__ __attribute__((aligned(16))) __bf16 tiles[NBUF][P::TILE];
-  // per staged row: -m (tstat[b][0][row]) and -Dl/Z (tstat[b][1][row]), in
+  // per staged row: -(m + kShareShift) (tstat[b][0][row]) and Dl/Z
+  // (tstat[b][1][row]), in
   // the order of the S / dP' accumulator registers
   __shared__ __attribute__((aligned(16))) float tstat[NBUF][2][32];
 
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
   const int key_j = kBwdKeys * kb16 - 1 + j;  // key of this lane's slot
   const int kmin = kBwdKeys * kb16 - 1;        // key of slot 0
 
-  const float cl2 = head_scale_log2(log_gain, bh % H, D);
+  const float cl2 = head_scale_log2(log_gain, bh % H, hd);
 
   // Stale LDS bits must not reach an MFMA as NaN through padding columns.
   {
@@ -116,8 +116,7 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
   }
 
   // K (rotated here when `rope_k`; otherwise it arrives rotated, or without
-  // RoPE; then scaled by c log2e, except bf16 operands, whose scores are
-  // scaled after the product) and V of this lane's slot: B operands of S /
+  // RoPE) and V of this lane's slot: B operands of S /
   // dP', k block kb, element e = d 32kb + 8g + e.
   Limbs kl[P::KB], vl[P::KB];
 #pragma unroll
@@ -133,7 +132,6 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
       const bool ok2 = ok && d0 + 4 * h2 < D;
       f32x4 a = ok2 ? ld4(kp + 4 * h2) : f32x4{0.f, 0.f, 0.f, 0.f};
       if (rope_k && ok2) a = rope4_in<E>(a, rope_entry(rope_k, krow, D, d0 + 4 * h2));
-      if (!BF) a *= cl2;
       const f32x4 b = ok2 ? ld4(vp + 4 * h2) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -141,9 +139,17 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
         xv[4 * h2 + e] = b[e];
       }
     }
+    if (kb < P::KB / 2) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xv[e] = -xv[e];  // see kDpFlip
+    }
     kl[kb] = split8(xk);
     vl[kb] = split8(xv);
   }
+
+  // with a single k block the sign changes between its limb products (kDpFlip)
+  Limbs vneg;
+  if constexpr (P::KB == 1) vneg = limbs_neg(vl[0]);
 
   f32x4 accv[P::NMB], acck[P::NMB];
 #pragma unroll
@@ -229,20 +235,24 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
       const __bf16* Ty = &tiles[buf][(P::PLANES - 3) * P::LIMB];
 
       // ---- S - m and dP' - Dl/Z (row blocks rb: queries i0 + 16rb + 4g + r) ----
-      // bf16 operands: S accumulates q.k from zero (Q and K bf16-valued: the
-      // h limb product alone) and takes c log2e and -m in one fused
-      // multiply-add; otherwise K carries c log2e and the accumulator starts
-      // from -m.
-      f32x4 sacc[2], pacc[2], negm[2];
+      // S accumulates q.k from zero (bf16 operands: the h limb product alone)
+      // and takes c log2e and the row shift in one fused multiply-add per
+      // score, as the forward forms it: the small limb products then round at
+      // their own size.  Started from the shift they rounded at |m|, and with
+      // scores of variance 16 the gradients' errors were 1.5 times as large.
+      f32x4 sacc[2], pacc[2];
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb) {
-        negm[rb] = *reinterpret_cast<const f32x4*>(&tstat[buf][0][16 * rb + 4 * g]);
-        sacc[rb] = BF ? f32x4{0.f, 0.f, 0.f, 0.f} : negm[rb];
+        sacc[rb] = f32x4{0.f, 0.f, 0.f, 0.f};
         pacc[rb] = *reinterpret_cast<const f32x4*>(&tstat[buf][1][16 * rb + 4 * g]);
       }
       prio_mfma_begin<!BF>();
 #pragma unroll
       for (int kb = 0; kb < P::KB; ++kb) {
+        if (P::KB > 1 && kb == P::KB / 2) {
+          pacc[0] = -pacc[0];
+          pacc[1] = -pacc[1];
+        }
         const int col = 32 * kb + 8 * g;
         Limbs qa[2], ya[2];
 #pragma unroll
@@ -263,18 +273,26 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
         // four independent accumulators per limb product
 #pragma unroll
         for (int st = 0; st < 6; ++st) {
+          if (P::KB == 1 && st == 3) {
+            pacc[0] = -pacc[0];
+            pacc[1] = -pacc[1];
+          }
+          const Limbs& vb = P::KB == 1 && st < 3 ? vneg : vl[kb];
           if (limb_step_used<BF, BF>(st)) sacc[0] = mfma16_step(st, qa[0], kl[kb], sacc[0]);
-          if (limb_step_used<false, BF>(st)) pacc[0] = mfma16_step(st, ya[0], vl[kb], pacc[0]);
+          if (limb_step_used<false, BF>(st)) pacc[0] = mfma16_step(st, ya[0], vb, pacc[0]);
           if (limb_step_used<BF, BF>(st)) sacc[1] = mfma16_step(st, qa[1], kl[kb], sacc[1]);
-          if (limb_step_used<false, BF>(st)) pacc[1] = mfma16_step(st, ya[1], vl[kb], pacc[1]);
+          if (limb_step_used<false, BF>(st)) pacc[1] = mfma16_step(st, ya[1], vb, pacc[1]);
         }
       }
       prio_mfma_end<!BF>();
-      if (BF) {
+      // the row shifts are read only now: held across the products they cost
+      // eight registers, which the single-buffered variant spills
+      asm volatile("" ::: "memory");
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
+      for (int rb = 0; rb < 2; ++rb) {
+        const f32x4 negm = *reinterpret_cast<const f32x4*>(&tstat[buf][0][16 * rb + 4 * g]);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) sacc[rb][r] = fmaf(sacc[rb][r], cl2, negm[rb][r]);
+        for (int r = 0; r < 4; ++r) sacc[rb][r] = fmaf(sacc[rb][r], cl2, negm[r]);
       }
 
       // ---- segments along the slots (adjacent lanes of each DPP row) ----
@@ -481,7 +499,7 @@ hipError_t launch_bwd_dkdv(const BwdIO& io, const BwdWork& ws, const BwdPass& pa
                      io.v, io.rope, io.k_rotated ? nullptr : io.rope, ws.limbs, ws.qstat,
                      io.log_gain, io.dk, io.dv, ws.dsbuf,
                      ws.kv_part, ws.gain_part, pass, BH, H, T, kvs.chunk, kvs.items,
-                     kvs.part_items, io.kv_f32);
+                     kvs.part_items, io.kv_f32, io.head_dim);
   return hipGetLastError();
 }
 

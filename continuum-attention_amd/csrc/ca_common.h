@@ -187,6 +187,14 @@ __device__ __forceinline__ Limbs split8(const float* x) {
                __builtin_bit_cast(bf16x8, L)};
 }
 
+// -x in limbs (the signs of its bf16 parts)
+__device__ __forceinline__ bf16x8 bf16x8_neg(bf16x8 x) {
+  return __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, x) ^ 0x80008000u);
+}
+__device__ __forceinline__ Limbs limbs_neg(const Limbs& x) {
+  return Limbs{bf16x8_neg(x.h), bf16x8_neg(x.m), bf16x8_neg(x.l)};
+}
+
 // Wave priority raised over a wave's matrix-product blocks (s_setprio), so
 // the SIMD's other waves fill the VALU while those MFMAs are issued.  ON for
 // operands that take all six limb products: fp32 config 2 dK/dV 0.2698 ->

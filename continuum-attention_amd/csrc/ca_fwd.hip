@@ -116,7 +116,7 @@ template <int D, class E, bool ROPE>
 __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fwd_kernel(
     View Qv, View Kv, View Vv, const float* __restrict__ rope, const float* __restrict__ log_gain,
     float* __restrict__ O, View Ov, float* __restrict__ stats, float* __restrict__ part, int BH,
-    int H, int T, int C, int G, int smax) {
+    int H, int T, int C, int G, int smax, int hd) {
   using P = Fwd<D>;
   // bf16 operands (with RoPE rounded to bf16 as the reference does) are
   // bf16-valued: their limb split is h = the value, m = l = 0, so a K or V
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
   // or unrotated without RoPE), so the compiler drops every key rotation
   const float* __restrict__ rope_k = ROPE ? rope : nullptr;
   const int head = bh % H;
-  const float cl2 = head_scale_log2(log_gain, head, D);
+  const float cl2 = head_scale_log2(log_gain, head, hd);
 
   // lane (q,h) holds Q[i][h*DH + k].  The scores are scaled after the
   // product, as the reference scales q.k (s = c log2e (q.k) - m_ref, one
@@ -493,7 +493,7 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
   float* dst;
   float scl;
   if (single) {
-    dst = O + slice + (size_t)i * D;
+    dst = O ? O + slice + (size_t)i * D : nullptr;  // y is optional (see FwdIO)
     scl = 1.0f / ztot;
   } else {
     // part layout: [BH][smax][T][D] outputs then [BH][smax][T][2] (m, Z)
@@ -513,7 +513,7 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
     return;
   }
   if (!qvalid) return;
-  // a single-split row is final: also written token-major in the input type
+  // a single-split row is final: also written in the input type
   E* otok = (single && Ov.base) ? view_slice<E>(Ov, bh, H) + (long long)i * Ov.rstride : nullptr;
 #pragma unroll
   for (int mb = 0; mb < P::NMB; ++mb) {
@@ -523,7 +523,7 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
       if (d0 < D) {
         f32x4 v4 = {acc_o[mb][4 * r4 + 0] * scl, acc_o[mb][4 * r4 + 1] * scl,
                     acc_o[mb][4 * r4 + 2] * scl, acc_o[mb][4 * r4 + 3] * scl};
-        *reinterpret_cast<f32x4*>(dst + d0) = v4;
+        if (dst) *reinterpret_cast<f32x4*>(dst + d0) = v4;
         if (otok) st4(otok + d0, v4);
       }
     }
@@ -623,7 +623,7 @@ template <int D, class E, bool ROPE>
 __global__ __launch_bounds__(512, (fwd16_waves_per_simd<D, E, ROPE>())) void ca_fwd16_kernel(
     View Qv, View Kv, View Vv, const float* __restrict__ rope, const float* __restrict__ log_gain,
     float* __restrict__ O, View Ov, float* __restrict__ stats, float* __restrict__ part, int BH,
-    int H, int T, int C, int G, int smax) {
+    int H, int T, int C, int G, int smax, int hd) {
   using P = Fwd16<D>;
   constexpr bool BF = std::is_same<E, __bf16>::value;
   constexpr int NL = BF ? 1 : 3;  // limb planes staged per K and V tile
@@ -658,7 +658,7 @@ __global__ __launch_bounds__(512, (fwd16_waves_per_simd<D, E, ROPE>())) void ca_
   const long long krs = Kv.rstride, vrs = Vv.rstride;
   const float* __restrict__ rope_k = ROPE ? rope : nullptr;
   const int head = bh % H;
-  const float cl2 = head_scale_log2(log_gain, head, D);
+  const float cl2 = head_scale_log2(log_gain, head, hd);
 
   // lane (q16, G) holds Q[i][32ks + 8G + e] (rotated when `rope`)
   float qv[P::KS][8];
@@ -957,7 +957,7 @@ __global__ __launch_bounds__(512, (fwd16_waves_per_simd<D, E, ROPE>())) void ca_
   float* dst;
   float scl;
   if (single) {
-    dst = O + slice + (size_t)i * D;
+    dst = O ? O + slice + (size_t)i * D : nullptr;  // y is optional (see FwdIO)
     scl = 1.0f / ztot;
   } else {
     dst = part + (((size_t)bh * smax + split) * T + i) * D;
@@ -980,7 +980,7 @@ __global__ __launch_bounds__(512, (fwd16_waves_per_simd<D, E, ROPE>())) void ca_
   for (int mb = 0; mb < P::NMB; ++mb) {
     const int d0 = 16 * mb + 4 * G4;
     const f32x4 v4 = acc_o[mb] * scl;
-    *reinterpret_cast<f32x4*>(dst + d0) = v4;
+    if (dst) *reinterpret_cast<f32x4*>(dst + d0) = v4;
     if (otok) st4(otok + d0, v4);
   }
   if (G4 == 0) {
@@ -1024,7 +1024,7 @@ __global__ __launch_bounds__(256) void ca_fwd_combine_kernel(const float* __rest
     acc += reinterpret_cast<const f32x4*>(part + base * D)[c] * f;
   }
   const float invz = 1.0f / Z;
-  reinterpret_cast<f32x4*>(O + (size_t)row * D)[c] = acc * invz;
+  if (O) reinterpret_cast<f32x4*>(O + (size_t)row * D)[c] = acc * invz;
   if (Ov.base) st4(view_slice<E>(Ov, bh, H) + (long long)i * Ov.rstride + 4 * c, acc * invz);
   if (c == 0) {
     stats[(size_t)row * 2 + 0] = M;
@@ -1051,20 +1051,20 @@ hipError_t launch_fwd(const FwdIO& io, float* part, int B, int H, int T, int C,
     if (io.rope && !io.k_rotated)
       hipLaunchKernelGGL((ca_fwd16_kernel<D, E, true>), dim3(items * BH), dim3(512), 0, stream,
                          io.q, io.k, io.v, io.rope, io.log_gain, io.y, io.out, io.stats, part, BH, H,
-                         T, C, G, smax);
+                         T, C, G, smax, io.head_dim);
     else
       hipLaunchKernelGGL((ca_fwd16_kernel<D, E, false>), dim3(items * BH), dim3(512), 0, stream,
                          io.q, io.k, io.v, io.rope, io.log_gain, io.y, io.out, io.stats, part, BH, H,
-                         T, C, G, smax);
+                         T, C, G, smax, io.head_dim);
   } else {
     if (io.rope && !io.k_rotated)
       hipLaunchKernelGGL((ca_fwd_kernel<D, E, true>), dim3(items * BH), dim3(256), 0, stream, io.q,
                          io.k, io.v, io.rope, io.log_gain, io.y, io.out, io.stats, part, BH, H, T,
-                         C, G, smax);
+                         C, G, smax, io.head_dim);
     else
       hipLaunchKernelGGL((ca_fwd_kernel<D, E, false>), dim3(items * BH), dim3(256), 0, stream, io.q,
                          io.k, io.v, io.rope, io.log_gain, io.y, io.out, io.stats, part, BH, H, T,
-                         C, G, smax);
+                         C, G, smax, io.head_dim);
   }
   timer_end(kFwd, stream);
   hipError_t e = hipGetLastError();

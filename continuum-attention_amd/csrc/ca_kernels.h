@@ -359,9 +359,11 @@ struct FwdIO {
   const float* rope;       // [T][D/2][2] (cos, sin) for q and k, or nullptr
   bool k_rotated;          // k is already rotated (launch_rope_keys): rope applies to q only
   const float* log_gain;   // [H]
-  float* y;                // fp32 [B,H,T,D] output (read by the backward)
+  float* y;                // fp32 [B,H,T,D] output, read by the backward (nullptr: not kept)
   View out;                // optional copy of the output in E (base nullptr: none)
   float* stats;            // [B*H*T][2]
+  int head_dim;            // head dim of the score scale 1/sqrt(head_dim): D, or less when the
+                           // rows are padded with zeros to D
 };
 struct BwdIO {
   View q, k, v;            // the forward's inputs
@@ -377,7 +379,28 @@ struct BwdIO {
   // passes sums dK and dV over the passes in fp32 and rounds them to E once
   // (launch_kv_cast) instead of after every pass
   bool kv_f32 = false;
+  int head_dim = 0;        // as in FwdIO
 };
+
+// Head dims without kernels of their own run on zero-padded rows: the least
+// kernel dim that holds D (0: none).
+__host__ __device__ constexpr int padded_head_dim(int D) {
+  return D <= 0 ? 0 : D <= 8 ? 8 : D <= 16 ? 16 : D <= 32 ? 32 : D <= 64 ? 64 : D <= 128 ? 128 : 0;
+}
+template <class E> struct PadSet {  // [rows][D] tensors and their padded copies
+  const E* src[4];
+  E* dst[4];
+};
+template <class S, class E> struct UnpadSet {
+  const S* src[3];
+  E* dst[3];
+};
+template <class E>
+hipError_t launch_pad(const PadSet<E>& set, int count, long long rows, int D, int DP,
+                      hipStream_t stream);
+template <class S, class E>
+hipError_t launch_unpad(const UnpadSet<S, E>& set, int count, long long rows, int D, int DP,
+                        hipStream_t stream);
 
 template <int D, class E>
 hipError_t launch_fwd(const FwdIO& io, float* part, int B, int H, int T, int C,
@@ -395,7 +418,7 @@ struct BwdWork {
   float* dsbuf;       // dS spill, 32x16 blocks
   __bf16* limbs;      // per slice and query tile of the pass, six bf16 planes [32 rows][D]:
                       // Q limbs h, m, l; dY/Z limbs h, m, l ([BH][tile][plane][32][D])
-  float* qstat;       // per slice and padded row of the pass's tiles: (-m, -D/Z)
+  float* qstat;       // per slice and padded row of the pass's tiles: (-(m + kShareShift), D/Z)
   float* gain_part;   // per dQ item
   float* dq_part;     // dQ chunk partials
   float* kv_part;     // dK/dV chunk partials: [BH][part item][kDkdvKeys][2][D]
@@ -416,6 +439,16 @@ __host__ __device__ inline int bwd_pass_tiles(const BwdPass& p) { return p.qb - 
 template <class E> __host__ __device__ constexpr int q_limb_planes() {
   return std::is_same<E, __bf16>::value ? 1 : 3;
 }
+// kDpFlip.  The matrix cores round their fp32 sums slightly downwards,
+// whatever the sign (about 2^-28 of the accumulator per dP' element,
+// measured): a bias common to a row's weight gradients, which the row's dS
+// then sums to instead of zero and the gain gradient collects over all rows
+// (-5e-5 on values of 10-30 at T = 2048, the largest error in it).  The
+// dK/dV kernel therefore forms -dP' over the first half of the k blocks, or
+// of the limb products where there is one block (V negated in registers, the
+// accumulator started from +Dl/Z), and changes the sign before the second
+// half, so that the halves' biases cancel: the gain gradient's mean error at
+// [2,16,2048,64] 3.6e-6 -> 1.3e-6, dK/dV time unchanged within the noise.
 __host__ __device__ constexpr int limb_tile_elems(int D, int planes = 6) { return planes * 32 * D; }
 inline size_t bwd_limb_elems(int BH, const BwdPass& p, int D) {
   return (size_t)BH * bwd_pass_tiles(p) * limb_tile_elems(D);

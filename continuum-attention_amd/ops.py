@@ -12,12 +12,15 @@ autograd Function ``_CAExactTiled`` (cuda/continuum_attention.py:650-783):
   (:765-766).
 
 Compute is float32 on the device (fp16/bf16 inputs are read as fp32, results
-cast back).  ``query_tile`` is accepted and validated; in the reference it only
-bounds the memory of the materialised ``[BH, Qt, K]`` weights
-(cuda/continuum_attention.py:957), which the fused kernels (D in 8, 16, 32,
-64, 128) never materialise, so it does not change their arithmetic; other head
-dims run the reference's query-tile structure, where it does bound memory.  All ``CA_CUDA_MODE`` values select the same
-exact fp32 path (the reference modes differ only in fp16 rounding and launch
+cast back): the kernels read fp32, bf16 and fp16 tensors as they are and
+round the output and the gradients to that type once.  ``query_tile`` is
+accepted and validated; in the reference it only bounds the memory of the
+materialised ``[BH, Qt, K]`` weights (cuda/continuum_attention.py:957), which
+the fused kernels never materialise, so it does not change their arithmetic.
+They serve head dims up to 128 (8, 16, 32, 64 and 128 directly, others on rows
+padded with zeros); larger ones run the reference's query-tile structure,
+where it does bound memory.  All ``CA_CUDA_MODE`` values select the same exact
+fp32 path (the reference modes differ only in fp16 rounding and launch
 structure).
 
 The reference's per-mode limits hold on every device (:662-665):
@@ -87,6 +90,16 @@ def _bwd_workspace_bytes(B: int, H: int, T: int, D: int) -> int:
 
 
 @functools.lru_cache(maxsize=256)
+def _fwd_op_workspace_bytes(dtype: int, B: int, H: int, T: int, D: int) -> int:
+    return int(_native.load().ca_fwd_op_workspace_bytes(dtype, B, H, T, D))
+
+
+@functools.lru_cache(maxsize=256)
+def _bwd_op_workspace_bytes(dtype: int, B: int, H: int, T: int, D: int) -> int:
+    return int(_native.load().ca_bwd_op_workspace_bytes(dtype, B, H, T, D))
+
+
+@functools.lru_cache(maxsize=256)
 def _bwd_qkv_workspace_bytes(B: int, H: int, T: int, D: int) -> int:
     return int(_native.load().ca_bwd_qkv_workspace_bytes(B, H, T, D))
 
@@ -98,8 +111,8 @@ def _fwd_qkv_workspace_bytes(B: int, H: int, T: int, D: int) -> int:
 
 def _clear_workspace_sizes() -> None:
     # the sizes follow the workspace cap and the split override
-    for f in (_fwd_workspace_bytes, _bwd_workspace_bytes, _fwd_qkv_workspace_bytes,
-              _bwd_qkv_workspace_bytes):
+    for f in (_fwd_workspace_bytes, _bwd_workspace_bytes, _fwd_op_workspace_bytes,
+              _bwd_op_workspace_bytes, _fwd_qkv_workspace_bytes, _bwd_qkv_workspace_bytes):
         f.cache_clear()
 
 
@@ -182,9 +195,95 @@ def ca_backward(q, k, v, log_gain, out, stats, dout):
     return dq, dk, dv, dg
 
 
+# ---- the operator in the tensors' own type, any head dim up to 128 ---------
+
+_OP_DTYPES = {torch.float32: _native.CA_DTYPE_F32, torch.bfloat16: _native.CA_DTYPE_BF16,
+              torch.float16: _native.CA_DTYPE_F16}
+_MAX_T = 65536              # the fused kernels' sequence limit
+_MAX_ELEMS = (1 << 31) - 1  # and their limit on the elements of a tensor
+
+
+def _fused(q, k, v) -> bool:
+    """Whether the fused kernels serve these tensors.  Head dims with kernels
+    of their own always go there (which reports what they refuse); others up
+    to 128, zero-padded, where the padded problem is within the kernels'
+    limits (shapes of q, k and v that differ stay with the query-tile path,
+    whose matmuls decide)."""
+    D = q.shape[-1]
+    if D in SUPPORTED_HEAD_DIMS:
+        return True
+    if not 0 < D < SUPPORTED_HEAD_DIMS[-1] or k.shape != q.shape or v.shape != q.shape:
+        return False
+    padded = next(d for d in SUPPORTED_HEAD_DIMS if d > D)
+    return q.shape[2] <= _MAX_T and q.numel() // D * padded <= _MAX_ELEMS
+
+
+def _operand(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    x = x.detach()
+    if x.dtype != dtype:
+        x = x.to(dtype)
+    x = x.contiguous()
+    if x.data_ptr() % 16:
+        x = x.clone()
+    return x
+
+
+def _op_forward(q, k, v, log_gain, keep_y):
+    """Output in the operands' type (fp32 for types without kernels of their
+    own), and the fp32 output and row statistics the backward reads (y is None
+    unless ``keep_y`` or it is the output itself)."""
+    lib = _native.load()
+    dev = _check_device(q, k, v, log_gain)
+    B, H, T, D = q.shape
+    if k.shape != q.shape or v.shape != q.shape:
+        raise ValueError(f"q, k, v shapes differ: {tuple(q.shape)} {tuple(k.shape)} {tuple(v.shape)}")
+    if log_gain.numel() != H:
+        raise ValueError(f"log_gain has {log_gain.numel()} entries, expected H={H}")
+    dtype = q.dtype if q.dtype in _OP_DTYPES else torch.float32
+    code = _OP_DTYPES[dtype]
+    qf, kf, vf = _operand(q, dtype), _operand(k, dtype), _operand(v, dtype)
+    gf = _as_f32(log_gain.reshape(H))
+    out = y = None
+    if code != _native.CA_DTYPE_F32 or D not in SUPPORTED_HEAD_DIMS:
+        out = torch.empty((B, H, T, D), device=dev, dtype=dtype)
+    if keep_y or out is None:
+        y = torch.empty((B, H, T, lib.ca_padded_head_dim(D)), device=dev, dtype=torch.float32)
+    stats = torch.empty((B * H * T, 2), device=dev, dtype=torch.float32)
+    nbytes = _fwd_op_workspace_bytes(code, B, H, T, D)
+    ws = torch.empty(max(nbytes, 1), device=dev, dtype=torch.uint8)
+    with _native.on_device(dev):
+        _native.check(lib.ca_fwd_op(qf.data_ptr(), kf.data_ptr(), vf.data_ptr(), code,
+                                    gf.data_ptr(), y.data_ptr() if y is not None else None,
+                                    out.data_ptr() if out is not None else None,
+                                    stats.data_ptr(), ws.data_ptr(), nbytes, B, H, T, D,
+                                    _stream(dev)))
+    return (y if out is None else out), y, stats
+
+
+def _op_backward(q, k, v, log_gain, y, stats, dout):
+    """(dq, dk, dv) in the type _op_forward computed in, and fp32 dlog_gain."""
+    lib = _native.load()
+    dev = _check_device(q, k, v, log_gain, y, stats, dout)
+    B, H, T, D = q.shape
+    dtype = q.dtype if q.dtype in _OP_DTYPES else torch.float32
+    code = _OP_DTYPES[dtype]
+    qf, kf, vf, df = (_operand(x, dtype) for x in (q, k, v, dout))
+    gf, yf, sf = _as_f32(log_gain.reshape(H)), _as_f32(y), _as_f32(stats)
+    dq, dk, dv = (torch.empty((B, H, T, D), device=dev, dtype=dtype) for _ in range(3))
+    dg = torch.empty(H, device=dev, dtype=torch.float32)
+    nbytes = _bwd_op_workspace_bytes(code, B, H, T, D)
+    ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+    with _native.on_device(dev):
+        _native.check(lib.ca_bwd_op(qf.data_ptr(), kf.data_ptr(), vf.data_ptr(), code,
+                                    gf.data_ptr(), yf.data_ptr(), sf.data_ptr(), df.data_ptr(),
+                                    dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dg.data_ptr(),
+                                    ws.data_ptr(), nbytes, B, H, T, D, _stream(dev)))
+    return dq, dk, dv, dg
+
+
 # ---- any head dimension: the query-tile structure over the HIP weight kernels
 #
-# Head dims without a fused kernel (D not in SUPPORTED_HEAD_DIMS) run the
+# Head dims above 128 (and padded problems past the kernels' limits) run the
 # reference operator's own structure (cuda/continuum_attention.py:666-694 and
 # :707-764) on the device: per query tile, fp32 GEMMs for the scores, W.V and
 # the gradient contractions, and the HIP weight kernels (ca_weights_f32,
@@ -276,7 +375,7 @@ class _CAExactTiled(torch.autograd.Function):
             raise ValueError("query_tile must be positive")
         mode = _mode()
         ctx.query_tile = int(query_tile)
-        ctx.fused = q.shape[-1] in SUPPORTED_HEAD_DIMS
+        ctx.fused = _fused(q, k, v)
         ctx.empty = False
         ctx.on_cpu = q.device.type == "cpu"
         check_mode_limits(mode, q.device.type == "cuda", q.dtype, v.dtype, q.shape[2], q.shape[3])
@@ -297,13 +396,14 @@ class _CAExactTiled(torch.autograd.Function):
         if ctx.on_cpu:
             ctx.save_for_backward(q, k, v, log_gain)
             return _cpu.forward(q, k, v, log_gain, ctx.query_tile)
+        if ctx.fused:
+            out, y, stats = _op_forward(q, k, v, log_gain, any(ctx.needs_input_grad))
+            if y is not None:
+                ctx.save_for_backward(q, k, v, log_gain, y, stats)
+            return out.to(v.dtype)
         with torch.autocast(device_type="cuda", enabled=False):
-            if ctx.fused:
-                out, stats = ca_forward(q, k, v, log_gain)
-                ctx.save_for_backward(q, k, v, log_gain, out, stats)
-            else:
-                out = tiled_forward(q, k, v, log_gain, ctx.query_tile)
-                ctx.save_for_backward(q, k, v, log_gain)
+            out = tiled_forward(q, k, v, log_gain, ctx.query_tile)
+            ctx.save_for_backward(q, k, v, log_gain)
         return out.to(v.dtype)
 
     @staticmethod
@@ -318,8 +418,8 @@ class _CAExactTiled(torch.autograd.Function):
             q, k, v, log_gain = ctx.saved_tensors
             dq, dk, dv, dg = _cpu.backward(q, k, v, log_gain, grad_y, ctx.query_tile)
         elif ctx.fused:
-            q, k, v, log_gain, out, stats = ctx.saved_tensors
-            dq, dk, dv, dg = ca_backward(q, k, v, log_gain, out, stats, grad_y)
+            q, k, v, log_gain, y, stats = ctx.saved_tensors
+            dq, dk, dv, dg = _op_backward(q, k, v, log_gain, y, stats, grad_y)
         else:
             q, k, v, log_gain = ctx.saved_tensors
             with torch.autocast(device_type="cuda", enabled=False):
@@ -331,9 +431,9 @@ def continuum_attention(q, k, v, log_gain, query_tile=64):
     """Exact causal Continuum Attention (cuda/continuum_attention.py:768-783).
 
     q, k, v: ``[B, H, T, D]`` (same dtype), log_gain: ``[H]``.  On the GPU,
-    D in {8, 16, 32, 64, 128} runs the fused kernels and any other D the
-    query-tile structure over the HIP weight kernels (``query_tile`` rows at a
-    time); CPU tensors run the float32 CPU path (``cpu.py``).
+    D up to 128 runs the fused kernels and larger D the query-tile structure
+    over the HIP weight kernels (``query_tile`` rows at a time); CPU tensors
+    run the float32 CPU path (``cpu.py``).
     Scores are ``exp(log_gain[h]) / sqrt(D) * q.k``; keys and values are
     linearly interpolated between adjacent positions with half-token end caps
     and integrated exactly.  Returns ``[B, H, T, D]`` in ``v.dtype``.

@@ -90,6 +90,36 @@ int ca_bwd_f32(const float* q, const float* k, const float* v, const float* log_
                float* dv, float* dlog_gain, void* workspace, size_t workspace_bytes, int B, int H,
                int T, int D, void* stream);
 
+/* Element types of the typed entry points below. */
+enum { CA_DTYPE_F32 = 0, CA_DTYPE_BF16 = 1, CA_DTYPE_F16 = 2 };
+
+/* The operator on [B,H,T,D] tensors of element type `dtype` (CA_DTYPE_*) and
+ * any head dim up to 128.  The kernels read 16-bit q, k, v (and dout) as they
+ * are and write the output and gradients rounded once to that type; scores,
+ * weights and sums are fp32.  Head dims other than 8, 16, 32, 64 and 128 run
+ * on rows padded with zeros in the workspace to the next of them
+ * (ca_padded_head_dim; 0: not supported); scores keep 1/sqrt(D).
+ * Forward: out [B,H,T,D] (dtype) and the fp32 output y
+ * [B,H,T,ca_padded_head_dim(D)] that ca_bwd_op reads.  Either may be NULL: out
+ * when y is the result (fp32, unpadded D), y when no backward follows.
+ * stats as in ca_fwd_f32.  q, k, v, out, dout and the gradients are 8-byte
+ * (16-bit types) or 16-byte (fp32) aligned, y 16-byte aligned.
+ * Replaces: the same reference code as ca_fwd_f32 / ca_bwd_f32, with the
+ * casts around it (cuda/continuum_attention.py:666-669, 765-766). */
+int ca_padded_head_dim(int D);
+size_t ca_fwd_op_workspace_bytes(int dtype, int B, int H, int T, int D);
+int ca_fwd_op(const void* q, const void* k, const void* v, int dtype, const float* log_gain,
+              float* y, void* out, float* stats, void* workspace, size_t workspace_bytes, int B,
+              int H, int T, int D, void* stream);
+/* Backward: dq, dk, dv [B,H,T,D] (dtype) and dlog_gain[H] from dout (dtype)
+ * and the forward's y and stats.  In passes (see the workspace cap) 16-bit
+ * dK and dV are summed in fp32 and rounded once, as in ca_bwd_qkv. */
+size_t ca_bwd_op_workspace_bytes(int dtype, int B, int H, int T, int D);
+int ca_bwd_op(const void* q, const void* k, const void* v, int dtype, const float* log_gain,
+              const float* y, const float* stats, const void* dout, void* dq, void* dk, void* dv,
+              float* dlog_gain, void* workspace, size_t workspace_bytes, int B, int H, int T,
+              int D, void* stream);
+
 /* Size of the static scratch array of ca_bwd_f32_noalloc, in MiB. */
 #define CA_NOALLOC_SCRATCH_MB 512
 
@@ -157,8 +187,6 @@ int ca_weights_bwd_f32(const float* scores, const float* grad_weights, float* we
  * operator, and the transpose/reshape of its output in
  * ContinuumSelfAttention.forward (cuda/continuum_attention.py:848-854), and
  * their autograd. */
-enum { CA_DTYPE_F32 = 0, CA_DTYPE_BF16 = 1, CA_DTYPE_F16 = 2 };
-
 size_t ca_fwd_qkv_workspace_bytes(int B, int H, int T, int D);
 int ca_fwd_qkv(const void* qkv, int dtype, const float* rope_cs, const float* log_gain, float* y,
                void* out, float* stats, void* workspace, size_t workspace_bytes, int B, int T,
