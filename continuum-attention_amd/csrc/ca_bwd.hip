@@ -23,7 +23,7 @@
 //                   the owned keys is also spilled, one 32-query column per
 //                   (query tile, key), for the dQ pass.
 //                   Each item also forms its gain partial
-//                   sum_j (k_j - k_0) . dK_j (= sum_ij dS_ij s_ij, since
+//                   sum_j (k_j - k_ref) . dK_j (= sum_ij dS_ij s_ij, since
 //                   s_ij = c q_i . k_j and every row of dS sums to zero).
 //   ca_bwd_dq       dQ = c dS (K - k_ref) over the spilled rows, one work
 //                   item per (slice, 128 queries, chunk of 32-key stages); H

@@ -46,6 +46,8 @@ struct Bwd {
 // wait and the other resident work groups' work.  fp32 at D = 64 runs it on
 // every grid (config 2 dK/dV 0.309 -> 0.291 ms, [1,16,2048,64] 0.162 ->
 // 0.161 ms against the double-buffered two-wave kernel on one box).
+// keys whose mean the gain gradient is formed relative to
+constexpr int kGainRefs = 4;
 // Direction of each item's walk over its query tiles (see the tile loop).
 constexpr bool kDkdvDescending = true;
 
@@ -118,6 +120,9 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
   // K (rotated here when `rope_k`; otherwise it arrives rotated, or without
   // RoPE) and V of this lane's slot: B operands of S /
   // dP', k block kb, element e = d 32kb + 8g + e.
+  // k blocks of dP' formed with the sign changed (kDpFlip): half of those that
+  // hold columns (zero-padded rows of a head dim hd <= 96 leave the fourth empty)
+  const int kflip = P::KB == 4 && hd <= 96 ? 1 : P::KB / 2;
   Limbs kl[P::KB], vl[P::KB];
 #pragma unroll
   for (int kb = 0; kb < P::KB; ++kb) {
@@ -139,7 +144,7 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
         xv[4 * h2 + e] = b[e];
       }
     }
-    if (kb < P::KB / 2) {
+    if (kb < kflip) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) xv[e] = -xv[e];  // see kDpFlip
     }
@@ -239,7 +244,9 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
       // and takes c log2e and the row shift in one fused multiply-add per
       // score, as the forward forms it: the small limb products then round at
       // their own size.  Started from the shift they rounded at |m|, and with
-      // scores of variance 16 the gradients' errors were 1.5 times as large.
+      // scores of variance 16 the gradients' errors were two to three times as
+      // large.  At D = 64 and 128 the scores, and with them the weights, equal
+      // the forward's bit for bit, so that they sum to the Z it divided by.
       f32x4 sacc[2], pacc[2];
 #pragma unroll
       for (int rb = 0; rb < 2; ++rb) {
@@ -249,7 +256,7 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
       prio_mfma_begin<!BF>();
 #pragma unroll
       for (int kb = 0; kb < P::KB; ++kb) {
-        if (P::KB > 1 && kb == P::KB / 2) {
+        if (P::KB > 1 && kb == kflip) {
           pacc[0] = -pacc[0];
           pacc[1] = -pacc[1];
         }
@@ -278,9 +285,10 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
             pacc[1] = -pacc[1];
           }
           const Limbs& vb = P::KB == 1 && st < 3 ? vneg : vl[kb];
-          if (limb_step_used<BF, BF>(st)) sacc[0] = mfma16_step(st, qa[0], kl[kb], sacc[0]);
+          const int ss = limb_step_swapped(st);  // the forward's order, K its first operand
+          if (limb_step_used<BF, BF>(ss)) sacc[0] = mfma16_step(ss, qa[0], kl[kb], sacc[0]);
           if (limb_step_used<false, BF>(st)) pacc[0] = mfma16_step(st, ya[0], vb, pacc[0]);
-          if (limb_step_used<BF, BF>(st)) sacc[1] = mfma16_step(st, qa[1], kl[kb], sacc[1]);
+          if (limb_step_used<BF, BF>(ss)) sacc[1] = mfma16_step(ss, qa[1], kl[kb], sacc[1]);
           if (limb_step_used<false, BF>(st)) pacc[1] = mfma16_step(st, ya[1], vb, pacc[1]);
         }
       }
@@ -413,28 +421,36 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
   // A single-chunk group writes dK/dV; the chunks of a longer group write
   // partials [key of the group][dV, dK][D] that ca_bwd_merge sums.
   // Each item also writes its part of the gain gradient
-  //   dlog_gain = sum_ij dS_ij s_ij = sum_j k_j . dK_j = sum_j (k_j - k_0) . dK_j
+  //   dlog_gain = sum_ij dS_ij s_ij = sum_j k_j . dK_j = sum_j (k_j - k_ref) . dK_j
   // (the last because sum_j dK_j = c sum_i q_i sum_j dS_ij = 0: every row of
-  // dS sums to zero), with k_0 the slice's first key: near-duplicate keys
-  // then contribute small differences instead of cancelling terms.
+  // dS sums to zero), with k_ref the mean of kGainRefs keys spread over the
+  // slice: near-duplicate keys then contribute small differences instead of
+  // cancelling terms, and what rounding leaves of a row's sum is weighed by the
+  // row's mean score relative to a typical key, not to one key.
   float gsum = 0.f;
   const bool owned_key = j >= 1 && j <= kBwdKeys && key_j < T && kb16 < nkb;
   if (owned_key) {
     const float ck = cl2 * kLn2;
-    const E* k0 = view_slice<const E>(Kv, bh, H);
-    const E* kj = k0 + (long long)key_j * Kv.rstride;
+    const E* ks = view_slice<const E>(Kv, bh, H);
+    const E* kj = ks + (long long)key_j * Kv.rstride;
 #pragma unroll
     for (int mb = 0; mb < P::NMB; ++mb) {
       const int d0 = 16 * mb + 4 * g;
       if (d0 < D) {
-        f32x4 a = ld4(kj + d0), b = ld4(k0 + d0);
-        if (rope_k) {
-          a = rope4_in<E>(a, rope_entry(rope_k, key_j, D, d0));
-          b = rope4_in<E>(b, rope_entry(rope_k, 0, D, d0));
+        auto key4 = [&](const E* kp, int key) {
+          const f32x4 x = ld4(kp + d0);
+          return rope_k ? rope4_in<E>(x, rope_entry(rope_k, key, D, d0)) : x;
+        };
+        f32x4 a = key4(kj, key_j);
+        f32x4 b = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < kGainRefs; ++u) {
+          const int key = (int)((long long)u * T / kGainRefs);
+          b += key4(ks + (long long)key * Kv.rstride, key);
         }
         const f32x4 dk = acck[mb] * ck;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) gsum = fmaf(a[r] - b[r], dk[r], gsum);
+        for (int r = 0; r < 4; ++r) gsum = fmaf(fmaf(b[r], -1.0f / kGainRefs, a[r]), dk[r], gsum);
       }
     }
   }

@@ -125,6 +125,10 @@ __host__ __device__ constexpr bool limb_step_used(int st) {
   const bool b_low = st == 1 || st == 2 || st == 4;  // uses b.m or b.l
   return !(ABF && a_low) && !(BBF && b_low);
 }
+// The step that multiplies the same limbs with the operands exchanged.
+__host__ __device__ constexpr int limb_step_swapped(int st) {
+  return st == 0 ? 2 : st == 2 ? 0 : st == 3 ? 4 : st == 4 ? 3 : st;
+}
 // c += a * b over 16 k values (32x32x16 tiles) with bf16-valued a: the three
 // products of a.h, small terms first (the nonzero steps of mfma_x6)
 __device__ __forceinline__ f32x16 mfma_x3_abf(bf16x8 ah, const Limbs& b, f32x16 c) {
