@@ -139,12 +139,12 @@ ca::DqSplit dq_split_for(int BH, int T, int D, const ca::BwdPass& p, bool for_si
 }
 ca::DkdvSplit dkdv_split_for(int BH, int D, int dtype, const ca::BwdPass& p, bool for_sizing) {
   if (g_split.dkdv_tiles > 0) return ca::dkdv_split_chunk(p, g_split.dkdv_tiles);
-  // D = 128: one dK/dV work group per CU instead of two (registers and LDS).
+  // D = 128: two dK/dV work groups per CU; split below two rounds of them.
   // bf16 operands at D <= 64: three per CU, and the split test asks for 1.5
   // rounds of them (9/4 of the two-per-CU count; at [1,16,2048,64] chunks of
   // 16 tiles took 0.277 ms per fwd+bwd against 0.283 ms for 24 and 0.281 ms
   // for 12).
-  // fp32 operands at D = 64 (the single-buffered kernel, three per CU): split
+  // fp32 and fp16 operands at D = 64 (the single-buffered kernel, three per CU): split
   // only below 1.5 rounds of three per CU (config 2, 37 key groups x 32
   // slices, stays unsplit: 24-tile chunks made dK/dV 8 us faster and the
   // dQ launch, which merges their partials, 13 us slower), then from 16-tile
@@ -164,10 +164,10 @@ ca::DkdvSplit dkdv_split_for(int BH, int D, int dtype, const ca::BwdPass& p, boo
   if (!for_sizing) {
     const int two_per_cu = dkdv_resident_groups();
     if (D > 64) {
-      res = two_per_cu / 2;
+      res = two_per_cu;
     } else if (dtype == CA_DTYPE_BF16) {
       res = std::min(two_per_cu * 9 / 4, kDqSplitBound);
-    } else if (dtype == CA_DTYPE_F32 && D == 64) {
+    } else if (D == 64) {
       res = std::min(two_per_cu * 9 / 4, kDqSplitBound);
       want = res;
       const ca::DkdvSplit s =

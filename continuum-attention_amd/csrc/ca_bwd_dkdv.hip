@@ -35,17 +35,20 @@ struct Bwd {
   static constexpr int CPT = (CHUNKS + 255) / 256;
 };
 
-// Waves per SIMD the register budget is set for: bf16 operands need fewer
-// limb registers and fit three (156 VGPRs at D = 64, 41 KB of LDS per work
-// group), which hides more of the segment math's latency (one CA-S layer:
-// 0.137 -> 0.132 ms); fp32 and fp16 operands keep two, except the
-// single-buffered variant (SB): one staged tile (31 KB) and no register
-// prefetch across the tile's work, three waves (168 VGPRs).  SB issues the
-// next tile's loads when its own products are issued, waits at the barrier
-// for the other waves, then stores: the load latency overlaps the barrier
-// wait and the other resident work groups' work.  fp32 at D = 64 runs it on
-// every grid (config 2 dK/dV 0.309 -> 0.291 ms, [1,16,2048,64] 0.162 ->
-// 0.161 ms against the double-buffered two-wave kernel on one box).
+// Waves per SIMD the register budget is set for, and whether the query tile
+// is single-buffered (SB): one staged tile and no register prefetch across
+// the tile's work.  SB issues the next tile's loads when its own products are
+// issued, waits at the barrier for the other waves, then stores: the load
+// latency overlaps the barrier wait and the other resident work groups' work,
+// and the registers and LDS it saves hold another wave per SIMD.
+//   D = 128: SB, two waves (254 VGPRs, 56 KB; double-buffered 307 and 111 KB
+//     held one): [2,16,2048,128] fp32 757 -> 521 us, [1,8,1537,128] 146 -> 113.
+//   D = 32 and 64, fp32 and fp16: SB, three waves (168 VGPRs, 31 KB at 64)
+//     against two ([2,16,2048,64] fp16 284 -> 254 us, [2,16,2048,32] fp32
+//     182 -> 167).
+//   bf16 at D <= 64 (fewer limb registers): double-buffered with three; SB
+//     measured 113.1 against 114.1 us at [1,16,2048,64], 113.4 against 111.1
+//     at [4,16,1001,64] and 148.5 against 145.4 at [2,16,2048,32].
 // keys whose mean the gain gradient is formed relative to
 constexpr int kGainRefs = 4;
 // Direction of each item's walk over its query tiles (see the tile loop).
@@ -53,12 +56,11 @@ constexpr bool kDkdvDescending = true;
 
 template <int D, class E, bool SB>
 constexpr int dkdv_waves_per_simd() {
-  return D > 64 ? 1 : (q_limb_planes<E>() == 1 || SB) ? 3 : 2;
+  return D > 64 ? 2 : (q_limb_planes<E>() == 1 || SB) ? 3 : 2;
 }
-// the single-buffered variant is built for fp32 operands at D = 64
 template <int D, class E>
 constexpr bool dkdv_has_single_buffer() {
-  return D == 64 && std::is_same<E, float>::value;
+  return D == 128 || (D >= 32 && !std::is_same<E, __bf16>::value);
 }
 
 template <int D, class E, bool SB>
