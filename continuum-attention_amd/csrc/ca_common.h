@@ -415,8 +415,8 @@ __device__ __forceinline__ float j2_odd(float y) {
 
 // Forward shares of one segment: L -> left key, R -> right key.
 // x is the signed natural score difference s_r - s_l; pl/pr are the endpoint
-// weights relative to the row shift.  Used by the materialised-weight row
-// kernels; the fused operator uses seg_shares below.
+// weights relative to the row shift.  Used by the three-pass weight row
+// kernel; the other kernels use the symmetric form below.
 // Both branches are evaluated and selected (no divergent control flow).
 __device__ __forceinline__ void seg_shares_x(float x, float pl, float pr, float& L, float& R) {
   const float dp = pr - pl;
@@ -433,8 +433,8 @@ __device__ __forceinline__ void seg_shares_x(float x, float pl, float pr, float&
   L = small ? ls : lc;
 }
 
-// Forward shares and score-gradient contributions of one segment (row
-// kernels).  gl/gr are the centred, 1/Z-scaled weight gradients
+// Forward shares and score-gradient contributions of one segment
+// (three-pass row kernel).  gl/gr are the centred, 1/Z-scaled weight gradients
 // g = (dY.v - Dl) / Z.
 __device__ __forceinline__ void seg_shares_grad_x(float x, float pl, float pr, float gl, float gr,
                                                   float& L, float& R, float& dL, float& dR) {
@@ -457,7 +457,7 @@ __device__ __forceinline__ void seg_shares_grad_x(float x, float pl, float pr, f
   dL = fmaf(gl, L - xm, gr * xm);
 }
 
-// ---- segments of the fused operator: symmetric half-difference form ---------
+// ---- segments in the symmetric half-difference form -------------------------
 // With h = (s_r - s_l) ln2 / 2 (half the natural score difference) and the
 // endpoint sum and difference S = p_r + p_l, dp = p_r - p_l, the moments of a
 // segment are, up to the common factor 4 below,
@@ -479,7 +479,7 @@ __device__ __forceinline__ void seg_shares_grad_x(float x, float pl, float pr, f
 // closed forms above), and half their rounding error: the series stays
 // accurate to a larger |h|, so the quotients start where they cancel less.
 //
-// The factor 4 is not divided out: the kernels run on endpoint weights a
+// The factor 4 is not divided out: the fused kernels run on endpoint weights a
 // quarter as large (p = 2^(s - m - kShareShift) with integer m, exact), so
 // that these shares are the weights relative to m themselves.
 constexpr float kHalfLn2 = 0.34657359027997265f;
@@ -501,19 +501,21 @@ __device__ __forceinline__ void seg_mean_tilt(float h, float pl, float pr, float
   a = small ? as : ac;
   d = small ? ds : dc;
 }
-// Shares (times 4) of one segment from log2-unit scores sl/sr and p = 2^s.
-__device__ __forceinline__ void seg_shares(float sl, float sr, float pl, float pr, float& L,
-                                           float& R) {
+// Shares (times 4) of one segment.
+__device__ __forceinline__ void seg_shares_h(float h, float pl, float pr, float& L, float& R) {
   float a, d;
-  seg_mean_tilt((sr - sl) * kHalfLn2, pl, pr, a, d);
+  seg_mean_tilt(h, pl, pr, a, d);
   R = a + d;
   L = a - d;
 }
-// The same with the score gradients; gl/gr as for seg_shares_grad_x.
-__device__ __forceinline__ void seg_shares_grad(float sl, float sr, float pl, float pr, float gl,
-                                                float gr, float& L, float& R, float& dL,
-                                                float& dR) {
-  const float h = (sr - sl) * kHalfLn2;
+// The same from log2-unit scores sl/sr and p = 2^s.
+__device__ __forceinline__ void seg_shares(float sl, float sr, float pl, float pr, float& L,
+                                           float& R) {
+  seg_shares_h((sr - sl) * kHalfLn2, pl, pr, L, R);
+}
+// Shares and score gradients (times 4); gl/gr as for seg_shares_grad_x.
+__device__ __forceinline__ void seg_shares_grad_h(float h, float pl, float pr, float gl, float gr,
+                                                  float& L, float& R, float& dL, float& dR) {
   const float dp = pr - pl, sp = pr + pl;
   const float inv_h = fast_rcp(h);
   const float ac = dp * inv_h;
@@ -531,6 +533,11 @@ __device__ __forceinline__ void seg_shares_grad(float sl, float sr, float pl, fl
   L = a - d;
   dR = fmaf(gr, R, -t);
   dL = fmaf(gl, L, t);
+}
+__device__ __forceinline__ void seg_shares_grad(float sl, float sr, float pl, float pr, float gl,
+                                                float gr, float& L, float& R, float& dL,
+                                                float& dR) {
+  seg_shares_grad_h((sr - sl) * kHalfLn2, pl, pr, gl, gr, L, R, dL, dR);
 }
 
 __device__ __forceinline__ float wave_max(float x) {
