@@ -9,12 +9,14 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import importlib.util
 import os
 
 import torch  # must be imported first: the library binds torch's HIP runtime
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libca_hip.so")
+TORCH_EXT_PATH = os.path.join(HERE, "_ca_torch.so")
 
 CA_OK = 0
 CA_ERR_INVALID = 1
@@ -129,6 +131,27 @@ def load() -> ctypes.CDLL:
         lib.ca_set_workspace_cap(int(float(cap_mb) * (1 << 20)))
     _lib = lib
     return lib
+
+
+_ext = None
+
+
+def torch_ext():
+    """The native autograd functions (csrc/ca_torch.cpp), loaded once.  Its
+    entries return None for a call that is not the plain case; the caller then
+    runs its Python function."""
+    global _ext
+    if _ext is None:
+        load()
+        if not os.path.exists(TORCH_EXT_PATH):
+            raise RuntimeError(
+                f"continuum-attention_amd: native module {TORCH_EXT_PATH} is not built; run "
+                "`python continuum-attention_amd/build.py` (or __graft_entry__.build())")
+        spec = importlib.util.spec_from_file_location("_ca_torch", TORCH_EXT_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _ext = module
+    return _ext
 
 
 def check(rc: int) -> None:

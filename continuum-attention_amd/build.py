@@ -1,7 +1,8 @@
-"""Builds libca_hip.so in-tree with hipcc for gfx950.
+"""Builds libca_hip.so (hipcc for gfx950) and _ca_torch.so (the torch binding of
+its autograd functions, host code only) in-tree.
 
 Usage: python continuum-attention_amd/build.py [--verbose]
-The shared library is written next to this file and loaded by _native.py.
+The shared libraries are written next to this file and loaded by _native.py.
 """
 from __future__ import annotations
 
@@ -17,6 +18,8 @@ LIB = os.path.join(HERE, "libca_hip.so")
 SOURCES = ["ca_fwd.hip", "ca_bwd.hip", "ca_bwd_dkdv.hip", "ca_weights.hip", "ca_norm.hip",
            "ca_optim.hip", "ca_swiglu.hip", "ca_abi.hip", "ca_noalloc.hip"]
 ARCH = os.environ.get("CA_OFFLOAD_ARCH", "gfx950")
+TORCH_SOURCE = "ca_torch.cpp"
+TORCH_EXT = os.path.join(HERE, "_ca_torch.so")
 
 HIPCC_FLAGS = [
     f"--offload-arch={ARCH}",
@@ -76,6 +79,37 @@ def _jobs() -> int:
     return max(1, min(8, n, len(SOURCES)))
 
 
+def _run(cmd, what: str, verbose: bool) -> None:
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{what} failed:\n{res.stdout}{res.stderr}")
+
+
+def compile_torch_ext(obj: str, verbose: bool) -> None:
+    """ca_torch.cpp against the installed torch's headers (host code only)."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    inc = [*include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-DTORCH_EXTENSION_NAME=_ca_torch",
+          "-DTORCH_API_INCLUDE_EXTENSION_H", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          *(x for d in inc for x in ("-isystem", d)), "-c", os.path.join(CSRC, TORCH_SOURCE),
+          "-o", obj], f"g++ on {TORCH_SOURCE}", verbose)
+
+
+def link_torch_ext(obj: str, verbose: bool) -> None:
+    from torch.utils.cpp_extension import library_paths
+    tmp = TORCH_EXT + ".tmp"
+    _run(["g++", "-shared", obj, "-o", tmp, *(f"-L{d}" for d in library_paths()), "-ltorch",
+          "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_python", f"-L{HERE}",
+          "-l:" + os.path.basename(LIB), "-Wl,-rpath,$ORIGIN"], "torch binding link", verbose)
+    os.replace(tmp, TORCH_EXT)
+
+
 def build(verbose: bool = False, extra_flags=None) -> str:
     build_dir = os.path.join(HERE, "_build")
     os.makedirs(build_dir, exist_ok=True)
@@ -90,7 +124,9 @@ def build(verbose: bool = False, extra_flags=None) -> str:
         return src, cmd, obj, res.returncode, out
 
     objs = []
+    ext_obj = os.path.join(build_dir, TORCH_SOURCE.replace(".cpp", ".o"))
     with concurrent.futures.ThreadPoolExecutor(_jobs()) as pool:
+        ext = pool.submit(compile_torch_ext, ext_obj, verbose)
         for src, cmd, obj, rc, out in pool.map(compile_one, SOURCES):
             if verbose:
                 print(" ".join(cmd), flush=True)
@@ -99,12 +135,14 @@ def build(verbose: bool = False, extra_flags=None) -> str:
             if verbose and out.strip():
                 print(out, flush=True)
             objs.append(obj)
+        ext.result()
     tmp = LIB + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}{res.stderr}")
     os.replace(tmp, LIB)
+    link_torch_ext(ext_obj, verbose)
     return LIB
 
 

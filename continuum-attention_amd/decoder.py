@@ -26,8 +26,8 @@ from torch import nn
 from torch.nn import functional as F
 
 from . import _native
-from .ops import (SUPPORTED_HEAD_DIMS, _bwd_qkv_workspace_bytes, _fwd_qkv_workspace_bytes, _mode,
-                  check_mode_limits, continuum_attention)
+from .ops import (SUPPORTED_HEAD_DIMS, _UNLIMITED_MODES, _bwd_qkv_workspace_bytes,
+                  _fwd_qkv_workspace_bytes, _mode, check_mode_limits, continuum_attention)
 
 _DTYPE_CODE = {torch.float32: _native.CA_DTYPE_F32, torch.bfloat16: _native.CA_DTYPE_BF16,
                torch.float16: _native.CA_DTYPE_F16}
@@ -193,6 +193,10 @@ class RMSNorm(nn.Module):
 
     def forward(self, x):
         if self._fusable(x):
+            if not torch.compiler.is_compiling():
+                y = _native.torch_ext().rmsnorm(x, self.weight, self.eps, self._out_dtype())
+                if y is not None:
+                    return y
             return _RMSNormFn.apply(x, self.weight, self.eps, self._out_dtype())
         return self._composition(x)
 
@@ -201,6 +205,10 @@ class RMSNorm(nn.Module):
         the norm that reads its result, fused when the input qualifies."""
         if (self._fusable(x) and res.shape == x.shape and res.device == x.device
                 and res.dtype in _DTYPE_CODE):
+            if not torch.compiler.is_compiling():
+                r = _native.torch_ext().add_rmsnorm(x, res, self.weight, self.eps, self._out_dtype())
+                if r is not None:
+                    return r
             return _AddRMSNormFn.apply(x, res, self.weight, self.eps, self._out_dtype())
         s = x + res
         return s, self(s)
@@ -346,8 +354,19 @@ def rope_continuum_attention(qkv, log_gain, theta, heads, query_tile=64):
     """``[B, T, 3C]`` qkv projection output -> ``[B, T, C]`` attention output
     (before the output projection), in qkv's dtype; see _RopeContinuumAttention.
     ``theta=None``: no rotary embedding (the prologue only splits the heads)."""
-    return _RopeContinuumAttention.apply(qkv, log_gain, None if theta is None else float(theta),
-                                         int(heads), int(query_tile))
+    theta, heads, query_tile = None if theta is None else float(theta), int(heads), int(query_tile)
+    # the plain case (see csrc/ca_torch.cpp) runs _RopeContinuumAttention's native counterpart
+    if (isinstance(qkv, torch.Tensor) and qkv.is_cuda and qkv.dim() == 3 and query_tile > 0
+            and qkv.dtype in _DTYPE_CODE and heads > 0 and _mode() in _UNLIMITED_MODES
+            and not torch.compiler.is_compiling()):
+        T, D = qkv.shape[1], qkv.shape[2] // 3 // heads
+        cs = (rope_cos_sin(T, D, theta, qkv.device, qkv.dtype)
+              if theta is not None and D in SUPPORTED_HEAD_DIMS and T > 0 else None)
+        if theta is None or cs is not None:
+            y = _native.torch_ext().rope_attention(qkv, log_gain, cs, heads)
+            if y is not None:
+                return y
+    return _RopeContinuumAttention.apply(qkv, log_gain, theta, heads, query_tile)
 
 
 # Largest vocabulary whose embedding gradient is formed as a one-hot GEMM

@@ -43,6 +43,7 @@ from . import _native
 from . import cpu as _cpu
 
 _MODES = ("dense", "prefix", "fused", "prefix_v5", "prefix_v6")
+_UNLIMITED_MODES = ("dense", "prefix")  # modes check_mode_limits has no limit for
 SUPPORTED_HEAD_DIMS = (8, 16, 32, 64, 128)
 
 
@@ -438,5 +439,11 @@ def continuum_attention(q, k, v, log_gain, query_tile=64):
     linearly interpolated between adjacent positions with half-token end caps
     and integrated exactly.  Returns ``[B, H, T, D]`` in ``v.dtype``.
     """
+    # the plain case (see csrc/ca_torch.cpp) runs _CAExactTiled's native counterpart
+    if (isinstance(q, torch.Tensor) and q.is_cuda and type(query_tile) is int and query_tile > 0
+            and _mode() in _UNLIMITED_MODES and not torch.compiler.is_compiling()):
+        y = _native.torch_ext().op(q, k, v, log_gain)
+        if y is not None:
+            return y
     return _CAExactTiled.apply(q.contiguous(), k.contiguous(), v.contiguous(), log_gain,
                                int(query_tile))

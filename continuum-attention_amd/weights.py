@@ -126,4 +126,8 @@ def continuous_attention_weights(logits: torch.Tensor) -> torch.Tensor:
         raise ValueError("This benchmark requires square full-sequence causal attention")
     if logits.device.type == "cpu":
         return _cpu.continuous_attention_weights(logits)
+    if logits.is_cuda and not torch.compiler.is_compiling():
+        w = _native.torch_ext().weights(logits)  # the plain case, natively
+        if w is not None:
+            return w
     return _CAWeights.apply(logits)
