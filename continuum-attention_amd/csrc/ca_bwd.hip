@@ -55,13 +55,14 @@ namespace ca {
 // last tile) are written as zeros, so the dK/dV kernel stages whole tiles
 // without bounds tests.
 template <int D, class E>
-__global__ __launch_bounds__(256) void ca_bwd_prep_kernel(View Qv, const float* __restrict__ rope,
-                                                          View dYv,
+__global__ __launch_bounds__(256) void ca_bwd_prep_kernel(View Qv, View Kv,
+                                                          const float* __restrict__ log_gain,
+                                                          const float* __restrict__ rope, View dYv,
                                                           const float* __restrict__ out,
                                                           const float* __restrict__ stats,
                                                           __bf16* __restrict__ limbs,
                                                           float* __restrict__ qstat, int H, int T,
-                                                          int row0, int ntiles, int rows) {
+                                                          int row0, int ntiles, int rows, int hd) {
   constexpr int C8 = D / 8;
   const int tix = blockIdx.x * 256 + threadIdx.x;
   const int row = tix / C8, c = tix % C8;  // row = bh * 32 ntiles + (t - row0)
@@ -94,6 +95,36 @@ __global__ __launch_bounds__(256) void ca_bwd_prep_kernel(View Qv, const float* 
     x += dy[u][0] * y[u][0] + dy[u][1] * y[u][1] + dy[u][2] * y[u][2] + dy[u][3] * y[u][3];
 #pragma unroll
   for (int o = C8 / 2; o >= 1; o >>= 1) x += __shfl_xor(x, o);
+  if (hd != D) {
+    // Zero-padded rows: the dK/dV kernel sums dS s with the scores relative to
+    // m + kShareShift, so a shift r near the row's weighted mean score keeps
+    // what rounding leaves of the row's sum of dS small in it.  With s_ref the
+    // score of a mean key and L = log2(Z 2^m / keys) the row's log mean weight,
+    // r = 2 L - s_ref is that mean for normally distributed scores (L - s_ref
+    // is half their variance) and near it for peaked rows.  Moved by whole
+    // octaves, weights and 1/Z scale exactly.
+    float sref = 0.f;
+    const E* kp = view_slice<const E>(Kv, bh, H) + 8 * c;
+#pragma unroll
+    for (int k = 0; k < kGainRefs; ++k) {
+      const E* kk = kp + (long long)((long long)k * T / kGainRefs) * Kv.rstride;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const f32x4 kx = ld4(kk + 4 * u);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sref = fmaf(qq[u][e], kx[e], sref);
+      }
+    }
+#pragma unroll
+    for (int o = C8 / 2; o >= 1; o >>= 1) sref += __shfl_xor(sref, o);
+    sref *= head_scale_log2(log_gain, bh % H, hd) * (1.0f / kGainRefs);
+    const float lmean = m - __log2f(invz) - __log2f((float)(t + 1));
+    const float n = rintf(m - (2.0f * lmean - sref)) + kShareShift;
+    if (ok && fabsf(n) < 48.f) {  // also false for rows with NaN or infinite scores
+      m -= n;
+      invz *= fast_exp2(-n);
+    }
+  }
   constexpr int QL = q_limb_planes<E>();
   __bf16* tile = limbs + ((size_t)bh * ntiles + r / 32) * limb_tile_elems(D, QL + 3) +
                  (r % 32) * D + 8 * c;
@@ -622,8 +653,9 @@ hipError_t launch_bwd(const BwdIO& io, const BwdWork& ws, const BwdPass& pass, c
   const int rows = BH * 32 * ntiles;
   timer_begin(kBwdPrep, stream);
   hipLaunchKernelGGL((ca_bwd_prep_kernel<D, E>), dim3((rows * (D / 8) + 255) / 256), dim3(256), 0,
-                     stream, io.q, io.rope, io.dout, io.y, io.stats, ws.limbs, ws.qstat, H, T,
-                     pass.row0, ntiles, rows);
+                     stream,
+                     io.q, io.k, io.log_gain, io.rope, io.dout, io.y, io.stats, ws.limbs, ws.qstat, H, T,
+                     pass.row0, ntiles, rows, io.head_dim);
   timer_end(kBwdPrep, stream);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;

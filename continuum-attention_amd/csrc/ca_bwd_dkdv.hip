@@ -49,8 +49,6 @@ struct Bwd {
 //   bf16 at D <= 64 (fewer limb registers): double-buffered with three; SB
 //     measured 113.1 against 114.1 us at [1,16,2048,64], 113.4 against 111.1
 //     at [4,16,1001,64] and 148.5 against 145.4 at [2,16,2048,32].
-// keys whose mean the gain gradient is formed relative to
-constexpr int kGainRefs = 4;
 // Direction of each item's walk over its query tiles (see the tile loop).
 constexpr bool kDkdvDescending = true;
 
@@ -157,6 +155,10 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
   // with a single k block the sign changes between its limb products (kDpFlip)
   Limbs vneg;
   if constexpr (P::KB == 1) vneg = limbs_neg(vl[0]);
+
+  // zero-padded rows: the gain gradient is summed as dS s (see the epilogue)
+  const bool gain_direct = hd != D;
+  float gdir = 0.f;
 
   f32x4 accv[P::NMB], acck[P::NMB];
 #pragma unroll
@@ -357,6 +359,13 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
       else
         segments(std::false_type{});
 
+      if (gain_direct) {
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) gdir = fmaf(dout_s[rb][r], sacc[rb][r], gdir);
+      }
+
       // ---- dS of (query tile qt, the block's keys) for the dQ pass ----
       if (ds_lane) {
         float* col = dsbuf + ds_tile + (size_t)ds_key * kDsColFloats + 4 * g;
@@ -429,9 +438,17 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
   // slice: near-duplicate keys then contribute small differences instead of
   // cancelling terms, and what rounding leaves of a row's sum is weighed by the
   // row's mean score relative to a typical key, not to one key.
+  // Zero-padded head dims sum dS_ij s_ij itself, as the query-tile path that
+  // serves larger ones does, with s_ij relative to a shift near the row's mean
+  // score (the prep kernel's choice): for large scores, whose mean lies far
+  // from a typical key's, the error is about half (gain gradient at
+  // [2,3,500,48] mixed keys 9.7e-7 against 2.9e-6, query tiles 1.5e-6), for 1% more
+  // of the kernel's time.
   float gsum = 0.f;
   const bool owned_key = j >= 1 && j <= kBwdKeys && key_j < T && kb16 < nkb;
-  if (owned_key) {
+  if (gain_direct) {
+    gsum = owned_key ? gdir * kLn2 : 0.f;
+  } else if (owned_key) {
     const float ck = cl2 * kLn2;
     const E* ks = view_slice<const E>(Kv, bh, H);
     const E* kj = ks + (long long)key_j * Kv.rstride;

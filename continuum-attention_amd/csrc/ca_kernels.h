@@ -439,6 +439,9 @@ __host__ __device__ inline int bwd_pass_tiles(const BwdPass& p) { return p.qb - 
 template <class E> __host__ __device__ constexpr int q_limb_planes() {
   return std::is_same<E, __bf16>::value ? 1 : 3;
 }
+// Keys of a slice, evenly spread, whose mean serves as its typical key in the
+// gain gradient.
+constexpr int kGainRefs = 4;
 // kDpFlip.  The matrix cores round their fp32 sums slightly downwards,
 // whatever the sign (about 2^-28 of the accumulator per dP' element,
 // measured): a bias common to a row's weight gradients, which the row's dS
