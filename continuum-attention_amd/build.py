@@ -55,12 +55,7 @@ _FINITE_MATH = ["-fno-honor-nans", "-fno-honor-infinities"]
 # loops as contraction across statements.
 _ATTN = _FINITE_MATH + ["-ffp-contract=on"]
 
-# Per-source flags: the dK/dV kernel schedules better with LLVM's max-ILP
-# machine-scheduler strategy (about 2% faster); the other kernels are slower
-# with it, so it applies to that translation unit only.
-SOURCE_FLAGS = {"ca_fwd.hip": _ATTN,
-                "ca_bwd.hip": _ATTN,
-                "ca_bwd_dkdv.hip": _ATTN + ["-mllvm", "-amdgpu-sched-strategy=max-ilp"]}
+SOURCE_FLAGS = {"ca_fwd.hip": _ATTN, "ca_bwd.hip": _ATTN, "ca_bwd_dkdv.hip": _ATTN}
 
 
 def hipcc() -> str:

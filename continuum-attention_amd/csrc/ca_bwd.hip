@@ -205,8 +205,7 @@ __device__ __forceinline__ void merge_kv_group(const float* __restrict__ kv_part
                                                int kv_part_items, bool kv_f32) {
   constexpr int C4 = D / 4;
   const int tid = threadIdx.x + 256 * slice;
-  int first = 0;  // item index of the group's chunk 0 (multi-chunk groups come first)
-  for (int gg = 0; gg < wg; ++gg) first += dkdv_group_chunks(gg, pass, kv_chunk);
+  const int first = dkdv_items_before(wg, pass, kv_chunk);  // item of the group's chunk 0
   const int nch = dkdv_group_chunks(wg, pass, kv_chunk);
   const bool accumulate = dkdv_qt0(wg) < pass.qa;
   const f32x4* part = reinterpret_cast<const f32x4*>(
@@ -279,12 +278,8 @@ __global__ __launch_bounds__(256, (std::is_same<E, __bf16>::value && D <= 64 ? 4
   // split chunks keep the grid balanced either way).
   const int item = n_items - 1 - (int)blockIdx.x / BH;
   // item -> (group, chunk), heaviest groups of the pass first
-  int qg = pass.g1 - 1, ch = item, nch = dq_group_chunks(qg, T, chunk);
-  while (ch >= nch && qg > pass.g0) {
-    ch -= nch;
-    --qg;
-    nch = dq_group_chunks(qg, T, chunk);
-  }
+  const ItemPos pos = dq_find_item(item, T, pass.g0, pass.g1, chunk);
+  const int qg = pass.g1 - 1 - pos.group, ch = pos.chunk, nch = pos.chunks;
   const int gstages = dq_group_stages(qg, T);
   const int clen = (gstages + nch - 1) / nch;
   const int st_lo = ch * clen;
@@ -524,8 +519,7 @@ __global__ __launch_bounds__(256) void ca_bwd_merge_kernel(const float* __restri
   const int m = blockIdx.x / NS;
   const int bh = m % BH, gi = m / BH;
   const int qg = pass.g1 - 1 - gi;
-  int first = 0;  // item index of the group's chunk 0
-  for (int gg = pass.g1 - 1; gg > qg; --gg) first += dq_group_chunks(gg, T, chunk);
+  const int first = dq_items_before(gi, T, pass.g0, pass.g1, chunk);  // item of the group's chunk 0
   const int nch = dq_group_chunks(qg, T, chunk);
   const f32x4* part = reinterpret_cast<const f32x4*>(dq_part + ((size_t)bh * n_part + first) * kDqRows * D);
   E* dQs = view_slice<E>(dQv, bh, H);

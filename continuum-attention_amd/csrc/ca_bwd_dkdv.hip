@@ -1,8 +1,5 @@
 // dK and dV of the Continuum Attention backward (gfx950): the ca_bwd_dkdv
-// kernel of the backward described in ca_bwd.hip, in a translation unit of
-// its own so that it can be compiled with its own instruction-scheduling
-// strategy (build.py: max-ilp here, measured 2% faster for this kernel and
-// slower for the others).
+// kernel of the backward described in ca_bwd.hip.
 //
 // Score-tile layout: the 16x16 result of S / dP' puts slot j
 // (key 14*kb - 1 + j) in lane j of each 16-lane row and queries 4*(l/16) + r
@@ -46,19 +43,19 @@ struct Bwd {
 //   D = 32 and 64, fp32 and fp16: SB, three waves (168 VGPRs, 31 KB at 64)
 //     against two ([2,16,2048,64] fp16 284 -> 254 us, [2,16,2048,32] fp32
 //     182 -> 167).
-//   bf16 at D <= 64 (fewer limb registers): double-buffered with three; SB
-//     measured 113.1 against 114.1 us at [1,16,2048,64], 113.4 against 111.1
-//     at [4,16,1001,64] and 148.5 against 145.4 at [2,16,2048,32].
+//   bf16 (fewer limb registers) at D = 32 and 64: SB, four waves (128 VGPRs,
+//     21 KB) against three double-buffered ([1,16,2048,64] 114 -> 107 us,
+//     [2,16,2048,64] 193 -> 189).
 // Direction of each item's walk over its query tiles (see the tile loop).
 constexpr bool kDkdvDescending = true;
 
 template <int D, class E, bool SB>
 constexpr int dkdv_waves_per_simd() {
-  return D > 64 ? 2 : (q_limb_planes<E>() == 1 || SB) ? 3 : 2;
+  return D > 64 ? 2 : q_limb_planes<E>() == 1 ? 4 : SB ? 3 : 2;
 }
 template <int D, class E>
 constexpr bool dkdv_has_single_buffer() {
-  return D == 128 || (D >= 32 && !std::is_same<E, __bf16>::value);
+  return D >= 32;
 }
 
 template <int D, class E, bool SB>
@@ -88,15 +85,10 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
   // item -> (key-block group, chunk of its query tiles in this pass)
   int wg = item, ch = 0, nch = 1;
   if (chunk < pass.qb - pass.qa) {
-    const int G = pass.kv_groups;
-    wg = 0;
-    ch = item;
-    nch = dkdv_group_chunks(0, pass, chunk);
-    while (ch >= nch && wg < G - 1) {
-      ch -= nch;
-      ++wg;
-      nch = dkdv_group_chunks(wg, pass, chunk);
-    }
+    const ItemPos pos = dkdv_find_item(item, pass, chunk);
+    wg = pos.group;
+    ch = pos.chunk;
+    nch = pos.chunks;
   }
   const int w0 = kDkdvKeys * wg;
 
@@ -111,8 +103,9 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
 
   const float cl2 = head_scale_log2(log_gain, bh % H, hd);
 
-  // Stale LDS bits must not reach an MFMA as NaN through padding columns.
-  {
+  // Stale LDS bits must not reach an MFMA as NaN through padding columns
+  // (D = 8: the transposed reads take 16 columns).
+  if (D < 16) {
     unsigned* z = reinterpret_cast<unsigned*>(&tiles[0][0]);
     for (int e = tid; e < NBUF * P::TILE / 2; e += 256) z[e] = 0u;
   }

@@ -62,24 +62,6 @@ __device__ __forceinline__ int arow_of_key(int k) {
   return (((k >> 2) & 3) << 3) | (((k >> 4) & 1) << 2) | (k & 3);
 }
 
-// Item decoding: items are (group g, split s) in descending g, then s.
-__device__ __forceinline__ void fwd_decode_item(int item, int G, int T, int C, int& g, int& s,
-                                                int& nsplit) {
-  const int ntiles_all = (T + 31) / 32;
-  for (int gg = G - 1; gg >= 0; --gg) {
-    int nt = min(4 * gg + 4, ntiles_all);
-    int ns = (nt + C - 1) / C;
-    if (item < ns) {
-      g = gg;
-      s = item;
-      nsplit = ns;
-      return;
-    }
-    item -= ns;
-  }
-  g = -1; s = 0; nsplit = 0;
-}
-
 // q . k of key `key` (RoPE applied to the key when `rope`), reduced over the
 // two lane halves that hold the query's halves.
 template <int D, class E>
@@ -130,9 +112,9 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
 
   const int bh = blockIdx.x % BH;
   const int item = blockIdx.x / BH;
-  int g, split, nsplit;
-  fwd_decode_item(item, G, T, C, g, split, nsplit);
-  if (g < 0) return;
+  const ItemPos pos = fwd_find_item(item, G, T, C);
+  const int g = G - 1 - pos.group, split = pos.chunk, nsplit = pos.chunks;
+  if (nsplit == 0) return;
 
   const int ntiles_all = (T + 31) / 32;
   const int nt = min(4 * g + 4, ntiles_all);
@@ -632,9 +614,9 @@ __global__ __launch_bounds__(512, (fwd16_waves_per_simd<D, E, ROPE>())) void ca_
 
   const int bh = blockIdx.x % BH;
   const int item = blockIdx.x / BH;
-  int g, split, nsplit;
-  fwd_decode_item(item, G, T, C, g, split, nsplit);
-  if (g < 0) return;
+  const ItemPos pos = fwd_find_item(item, G, T, C);
+  const int g = G - 1 - pos.group, split = pos.chunk, nsplit = pos.chunks;
+  if (nsplit == 0) return;
 
   const int ntiles_all = (T + 31) / 32;
   const int nt = min(4 * g + 4, ntiles_all);

@@ -11,11 +11,53 @@
 
 namespace ca {
 
+// Work items.  A grid's groups are cut into chunks and its items numbered group
+// by group, from the group with most chunks (group 0 in this order) to those
+// with fewest; count(c) is how many groups have at least c chunks, so the
+// groups with exactly c are the contiguous run [count(c + 1), count(c)).  Items
+// are found and counted in one step per chunk count (at most a few dozen)
+// instead of a division per group, a serial chain at the start of every work
+// group (T = 8192: 64 forward and 147 dK/dV groups).
+struct ItemPos {
+  int group, chunk, chunks;  // position in that order; chunks = 0: past the last item
+};
+template <class Count>
+__host__ __device__ inline ItemPos find_item(int item, int max_chunks, Count count) {
+  int g0 = 0;
+  for (int c = max_chunks; c >= 1; --c) {
+    const int g1 = count(c), n = (g1 - g0) * c;
+    if (item < n) return ItemPos{g0 + item / c, item % c, c};
+    item -= n;
+    g0 = g1;
+  }
+  return ItemPos{0, 0, 0};
+}
+// items of the groups before group g
+template <class Count>
+__host__ __device__ inline int items_before(int g, int max_chunks, Count count) {
+  int n = 0;
+  for (int c = 1; c <= max_chunks; ++c) {
+    const int k = count(c);
+    n += k < g ? k : g;
+  }
+  return n;
+}
+
 // Forward work decomposition: 128-query groups, 32-key weight tiles, splits of
-// at most C tiles per work item.
+// at most C tiles per work item.  Groups are numbered from the last (longest
+// rows) down: group G-1-n is n-th.
 inline int fwd_group_tiles(int g, int T) {
   const int all = (T + 31) / 32;
   return (4 * g + 4 < all) ? 4 * g + 4 : all;
+}
+__host__ __device__ inline ItemPos fwd_find_item(int item, int G, int T, int C) {
+  const int all = (T + 31) / 32;
+  const int longest = 4 * G < all ? 4 * G : all;
+  // groups g with min(4g + 4, all) > x: none when all <= x, else g >= x / 4
+  return find_item(item, (longest + C - 1) / C, [=](int c) {
+    const int x = (c - 1) * C;
+    return all > x ? G - x / 4 : 0;
+  });
 }
 inline int fwd_max_splits(int T, int C) {
   const int G = (T + 127) / 128;
@@ -172,6 +214,21 @@ __host__ __device__ inline int dq_group_stages(int qg, int T) {
 __host__ __device__ inline int dq_group_chunks(int qg, int T, int chunk) {
   return (dq_group_stages(qg, T) + chunk - 1) / chunk;
 }
+// dQ groups g1-1 .. g0 in that order (position n is group g1-1-n)
+__host__ __device__ inline int dq_groups_with(int c, int T, int g0, int g1, int chunk) {
+  const int x = (c - 1) * chunk;  // stages = min(4g + 4, num_q_tiles) > x
+  if (num_q_tiles(T) <= x) return 0;
+  const int lo = x / kDqTiles > g0 ? x / kDqTiles : g0;
+  return lo < g1 ? g1 - lo : 0;
+}
+__host__ __device__ inline ItemPos dq_find_item(int item, int T, int g0, int g1, int chunk) {
+  return find_item(item, dq_group_chunks(g1 - 1, T, chunk),
+                   [=](int c) { return dq_groups_with(c, T, g0, g1, chunk); });
+}
+__host__ __device__ inline int dq_items_before(int n, int T, int g0, int g1, int chunk) {
+  return items_before(n, dq_group_chunks(g1 - 1, T, chunk),
+                      [=](int c) { return dq_groups_with(c, T, g0, g1, chunk); });
+}
 struct DqSplit {
   int chunk;         // key stages per chunk (upper bound)
   int items;         // work items per slice
@@ -240,6 +297,23 @@ __host__ __device__ inline int dkdv_group_tiles(int wg, const BwdPass& p) {
 }
 __host__ __device__ inline int dkdv_group_chunks(int wg, const BwdPass& p, int chunk) {
   return (dkdv_group_tiles(wg, p) + chunk - 1) / chunk;
+}
+// key groups (from 0 up) of the pass with at least c chunks: their tiles from
+// floor(56 wg / 32) = floor(7 wg / 4) on number more than (c - 1) chunk
+static_assert(kDkdvKeys * 4 == 7 * 32, "dkdv_groups_with counts floor(7 wg / 4)");
+__host__ __device__ inline int dkdv_groups_with(int c, const BwdPass& p, int chunk) {
+  const int x = (c - 1) * chunk, y = p.qb - x;
+  if (p.qb - p.qa <= x) return 0;
+  const int n = (4 * y + 6) / 7;  // floor(7 wg / 4) < y
+  return n < p.kv_groups ? n : p.kv_groups;
+}
+__host__ __device__ inline ItemPos dkdv_find_item(int item, const BwdPass& p, int chunk) {
+  return find_item(item, dkdv_group_chunks(0, p, chunk),
+                   [&](int c) { return dkdv_groups_with(c, p, chunk); });
+}
+__host__ __device__ inline int dkdv_items_before(int wg, const BwdPass& p, int chunk) {
+  return items_before(wg, dkdv_group_chunks(0, p, chunk),
+                      [&](int c) { return dkdv_groups_with(c, p, chunk); });
 }
 struct DkdvSplit {
   int chunk;         // query tiles per chunk (upper bound)
