@@ -134,12 +134,10 @@ __global__ __launch_bounds__(256) void ca_bwd_prep_kernel(View Qv, View Kv,
     for (int u = 0; u < 8; ++u) e[u] = v[u >> 2][u & 3] * scale;
     const Limbs lb = split8(e);
     *reinterpret_cast<bf16x8*>(tile + (p0 + 0) * 32 * D) = lb.h;
-    if (nl > 1) {
-      *reinterpret_cast<bf16x8*>(tile + (p0 + 1) * 32 * D) = lb.m;
-      *reinterpret_cast<bf16x8*>(tile + (p0 + 2) * 32 * D) = lb.l;
-    }
+    if (nl > 1) *reinterpret_cast<bf16x8*>(tile + (p0 + 1) * 32 * D) = lb.m;
+    if (nl > 2) *reinterpret_cast<bf16x8*>(tile + (p0 + 2) * 32 * D) = lb.l;
   };
-  put(0, QL, qq, 1.0f);  // bf16 operands: Q is bf16-valued, its h limb is exact
+  put(0, QL, qq, 1.0f);  // 16-bit operands: exact in their first limbs
   put(QL, 3, dy, invz);
   if (c == 0) {
     // as the dK/dV kernel's score shift and dP' accumulator start take them
@@ -445,7 +443,7 @@ __global__ __launch_bounds__(256, (std::is_same<E, __bf16>::value && D <= 64 ? 4
         }
 #pragma unroll
         for (int st = 0; st < 6; ++st) {
-          if (limb_step_used<false, BF>(st)) {
+          if (limb_step_used<3, BF ? 1 : 3>(st)) {
             acc[0][nb] = mfma16_step(st, al0, bl, acc[0][nb]);
             acc[1][nb] = mfma16_step(st, al1, bl, acc[1][nb]);
           }

@@ -66,12 +66,13 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
     float* __restrict__ dsbuf, float* __restrict__ kv_part, float* __restrict__ gain_part,
     BwdPass pass, int BH, int H, int T, int chunk, int n_items, int n_part, bool kv_f32,
     int hd) {
-  // bf16 operands: Q, K (rotated and rounded as the reference rounds them)
-  // and V are bf16-valued, so the tile carries Q's h limb alone and the
-  // products with Q or V skip their zero limb products (limb_step_used), with
-  // the same sums bit for bit.
-  constexpr bool BF = q_limb_planes<E>() == 1;
-  using P = Bwd<D, q_limb_planes<E>()>;
+  // 16-bit operands: Q, K (rotated and rounded as the reference rounds them)
+  // and V split into fewer limbs (value_limbs), so the tile carries Q's
+  // nonzero planes alone and the products with Q, K or V skip their zero limb
+  // products (limb_step_used), with the same sums bit for bit.
+  constexpr int QL = q_limb_planes<E>();
+  constexpr bool BF = QL == 1;
+  using P = Bwd<D, QL>;
   constexpr int NBUF = SB ? 1 : 2;
   __shared__ __attribute__((aligned(16))) __bf16 tiles[NBUF][P::TILE];
   // per staged row: -(m + kShareShift) (tstat[b][0][row]) and Dl/Z
@@ -264,14 +265,8 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
           qa[rb] = ya[rb] = Limbs{bf16x8{}, bf16x8{}, bf16x8{}};
           if (col < D) {
             const int o = (16 * rb + j) * P::LDR + col;
-            qa[rb].h = *reinterpret_cast<const bf16x8*>(Tq + o);
-            if (!BF) {
-              qa[rb].m = *reinterpret_cast<const bf16x8*>(Tq + P::LIMB + o);
-              qa[rb].l = *reinterpret_cast<const bf16x8*>(Tq + 2 * P::LIMB + o);
-            }
-            ya[rb].h = *reinterpret_cast<const bf16x8*>(Ty + o);
-            ya[rb].m = *reinterpret_cast<const bf16x8*>(Ty + P::LIMB + o);
-            ya[rb].l = *reinterpret_cast<const bf16x8*>(Ty + 2 * P::LIMB + o);
+            qa[rb] = limbs_at<QL>(Tq + o, P::LIMB);
+            ya[rb] = limbs_at<3>(Ty + o, P::LIMB);
           }
         }
         // four independent accumulators per limb product
@@ -283,10 +278,10 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
           }
           const Limbs& vb = P::KB == 1 && st < 3 ? vneg : vl[kb];
           const int ss = limb_step_swapped(st);  // the forward's order, K its first operand
-          if (limb_step_used<BF, BF>(ss)) sacc[0] = mfma16_step(ss, qa[0], kl[kb], sacc[0]);
-          if (limb_step_used<false, BF>(st)) pacc[0] = mfma16_step(st, ya[0], vb, pacc[0]);
-          if (limb_step_used<BF, BF>(ss)) sacc[1] = mfma16_step(ss, qa[1], kl[kb], sacc[1]);
-          if (limb_step_used<false, BF>(st)) pacc[1] = mfma16_step(st, ya[1], vb, pacc[1]);
+          if (limb_step_used<QL, QL>(ss)) sacc[0] = mfma16_step(ss, qa[0], kl[kb], sacc[0]);
+          if (limb_step_used<3, QL>(st)) pacc[0] = mfma16_step(st, ya[0], vb, pacc[0]);
+          if (limb_step_used<QL, QL>(ss)) sacc[1] = mfma16_step(ss, qa[1], kl[kb], sacc[1]);
+          if (limb_step_used<3, QL>(st)) pacc[1] = mfma16_step(st, ya[1], vb, pacc[1]);
         }
       }
       prio_mfma_end<!BF>();
@@ -389,16 +384,13 @@ __global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd
         ya.m = lds_read_tr8(Ty + P::LIMB + o0, Ty + P::LIMB + o1);
         ya.l = lds_read_tr8(Ty + 2 * P::LIMB + o0, Ty + 2 * P::LIMB + o1);
         qa.h = lds_read_tr8(Tq + o0, Tq + o1);
-        if (BF) {
-          qa.m = qa.l = bf16x8{};
-        } else {
-          qa.m = lds_read_tr8(Tq + P::LIMB + o0, Tq + P::LIMB + o1);
-          qa.l = lds_read_tr8(Tq + 2 * P::LIMB + o0, Tq + 2 * P::LIMB + o1);
-        }
+        qa.m = qa.l = bf16x8{};
+        if (QL > 1) qa.m = lds_read_tr8(Tq + P::LIMB + o0, Tq + P::LIMB + o1);
+        if (QL > 2) qa.l = lds_read_tr8(Tq + 2 * P::LIMB + o0, Tq + 2 * P::LIMB + o1);
 #pragma unroll
         for (int st = 0; st < 6; ++st) {
           accv[mb] = mfma16_step(st, ya, wb, accv[mb]);
-          if (limb_step_used<BF, false>(st)) acck[mb] = mfma16_step(st, qa, db, acck[mb]);
+          if (limb_step_used<QL, 3>(st)) acck[mb] = mfma16_step(st, qa, db, acck[mb]);
         }
       }
       prio_mfma_end<!BF>();

@@ -35,6 +35,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace ca {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -73,15 +75,6 @@ struct Limbs {  // one 8-element MFMA operand in three limbs (4 VGPRs each)
 __device__ __forceinline__ f32x16 mfma_bf16(bf16x8 a, bf16x8 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
-// c += a * b over 16 k values, to fp32 accuracy
-__device__ __forceinline__ f32x16 mfma_x6(const Limbs& a, const Limbs& b, f32x16 c) {
-  c = mfma_bf16(a.l, b.h, c);
-  c = mfma_bf16(a.m, b.m, c);
-  c = mfma_bf16(a.h, b.l, c);
-  c = mfma_bf16(a.m, b.h, c);
-  c = mfma_bf16(a.h, b.m, c);
-  return mfma_bf16(a.h, b.h, c);
-}
 
 // 16x16x32 tile (v_mfma_f32_16x16x32_bf16): A lane l supplies row l%16,
 // k = 8*(l/16) + e; B lane l supplies column l%16, same k; the result lane l
@@ -89,16 +82,8 @@ __device__ __forceinline__ f32x16 mfma_x6(const Limbs& a, const Limbs& b, f32x16
 __device__ __forceinline__ f32x4 mfma16_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ f32x4 mfma16_x6(const Limbs& a, const Limbs& b, f32x4 c) {
-  c = mfma16_bf16(a.l, b.h, c);
-  c = mfma16_bf16(a.m, b.m, c);
-  c = mfma16_bf16(a.h, b.l, c);
-  c = mfma16_bf16(a.m, b.h, c);
-  c = mfma16_bf16(a.h, b.m, c);
-  return mfma16_bf16(a.h, b.h, c);
-}
 
-// One of the six limb products of mfma16_x6 (step 0..5, small terms first);
+// One of the six limb products of a 16x16x32 tile (step 0..5, small terms first);
 // issuing step k on several independent accumulators before step k+1 keeps
 // dependent MFMAs apart.
 __device__ __forceinline__ f32x4 mfma16_step(int step, const Limbs& a, const Limbs& b, f32x4 c) {
@@ -112,31 +97,49 @@ __device__ __forceinline__ f32x4 mfma16_step(int step, const Limbs& a, const Lim
   }
 }
 
-// bf16-valued operands: an fp32 value that is exactly a bf16 number splits
-// into h = the value and m = l = 0, so the limb products that use its m or l
+// 16-bit-valued operands: an fp32 value that is exactly a bf16 number splits
+// into h = the value and m = l = 0, and one that is exactly an fp16 number (11
+// significant bits) into h and m with l = 0.  Limb products that use a zero
 // limb are exactly zero and are skipped (an MFMA adding zero products leaves
 // the accumulator unchanged, so the result is the same bit for bit).
-// limb_step_used<ABF, BBF>(st): step st of mfma16_step (a.l b.h, a.m b.m,
-// a.h b.l, a.m b.h, a.h b.m, a.h b.h) is nonzero when operand a (ABF) / b
-// (BBF) is bf16-valued.
-template <bool ABF, bool BBF>
+// value_limbs<E>(): nonzero limbs of a value of type E.
+// limb_step_used<NA, NB>(st): step st of mfma16_step (a.l b.h, a.m b.m,
+// a.h b.l, a.m b.h, a.h b.m, a.h b.h) is nonzero for operands a and b of NA and
+// NB limbs: 1, 4 or 6 steps for two operands of 1, 2 or 3 limbs.
+template <class E> __host__ __device__ constexpr int value_limbs() {
+  return std::is_same<E, __bf16>::value ? 1 : std::is_same<E, _Float16>::value ? 2 : 3;
+}
+template <int NA, int NB>
 __host__ __device__ constexpr bool limb_step_used(int st) {
-  const bool a_low = st == 0 || st == 1 || st == 3;  // uses a.m or a.l
-  const bool b_low = st == 1 || st == 2 || st == 4;  // uses b.m or b.l
-  return !(ABF && a_low) && !(BBF && b_low);
+  const int a = st == 0 ? 2 : st == 1 || st == 3 ? 1 : 0;  // limb of a the step takes
+  const int b = st == 2 ? 2 : st == 1 || st == 4 ? 1 : 0;  // limb of b
+  return a < NA && b < NB;
+}
+// c += a * b over 16 k values (32x32x16 tiles), operands of NA and NB limbs, to
+// fp32 accuracy: the steps of mfma16_step in their order
+template <int NA, int NB>
+__device__ __forceinline__ f32x16 mfma32_limbs(const Limbs& a, const Limbs& b, f32x16 c) {
+  if (limb_step_used<NA, NB>(0)) c = mfma_bf16(a.l, b.h, c);
+  if (limb_step_used<NA, NB>(1)) c = mfma_bf16(a.m, b.m, c);
+  if (limb_step_used<NA, NB>(2)) c = mfma_bf16(a.h, b.l, c);
+  if (limb_step_used<NA, NB>(3)) c = mfma_bf16(a.m, b.h, c);
+  if (limb_step_used<NA, NB>(4)) c = mfma_bf16(a.h, b.m, c);
+  return mfma_bf16(a.h, b.h, c);
+}
+// Operand of NL limbs from its planes (`stride` bf16 apart) at p.
+template <int NL>
+__device__ __forceinline__ Limbs limbs_at(const __bf16* p, int stride) {
+  Limbs r;
+  r.h = *reinterpret_cast<const bf16x8*>(p);
+  r.m = r.l = bf16x8{};
+  if (NL > 1) r.m = *reinterpret_cast<const bf16x8*>(p + stride);
+  if (NL > 2) r.l = *reinterpret_cast<const bf16x8*>(p + 2 * stride);
+  return r;
 }
 // The step that multiplies the same limbs with the operands exchanged.
 __host__ __device__ constexpr int limb_step_swapped(int st) {
   return st == 0 ? 2 : st == 2 ? 0 : st == 3 ? 4 : st == 4 ? 3 : st;
 }
-// c += a * b over 16 k values (32x32x16 tiles) with bf16-valued a: the three
-// products of a.h, small terms first (the nonzero steps of mfma_x6)
-__device__ __forceinline__ f32x16 mfma_x3_abf(bf16x8 ah, const Limbs& b, f32x16 c) {
-  c = mfma_bf16(ah, b.l, c);
-  c = mfma_bf16(ah, b.m, c);
-  return mfma_bf16(ah, b.h, c);
-}
-
 // Transposed LDS read (ds_read_b64_tr_b16): within each 16-lane group, lane
 // i receives element (i & 3) of the 4 bf16 that lanes 4j + (i >> 2) address,
 // for j = 0..3.  With lane i' = 4j + m pointing at row r0 + j, column c0 + 4m
@@ -175,6 +178,19 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned& h, unsign
   m = cvt_pk_bf16(ra, rb);
   const float sa = ra - __uint_as_float(m << 16), sb = rb - __uint_as_float(m & 0xffff0000u);
   l = cvt_pk_bf16(sa, sb);
+}
+// limbs of a pair of values of NL limbs (unused ones not written)
+template <int NL>
+__device__ __forceinline__ void split_pair_limbs(float a, float b, unsigned (&w)[3]) {
+  w[0] = cvt_pk_bf16(a, b);
+  if (NL > 1) {
+    const float ra = a - __uint_as_float(w[0] << 16), rb = b - __uint_as_float(w[0] & 0xffff0000u);
+    w[1] = cvt_pk_bf16(ra, rb);
+    if (NL > 2) {
+      const float sa = ra - __uint_as_float(w[1] << 16), sb = rb - __uint_as_float(w[1] & 0xffff0000u);
+      w[2] = cvt_pk_bf16(sa, sb);
+    }
+  }
 }
 // limbs of 8 floats (one MFMA operand)
 __device__ __forceinline__ Limbs split8(const float* x) {

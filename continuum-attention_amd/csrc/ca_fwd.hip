@@ -15,7 +15,7 @@
 // (log-sum-exp style; deterministic order).
 //
 // Both products run as bf16x6 (six limb products per fp32 product, fp32
-// accumulation; mfma_x6) on v_mfma_f32_32x32x16_bf16.  Per wave, the S^T =
+// accumulation; mfma32_limbs) on v_mfma_f32_32x32x16_bf16.  Per wave, the S^T =
 // K Q^T tile (32 keys x 32 queries) has keys permuted so that lane (q, h)
 // holds 16 consecutive keys of query q; the K tile is stored in that row
 // order.  Segment neighbours are then in the same lane; only the segment
@@ -100,12 +100,12 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
     float* __restrict__ O, View Ov, float* __restrict__ stats, float* __restrict__ part, int BH,
     int H, int T, int C, int G, int smax, int hd) {
   using P = Fwd<D>;
-  // bf16 operands (with RoPE rounded to bf16 as the reference does) are
-  // bf16-valued: their limb split is h = the value, m = l = 0, so a K or V
-  // tile is staged as its h plane alone and every product with it takes the
-  // three nonzero limb products (mfma_x3_abf), bit for bit the same sums.
+  // 16-bit operands (with RoPE rounded to their type as the reference does)
+  // split into fewer limbs (value_limbs): a K or V tile is staged as those
+  // planes alone and its products take the nonzero steps, bit for bit the
+  // same sums.
   constexpr bool BF = std::is_same<E, __bf16>::value;
-  constexpr int NL = BF ? 1 : 3;  // limb planes staged per K and V tile
+  constexpr int NL = value_limbs<E>();  // limb planes staged per K and V tile
   // [buffer][limb][plane]
   __shared__ __attribute__((aligned(16))) __bf16 lds_k[2][NL][P::KPLANE];
   __shared__ __attribute__((aligned(16))) __bf16 lds_vt[2][NL][P::VPLANE];
@@ -281,12 +281,12 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
             *reinterpret_cast<u32x2*>(&lds_k[buf][0][off]) =
                 u32x2{cvt_pk_bf16(kv[0], kv[1]), cvt_pk_bf16(kv[2], kv[3])};
           } else {
-            unsigned h0, m0, l0, h1, m1, l1;
-            split_pair(kv[0], kv[1], h0, m0, l0);
-            split_pair(kv[2], kv[3], h1, m1, l1);
-            *reinterpret_cast<u32x2*>(&lds_k[buf][0][off]) = u32x2{h0, h1};
-            *reinterpret_cast<u32x2*>(&lds_k[buf][1][off]) = u32x2{m0, m1};
-            *reinterpret_cast<u32x2*>(&lds_k[buf][2][off]) = u32x2{l0, l1};
+            unsigned w0[3], w1[3];
+            split_pair_limbs<NL>(kv[0], kv[1], w0);
+            split_pair_limbs<NL>(kv[2], kv[3], w1);
+#pragma unroll
+            for (int l = 0; l < NL; ++l)
+              *reinterpret_cast<u32x2*>(&lds_k[buf][l][off]) = u32x2{w0[l], w1[l]};
           }
         }
       }
@@ -309,12 +309,11 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
           const f32x4 va = raw_to_f32(pre_v[j][0], Vs), vb = raw_to_f32(pre_v[j][1], Vs);
 #pragma unroll
           for (int x = 0; x < 4; ++x) {
-            unsigned hv, mv, lv;
-            split_pair(va[x], vb[x], hv, mv, lv);
+            unsigned wv[3];
+            split_pair_limbs<NL>(va[x], vb[x], wv);
             const int off = (4 * c + x) * P::VROW + 2 * pp;
-            *reinterpret_cast<unsigned*>(&lds_vt[buf][0][off]) = hv;
-            *reinterpret_cast<unsigned*>(&lds_vt[buf][1][off]) = mv;
-            *reinterpret_cast<unsigned*>(&lds_vt[buf][2][off]) = lv;
+#pragma unroll
+            for (int l = 0; l < NL; ++l) *reinterpret_cast<unsigned*>(&lds_vt[buf][l][off]) = wv[l];
           }
         }
       }
@@ -346,16 +345,7 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
         const __bf16* krow = &lds_k[buf][0][q * P::KROW + h * 8 * P::KB];
 #pragma unroll
         for (int kb = 0; kb < P::KB; ++kb) {
-          if constexpr (BF) {
-            // both operands bf16-valued: the h limbs carry the whole product
-            sacc = mfma_bf16(*reinterpret_cast<const bf16x8*>(krow + 8 * kb), qb[kb].h, sacc);
-          } else {
-            Limbs ka;
-            ka.h = *reinterpret_cast<const bf16x8*>(krow + 8 * kb);
-            ka.m = *reinterpret_cast<const bf16x8*>(krow + P::KPLANE + 8 * kb);
-            ka.l = *reinterpret_cast<const bf16x8*>(krow + 2 * P::KPLANE + 8 * kb);
-            sacc = mfma_x6(ka, qb[kb], sacc);
-          }
+          sacc = mfma32_limbs<NL, NL>(limbs_at<NL>(krow + 8 * kb, P::KPLANE), qb[kb], sacc);
         }
       }
       prio_mfma_end<!BF>();
@@ -442,17 +432,9 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
 #pragma unroll
         for (int mb = 0; mb < P::NMB; ++mb) {
           const __bf16* vrow = &lds_vt[buf][0][(dok ? 32 * mb + q : 0) * P::VROW + 16 * h + 8 * kb];
-          if constexpr (BF) {
-            const bf16x8 vh = dok ? *reinterpret_cast<const bf16x8*>(vrow) : bf16x8{};
-            acc_o[mb] = mfma_x3_abf(vh, wb, acc_o[mb]);
-          } else {
-            Limbs va;
-            va.h = *reinterpret_cast<const bf16x8*>(vrow);
-            va.m = *reinterpret_cast<const bf16x8*>(vrow + P::VPLANE);
-            va.l = *reinterpret_cast<const bf16x8*>(vrow + 2 * P::VPLANE);
-            if (!dok) va = Limbs{bf16x8{}, bf16x8{}, bf16x8{}};
-            acc_o[mb] = mfma_x6(va, wb, acc_o[mb]);
-          }
+          Limbs va = limbs_at<NL>(vrow, P::VPLANE);
+          if (!dok) va = Limbs{bf16x8{}, bf16x8{}, bf16x8{}};
+          acc_o[mb] = mfma32_limbs<NL, 3>(va, wb, acc_o[mb]);
         }
       }
       prio_mfma_end<!BF>();
@@ -608,7 +590,7 @@ __global__ __launch_bounds__(512, (fwd16_waves_per_simd<D, E, ROPE>())) void ca_
     int H, int T, int C, int G, int smax, int hd) {
   using P = Fwd16<D>;
   constexpr bool BF = std::is_same<E, __bf16>::value;
-  constexpr int NL = BF ? 1 : 3;  // limb planes staged per K and V tile
+  constexpr int NL = value_limbs<E>();  // limb planes staged per K and V tile
   __shared__ __attribute__((aligned(16))) __bf16 lds_k[2][NL][P::KPLANE];
   __shared__ __attribute__((aligned(16))) __bf16 lds_vt[2][NL][P::VPLANE];
 
@@ -749,12 +731,12 @@ __global__ __launch_bounds__(512, (fwd16_waves_per_simd<D, E, ROPE>())) void ca_
             *reinterpret_cast<u32x2*>(&lds_k[buf][0][off]) =
                 u32x2{cvt_pk_bf16(kv[0], kv[1]), cvt_pk_bf16(kv[2], kv[3])};
           } else {
-            unsigned h0, m0, l0, h1, m1, l1;
-            split_pair(kv[0], kv[1], h0, m0, l0);
-            split_pair(kv[2], kv[3], h1, m1, l1);
-            *reinterpret_cast<u32x2*>(&lds_k[buf][0][off]) = u32x2{h0, h1};
-            *reinterpret_cast<u32x2*>(&lds_k[buf][1][off]) = u32x2{m0, m1};
-            *reinterpret_cast<u32x2*>(&lds_k[buf][2][off]) = u32x2{l0, l1};
+            unsigned w0[3], w1[3];
+            split_pair_limbs<NL>(kv[0], kv[1], w0);
+            split_pair_limbs<NL>(kv[2], kv[3], w1);
+#pragma unroll
+            for (int l = 0; l < NL; ++l)
+              *reinterpret_cast<u32x2*>(&lds_k[buf][l][off]) = u32x2{w0[l], w1[l]};
           }
         }
       }
@@ -776,12 +758,11 @@ __global__ __launch_bounds__(512, (fwd16_waves_per_simd<D, E, ROPE>())) void ca_
           const f32x4 va = raw_to_f32(pre_v[j][0], Vs), vb = raw_to_f32(pre_v[j][1], Vs);
 #pragma unroll
           for (int x = 0; x < 4; ++x) {
-            unsigned hv, mv, lv;
-            split_pair(va[x], vb[x], hv, mv, lv);
+            unsigned wv[3];
+            split_pair_limbs<NL>(va[x], vb[x], wv);
             const int off = (4 * c + x) * P::VROW + 2 * pp;
-            *reinterpret_cast<unsigned*>(&lds_vt[buf][0][off]) = hv;
-            *reinterpret_cast<unsigned*>(&lds_vt[buf][1][off]) = mv;
-            *reinterpret_cast<unsigned*>(&lds_vt[buf][2][off]) = lv;
+#pragma unroll
+            for (int l = 0; l < NL; ++l) *reinterpret_cast<unsigned*>(&lds_vt[buf][l][off]) = wv[l];
           }
         }
       }
@@ -806,19 +787,10 @@ __global__ __launch_bounds__(512, (fwd16_waves_per_simd<D, E, ROPE>())) void ca_
       for (int ks = 0; ks < P::KS; ++ks) {
         const __bf16* kr0 = &lds_k[buf][0][q16 * P::KROW + 32 * ks + 8 * G4];
         const __bf16* kr1 = kr0 + 16 * P::KROW;
-        if constexpr (BF) {
-          sacc[0] = mfma16_bf16(*reinterpret_cast<const bf16x8*>(kr0), qb[ks].h, sacc[0]);
-          sacc[1] = mfma16_bf16(*reinterpret_cast<const bf16x8*>(kr1), qb[ks].h, sacc[1]);
-        } else {
-          Limbs ka0, ka1;
-          ka0.h = *reinterpret_cast<const bf16x8*>(kr0);
-          ka0.m = *reinterpret_cast<const bf16x8*>(kr0 + P::KPLANE);
-          ka0.l = *reinterpret_cast<const bf16x8*>(kr0 + 2 * P::KPLANE);
-          ka1.h = *reinterpret_cast<const bf16x8*>(kr1);
-          ka1.m = *reinterpret_cast<const bf16x8*>(kr1 + P::KPLANE);
-          ka1.l = *reinterpret_cast<const bf16x8*>(kr1 + 2 * P::KPLANE);
+        const Limbs ka0 = limbs_at<NL>(kr0, P::KPLANE), ka1 = limbs_at<NL>(kr1, P::KPLANE);
 #pragma unroll
-          for (int st = 0; st < 6; ++st) {
+        for (int st = 0; st < 6; ++st) {
+          if (limb_step_used<NL, NL>(st)) {
             sacc[0] = mfma16_step(st, ka0, qb[ks], sacc[0]);
             sacc[1] = mfma16_step(st, ka1, qb[ks], sacc[1]);
           }
@@ -900,19 +872,11 @@ __global__ __launch_bounds__(512, (fwd16_waves_per_simd<D, E, ROPE>())) void ca_
       for (int m2 = 0; m2 < P::NMB; m2 += 2) {
         Limbs va[2];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const __bf16* vr = &lds_vt[buf][0][(16 * (m2 + u) + q16) * P::VROW + 8 * G4];
-          va[u].h = *reinterpret_cast<const bf16x8*>(vr);
-          if (BF) {
-            va[u].m = va[u].l = bf16x8{};
-          } else {
-            va[u].m = *reinterpret_cast<const bf16x8*>(vr + P::VPLANE);
-            va[u].l = *reinterpret_cast<const bf16x8*>(vr + 2 * P::VPLANE);
-          }
-        }
+        for (int u = 0; u < 2; ++u)
+          va[u] = limbs_at<NL>(&lds_vt[buf][0][(16 * (m2 + u) + q16) * P::VROW + 8 * G4], P::VPLANE);
 #pragma unroll
         for (int st = 0; st < 6; ++st) {
-          if (limb_step_used<BF, false>(st)) {
+          if (limb_step_used<NL, 3>(st)) {
             acc_o[m2] = mfma16_step(st, va[0], wb, acc_o[m2]);
             acc_o[m2 + 1] = mfma16_step(st, va[1], wb, acc_o[m2 + 1]);
           }

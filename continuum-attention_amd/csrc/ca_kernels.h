@@ -506,13 +506,10 @@ hipError_t launch_bwd_dkdv(const BwdIO& io, const BwdWork& ws, const BwdPass& pa
 // major, rows past T zero) so that the dK/dV kernel stages a tile as one
 // contiguous block with no bounds tests.
 __host__ __device__ inline int bwd_pass_tiles(const BwdPass& p) { return p.qb - p.qa; }
-// Limb planes per staged query tile: the Q limbs, then the three dY/Z limbs.
-// bf16 operands have a bf16-valued Q (RoPE included, rounded as the
-// reference rounds it), whose m and l limbs are zero: its tiles carry the h
-// plane alone.  Workspaces are sized for six planes.
-template <class E> __host__ __device__ constexpr int q_limb_planes() {
-  return std::is_same<E, __bf16>::value ? 1 : 3;
-}
+// Limb planes per staged query tile: the Q limbs (RoPE included, rounded as
+// the reference rounds it; value_limbs of them), then the three dY/Z limbs.
+// Workspaces are sized for six planes.
+template <class E> __host__ __device__ constexpr int q_limb_planes() { return value_limbs<E>(); }
 // Keys of a slice, evenly spread, whose mean serves as its typical key in the
 // gain gradient.
 constexpr int kGainRefs = 4;
