@@ -53,14 +53,14 @@ using ca::check_shape;
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-// The dQ and dK/dV passes split their work items when their grids would not
-// fill the device (ca::dq_split, ca::dkdv_split).  The workspace is sized as
-// if kDqSplitBound work groups were resident, so its size does not depend on
-// the device; the device's own resident counts (at most this bound) pick the
-// splits.
+// The dQ and dK/dV passes split their work items (dq_split_for,
+// dkdv_split_for).  The workspace is sized as if kDqSplitBound work groups were
+// resident (ca::dq_split, ca::dkdv_split), so its size does not depend on the
+// device; a launch takes no split whose partials would not fit it.
 constexpr int kDqSplitBound = 2048;
 
-int dkdv_resident_groups() {
+// Compute units of the current device.
+int device_cus() {
   static std::atomic<int> cache[64];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return 0;
@@ -70,38 +70,93 @@ int dkdv_resident_groups() {
   }
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-  const int r = std::min(cus * ca::kDkdvGroupsPerCu, kDqSplitBound);
-  if (dev >= 0 && dev < 64) cache[dev].store(r, std::memory_order_relaxed);
-  return r;
+  if (dev >= 0 && dev < 64) cache[dev].store(cus, std::memory_order_relaxed);
+  return cus;
 }
 
-// forward work groups resident on the current device (2 per CU, 1 for D > 64)
-int fwd_resident_groups(int D) {
-  static std::atomic<int> cache[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 0;
-  int cus = 0;
-  if (dev >= 0 && dev < 64) cus = cache[dev].load(std::memory_order_relaxed);
-  if (!cus) {
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    if (dev >= 0 && dev < 64) cache[dev].store(cus, std::memory_order_relaxed);
-  }
-  return std::min(cus * (D > 64 ? 1 : 2), kFwdSplitBound);
+// Split lengths.  A grid's groups (of very different lengths: causal rows) are
+// cut into chunks so that the device's work-group slots finish together; each
+// chunk of a cut group writes a partial result that another launch, or
+// another launch's tail, reads back.  The length is picked by estimated time:
+// the items are dealt out in dispatch order, each to the slot that is free
+// first, and
+//   time = step_us (ideal + kTail (last slot's end - ideal)) + partials + launch
+// with ideal the slots' mean load.  kTail < 1: near the end fewer work groups
+// share a CU and each runs faster.  Against sweeps of every length on the
+// device the estimate picks the measured best or a length within 2% of it.
+// Before (thresholds on the number of items) / now, time per fwd+bwd:
+//   [1,16,2048,64] bf16 layer 239 / 228 us
+//   [4,16,1001,64] bf16 228 / 214 us   [2,16,2048,64] bf16 407 / 395 us
+//   [8,16,2048,64] bf16 1605 / 1500 us [1,16,8192,64] fp32 3730 / 3635 us
+//   [1,8,1537,128] fp32 209 / 180 us   [2,8,768,80] fp32 164 / 144 us
+//   [2,16,2048,64] fp32 510-516 / 512-517 us, [4,16,512,64] fp32 116 / 118 us
+// The forward's length must not depend on the operand type: the types'
+// outputs are compared bit for bit.
+struct SplitModel {
+  int resident;      // work groups the device holds at once
+  int overhead;      // an item's prologue and epilogue, in steps
+  double step_us;    // one step of one item with the device full
+  double part_us;    // device time per partial item, written and read back
+  double launch_us;  // extra launch when anything is split
+};
+constexpr double kTail = 0.6;
+// From this many rounds of whole groups on the tail is under 2% of the time
+// and nothing is cut; it also bounds the host's work per estimate.
+constexpr int kSplitRounds = 64;
+inline bool many_rounds(const SplitModel& m, int groups, int BH) {
+  return (long long)groups * BH >= (long long)kSplitRounds * m.resident;
 }
 
-int dq_resident_groups() {
-  static std::atomic<int> cache[64];
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 0;
-  if (dev >= 0 && dev < 64) {
-    const int c = cache[dev].load(std::memory_order_relaxed);
-    if (c) return c;
+// items(f) calls f(length) for each item of a slice in dispatch order; every
+// item is launched for all BH slices.
+template <class Items>
+double split_cost(const SplitModel& m, int BH, int part_items, Items items) {
+  std::vector<int> free_at(64, 0);  // slots that become free at each step
+  free_at[0] = m.resident;
+  size_t lo = 0;
+  int last = 0;
+  double total = 0;
+  items([&](int len) {
+    const int t = len + m.overhead;
+    total += (double)t * BH;
+    for (int need = BH; need > 0;) {
+      while (free_at[lo] == 0) ++lo;
+      const int n = std::min(need, free_at[lo]);
+      free_at[lo] -= n;
+      const size_t end = lo + t;
+      if (end >= free_at.size()) free_at.resize(2 * end, 0);
+      free_at[end] += n;
+      last = std::max(last, (int)end);
+      need -= n;
+    }
+  });
+  const double ideal = total / m.resident;
+  return m.step_us * (ideal + kTail * std::max(0.0, last - ideal)) +
+         (part_items ? m.part_us * part_items * BH + m.launch_us : 0.0);
+}
+
+// The estimates are functions of a few numbers; a thread keeps its last ones.
+struct SplitKey {
+  int kind, BH, T, D, a, b, resident, limit;
+  bool operator==(const SplitKey& o) const {
+    return kind == o.kind && BH == o.BH && T == o.T && D == o.D && a == o.a && b == o.b &&
+           resident == o.resident && limit == o.limit;
   }
-  int cus = 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-  const int r = std::min(cus * ca::kDqGroupsPerCu, kDqSplitBound);
-  if (dev >= 0 && dev < 64) cache[dev].store(r, std::memory_order_relaxed);
-  return r;
+};
+template <class Pick>
+int cached_split(const SplitKey& key, Pick pick) {
+  struct Entry {
+    SplitKey key;
+    int value;
+  };
+  static thread_local Entry cache[64] = {};
+  static thread_local int next = 0;
+  for (const Entry& e : cache)
+    if (e.value && e.key == key) return e.value;
+  const int v = pick();
+  cache[next] = Entry{key, v};
+  next = (next + 1) % 64;
+  return v;
 }
 
 // Forced split lengths (ca_debug_set_splits; 0 = automatic).  When one is
@@ -121,64 +176,107 @@ size_t g_workspace_cap = size_t(1) << 30;
 // partials fit; a split as long as the longest row needs no partials.
 int fwd_split(int BH, int T, int D, bool for_sizing, size_t bytes = SIZE_MAX) {
   if (g_split.fwd_tiles > 0) return g_split.fwd_tiles;
-  const int C = ca::fwd_split_tiles(BH, T, for_sizing ? kFwdSplitBound : fwd_resident_groups(D));
-  if (ca::fwd_part_floats(BH, T, C, D) * sizeof(float) <= bytes) return C;
   const int G = (T + 127) / 128;
   const int max_tiles = ca::fwd_group_tiles(G - 1, T);
-  const size_t per_split = (size_t)BH * T * (D + 2) * sizeof(float);
-  const size_t fit = bytes / per_split;  // splits the partials can hold
-  if (fit < 2) return max_tiles;
-  const int cf = (int)((max_tiles + fit - 1) / fit);
-  return cf > C ? cf : C;
+  int C = ca::fwd_split_tiles(BH, T, kFwdSplitBound);
+  if (ca::fwd_part_floats(BH, T, C, D) * sizeof(float) > bytes) {
+    const size_t per_split = (size_t)BH * T * (D + 2) * sizeof(float);
+    const size_t fit = bytes / per_split;  // splits the partials can hold
+    C = fit < 2 ? max_tiles : std::max(C, (int)((max_tiles + fit - 1) / fit));
+  }
+  if (for_sizing || C >= max_tiles) return C;
+  const int cus = device_cus();
+  if (!cus) return C;
+  // D <= 64: two work groups per CU
+  const SplitModel m{D > 64 ? cus : 2 * cus, 1, D > 64 ? 4.1 : 2.0 + 2.3 * D / 64, 0.017 * D / 64, 4.0};
+  if (many_rounds(m, G, BH)) return max_tiles;
+  return cached_split(SplitKey{0, BH, T, D, 0, 0, m.resident, C}, [&] {
+    int best = max_tiles;
+    double cost = 1e30;
+    for (int c : {max_tiles, 48, 32, 24, 20, 16, 12, 8, 6, 4, C}) {
+      if (c < C || c > max_tiles) continue;
+      int parts = 0;
+      const double t0 = split_cost(m, BH, 0, [&](auto f) {
+        for (int g = G - 1; g >= 0; --g) {
+          const int nt = ca::fwd_group_tiles(g, T);
+          if (nt > c) parts += (nt + c - 1) / c;
+          for (int t = 0; t < nt; t += c) f(std::min(c, nt - t));
+        }
+      });
+      const double t = t0 + (parts ? m.part_us * parts * BH + m.launch_us : 0.0);
+      if (t < cost) {
+        cost = t;
+        best = c;
+      }
+    }
+    return best;
+  });
 }
 ca::DqSplit dq_split_for(int BH, int T, int D, const ca::BwdPass& p, bool for_sizing) {
   if (g_split.dq_stages > 0) return ca::dq_split_chunk(T, p, g_split.dq_stages);
-  // D = 128 kernels hold fewer dQ work groups per CU (two instead of three)
-  const int res = for_sizing ? kDqSplitBound : (D > 64 ? dq_resident_groups() * 2 / 3 : dq_resident_groups());
-  return ca::dq_split(BH, T, p, res);
+  const ca::DqSplit sized = ca::dq_split(BH, T, p, kDqSplitBound);
+  const int cus = for_sizing ? 0 : device_cus();
+  if (!cus) return sized;
+  const int whole = ca::num_q_tiles(T);
+  // three work groups per CU, two at D = 128
+  const SplitModel m{D > 64 ? 2 * cus : 3 * cus, 1, 3.2 * std::max(D, 32) / 64, 0.016 * D / 64, 4.5};
+  if (many_rounds(m, p.g1 - p.g0, BH)) return ca::dq_split_chunk(T, p, whole);
+  const int chunk = cached_split(SplitKey{1, BH, T, D, p.g0, p.g1, m.resident, sized.part_items}, [&] {
+    int best = whole;
+    double cost = 1e30;
+    for (int c : {whole, 64, 48, 40, 28, 21, 14, 10, 7}) {
+      if (c > whole) continue;
+      const ca::DqSplit s = ca::dq_split_chunk(T, p, c);
+      if (s.part_items > sized.part_items) continue;
+      const double t = split_cost(m, BH, s.part_items, [&](auto f) {
+        for (int g = p.g0; g < p.g1; ++g) {  // dispatched lightest first
+          const int n = ca::dq_group_stages(g, T), nch = (n + c - 1) / c, len = (n + nch - 1) / nch;
+          for (int t = (nch - 1) * len; t >= 0; t -= len) f(std::max(0, std::min(len, n - t)));
+        }
+      });
+      if (t < cost) {
+        cost = t;
+        best = c;
+      }
+    }
+    return best;
+  });
+  return ca::dq_split_chunk(T, p, chunk);
 }
 ca::DkdvSplit dkdv_split_for(int BH, int D, int dtype, const ca::BwdPass& p, bool for_sizing) {
   if (g_split.dkdv_tiles > 0) return ca::dkdv_split_chunk(p, g_split.dkdv_tiles);
-  // D = 128: two dK/dV work groups per CU; split below two rounds of them.
-  // bf16 operands at D <= 64: three per CU, and the split test asks for 1.5
-  // rounds of them (9/4 of the two-per-CU count; at [1,16,2048,64] chunks of
-  // 16 tiles took 0.277 ms per fwd+bwd against 0.283 ms for 24 and 0.281 ms
-  // for 12).
-  // fp32 and fp16 operands at D = 64 (the single-buffered kernel, three per CU): split
-  // only below 1.5 rounds of three per CU (config 2, 37 key groups x 32
-  // slices, stays unsplit: 24-tile chunks made dK/dV 8 us faster and the
-  // dQ launch, which merges their partials, 13 us slower), then from 16-tile
-  // chunks down until one round is filled.  Kernel time per fwd+bwd
-  // (rocprof, sum of the operator's kernels) against the earlier rule (1.5
-  // rounds, from 24 tiles): [16,4,512,64] (one CA-P layer) 125.1 -> 117.4 us
-  // (12-tile chunks instead of 6), [2,8,1024,64] 118.5 -> 111.8 us,
-  // [1,16,1024,64] 118.3 -> 112.2 us, [4,8,700,64] 119.1 -> 114.4 us,
-  // [1,32,1500,64] 368.4 -> 354.2 us (16 instead of 24), but [2,4,2048,64]
-  // 176.8 -> 183.3 us (12 instead of 8); config 2, config 5 and
-  // [1,16,2048,64] keep their lengths.  The workspace is
-  // sized for chunks from kDkdvChunkTiles down (for_sizing), so a shorter
-  // first chunk is taken only where its items and partials fit that size;
-  // elsewhere the earlier rule applies.
-  int res = kDqSplitBound;
-  long long want = -1;
-  if (!for_sizing) {
-    const int two_per_cu = dkdv_resident_groups();
-    if (D > 64) {
-      res = two_per_cu;
-    } else if (dtype == CA_DTYPE_BF16) {
-      res = std::min(two_per_cu * 9 / 4, kDqSplitBound);
-    } else if (D == 64) {
-      res = std::min(two_per_cu * 9 / 4, kDqSplitBound);
-      want = res;
-      const ca::DkdvSplit s =
-          ca::dkdv_split(BH, p, std::min(two_per_cu * 3 / 2, kDqSplitBound), want, 16);
-      const ca::DkdvSplit sized = dkdv_split_for(BH, D, dtype, p, true);
-      if (s.items <= sized.items && s.part_items <= sized.part_items) return s;
-    } else {
-      res = two_per_cu;
+  // the workspace is sized for these items and partials
+  const ca::DkdvSplit sized = ca::dkdv_split(BH, p, kDqSplitBound);
+  const int cus = for_sizing ? 0 : device_cus();
+  if (!cus) return sized;
+  const bool bf16 = dtype == CA_DTYPE_BF16;
+  const int whole = p.qb - p.qa;
+  // work groups per CU: dkdv_waves_per_simd (four waves each)
+  const SplitModel m{cus * (D > 64 ? 2 : bf16 ? 4 : 3), 2, D > 64 ? 6.9 : 1.9 + 2.9 * D / 64,
+                     0.02 * D / 64, 0.0};
+  if (many_rounds(m, p.kv_groups, BH)) return ca::dkdv_split_chunk(p, whole);
+  const int chunk = cached_split(SplitKey{2 + bf16, BH, p.kv_groups, D, p.qa, p.qb, m.resident,
+                                          sized.part_items}, [&] {
+    int best = whole;
+    double cost = 1e30;
+    for (int c : {whole, 48, 40, 32, 28, 24, 20, 16, 14, 12, 10, 8, 6}) {
+      if (c > whole) continue;
+      const ca::DkdvSplit s = ca::dkdv_split_chunk(p, c);
+      if (s.items > sized.items || s.part_items > sized.part_items) continue;
+      const double t = split_cost(m, BH, s.part_items, [&](auto f) {
+        for (int w = 0; w < p.kv_groups; ++w) {
+          const int n = ca::dkdv_group_tiles(w, p), nch = (n + c - 1) / c, len = (n + nch - 1) / nch;
+          for (int t = 0; t < nch; ++t) f(std::max(0, std::min(len, n - t * len)));
+        }
+      });
+      if (t < cost) {
+        cost = t;
+        best = c;
+      }
     }
-  }
-  return ca::dkdv_split(BH, p, res, want);
+    return best;
+  });
+  return ca::dkdv_split_chunk(p, chunk);
 }
 
 // Workspace layout of one backward pass (every pass lays its buffers out from
@@ -188,7 +286,7 @@ struct BwdLayout {
 };
 BwdLayout bwd_layout(int B, int H, int T, int D, const ca::BwdPass& p) {
   const int BH = B * H;
-  const ca::DqSplit sp = dq_split_for(BH, T, D, p, true);  // the largest split
+  const ca::DqSplit sp = dq_split_for(BH, T, D, p, true);
   const ca::DkdvSplit kvs = dkdv_split_for(BH, D, CA_DTYPE_F32, p, true);
   BwdLayout L;
   L.ds = 0;

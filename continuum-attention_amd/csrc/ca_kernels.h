@@ -69,17 +69,17 @@ inline int fwd_num_items(int T, int C) {
   for (int g = 0; g < G; ++g) n += (fwd_group_tiles(g, T) + C - 1) / C;
   return n;
 }
-// Split length: 12 tiles up to T = 2048; for short rows (at most four
-// 128-query groups) 8, 6 or 4 while the grid of BH * items would not fill
-// `resident` work groups; past T = 2048, 12 sqrt(T / 2048) tiles rounded to a
-// multiple of 4 (16, 24, 32, 48 at T = 4096 .. 32768), as the grid then
-// fills the device either way and each split adds combine traffic (same-box
-// fwd+bwd at [1,16,T,64] with 12 tiles against the longer split: T = 4096
-// 1.026 -> 1.017 ms, 8192 4.04 -> 4.00 ms, 16384 16.27 -> 15.81 ms; at T =
-// 2048 longer splits were no faster).
+// Shortest split the workspace is sized for: 12 tiles up to T = 2048; for
+// short rows (at most eight 128-query groups) 8, 6 or 4 while the grid of BH *
+// items would not fill `resident` work groups; past T = 2048, 12 sqrt(T / 2048)
+// tiles rounded to a multiple of 4 (16, 24, 32, 48 at T = 4096 .. 32768), as
+// the grid then fills the device either way and each split adds combine
+// traffic (same-box fwd+bwd at [1,16,T,64] with 12 tiles against the longer
+// split: T = 4096 1.026 -> 1.017 ms, 8192 4.04 -> 4.00 ms, 16384 16.27 ->
+// 15.81 ms).  The launch picks the length (split_cost), this one or longer.
 constexpr int kFwdSplitTiles = 12;
 constexpr int kFwdSplitSmall[] = {8, 6, 4};
-constexpr int kFwdSplitShortT = 512;
+constexpr int kFwdSplitShortT = 1024;
 constexpr int kFwdSplitLongT = 2048;
 inline int fwd_split_tiles(int BH, int T, int resident) {
   int C = kFwdSplitTiles;
@@ -203,8 +203,8 @@ __host__ __device__ inline BwdPass bwd_pass(int T, int g0, int g1) {
 // slice from the last (heaviest) group of the pass down, so the chunks of
 // multi-chunk groups come first; those items write partial dQ tiles that a
 // second kernel sums in chunk order.
-constexpr int kDqChunkStages = 28;       // split chunk length in 32-key stages (896 keys)
-constexpr int kDqChunkStagesShort = 21;  // when 28-stage chunks still leave the GPU short of a round
+constexpr int kDqChunkStages = 28;       // 32-key stages (896 keys)
+constexpr int kDqChunkStagesShort = 21;
 // key stages of group qg (those met by its last query tile)
 __host__ __device__ inline int dq_group_stages(int qg, int T) {
   const int nqt = num_q_tiles(T);
@@ -247,12 +247,10 @@ inline DqSplit dq_split_chunk(int T, const BwdPass& p, int chunk) {
   }
   return s;
 }
-// resident_groups: dQ work groups the GPU holds at once (0: never split).
-// Splitting more finely only adds work groups (and partial tiles), so the
-// workspace sized for the largest resident_groups covers every smaller one.
-// Shorter chunks while the grid would fill less than half a round (few
-// slices, short rows): more dQ work groups, at the price of more partials to
-// merge, which outweighs the gain once half a round is filled.
+// The finest split the workspace is sized for, as if the device held
+// resident_groups dQ work groups: chunks of kDqChunkStages unless the whole
+// groups fill it, shorter ones while even those leave it short of a round.
+// The launch picks its own length (split_cost) among those whose partials fit.
 constexpr int kDqChunkSmall[] = {14, 10, 7};
 inline DqSplit dq_split(int BH, int T, const BwdPass& p, int resident_groups) {
   if ((long long)(p.g1 - p.g0) * BH >= resident_groups)
@@ -266,22 +264,14 @@ inline DqSplit dq_split(int BH, int T, const BwdPass& p, int resident_groups) {
   }
   return s;
 }
-// dQ work groups per CU the split heuristic counts as resident: 3, although
-// the D = 64 kernel's 124 VGPRs allow 4 (counting 4 picks shorter chunks at
-// [2,16,2048,64], measured 4% slower)
-constexpr int kDqGroupsPerCu = 3;
 
 // dK/dV work items: key-block group wg (kDkdvWaves blocks, kDkdvKeys keys) of
-// one slice and a chunk of the pass's query tiles that see its keys.  When
-// the grid of whole groups would not fill the GPU for two rounds (small B*H),
-// a group's query range is cut into chunks of at most kDkdvChunkTiles tiles,
-// so the groups with the longest ranges do not set the launch time alone; the
-// chunks write partial dK/dV that a merge sums in chunk order.  Items are
-// numbered per slice from group 0 (the longest range) up, chunks of a group
-// together.
+// one slice and a chunk of the pass's query tiles that see its keys.  Where
+// the whole groups would leave the GPU idle at the end (few slices, unequal
+// ranges) a group's query range is cut into chunks; the chunks write partial
+// dK/dV that a merge sums in chunk order.  Items are numbered per slice from
+// group 0 (the longest range) up, chunks of a group together.
 constexpr int kDkdvKeys = kDkdvWaves * kBwdKeys;
-constexpr int kDkdvChunkTiles = 24;
-constexpr int kDkdvGroupsPerCu = 2;
 __host__ __device__ inline int dkdv_num_groups(int T) {
   return (bwd_num_key_blocks(T) + kDkdvWaves - 1) / kDkdvWaves;
 }
@@ -333,22 +323,17 @@ inline DkdvSplit dkdv_split_chunk(const BwdPass& p, int chunk) {
   }
   return s;
 }
-// Shorter chunks while the first length (kDkdvChunkTiles unless given)
-// leaves less than one round (fewer would only add partials and merge
-// work): the first length whose items fill a round is taken, else the last.
-// resident_groups: dK/dV work groups the GPU holds at once (0: never split).
-constexpr int kDkdvChunkSmall[] = {16, 12, 8, 6};
-// want_groups: split only when the whole groups number fewer (default: two
-// rounds of resident_groups).
-inline DkdvSplit dkdv_split(int BH, const BwdPass& p, int resident_groups, long long want_groups = -1,
-                            int first_chunk = kDkdvChunkTiles) {
-  const long long want = want_groups >= 0 ? want_groups : 2LL * resident_groups;
-  if ((long long)p.kv_groups * BH >= want) return dkdv_split_chunk(p, p.qb - p.qa);
-  DkdvSplit s = dkdv_split_chunk(p, first_chunk);
-  for (int c : kDkdvChunkSmall) {
-    if (c >= first_chunk) continue;
-    if ((long long)s.items * BH >= resident_groups) break;
+// The finest split the workspace is sized for, as if the device held
+// resident_groups work groups: whole groups if they fill two rounds, else the
+// longest of these lengths whose items fill one (or the shortest).  The launch
+// picks its own length (split_cost) among those whose partials fit.
+constexpr int kDkdvChunkLengths[] = {24, 16, 12, 8, 6};
+inline DkdvSplit dkdv_split(int BH, const BwdPass& p, int resident_groups) {
+  DkdvSplit s = dkdv_split_chunk(p, p.qb - p.qa);
+  if ((long long)p.kv_groups * BH >= 2LL * resident_groups) return s;
+  for (int c : kDkdvChunkLengths) {
     s = dkdv_split_chunk(p, c);
+    if ((long long)s.items * BH >= resident_groups) break;
   }
   return s;
 }
