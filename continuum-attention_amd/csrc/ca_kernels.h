@@ -474,11 +474,11 @@ hipError_t launch_rope_keys(View k, const float* rope, void* out, int BH, int H,
 // planes and qstat rows, gain partials per dQ item, dQ and dK/dV chunk
 // partials).
 struct BwdWork {
-  float* dsbuf;       // dS spill, 32x16 blocks
-  __bf16* limbs;      // per slice and query tile of the pass, six bf16 planes [32 rows][D]:
-                      // Q limbs h, m, l; dY/Z limbs h, m, l ([BH][tile][plane][32][D])
+  float* dsbuf;       // dS spill, key-major columns of 32 queries
+  __bf16* limbs;      // per slice and query tile of the pass, bf16 planes [32 rows][D]: the Q
+                      // limbs (q_limb_planes), then dY/Z limbs h, m, l ([BH][tile][plane][32][D])
   float* qstat;       // per slice and padded row of the pass's tiles: (-(m + kShareShift), D/Z)
-  float* gain_part;   // per dQ item
+  float* gain_part;   // per dK/dV item
   float* dq_part;     // dQ chunk partials
   float* kv_part;     // dK/dV chunk partials: [BH][part item][kDkdvKeys][2][D]
 };

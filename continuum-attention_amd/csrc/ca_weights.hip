@@ -12,7 +12,8 @@
 // 0 .. start + r % Q (the host checks start + Q <= K).  stats is
 // [rows][2] = (row max m, 1/Z) in natural units, as the reference's.
 //
-// One wave per row, four rows per 256-thread work group.  Lane l of step t
+// One wave per row, four rows per 256-thread work group.  Rows of 65 to 2048
+// keys run in ca_weights_reg_kernel (below), others here: lane l of step t
 // owns key j = 64 t + l and evaluates the segment (j, j+1) once: its left
 // share stays with key j and its right share moves to key j+1 with one lane
 // shift.  Scores are read coalesced; neighbours come from lane shuffles (the

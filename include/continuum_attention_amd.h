@@ -1,8 +1,9 @@
 /* C ABI of the MI355X-native Continuum Attention operator (libca_hip.so).
  *
  * Plain pointers, sizes and an opaque HIP stream handle; no torch or HIP types
- * in the signatures.  All tensors are float32, contiguous, device-resident,
- * laid out [B, H, T, D] (row-major, D fastest).  The caller allocates every
+ * in the signatures.  Tensors are float32 unless an entry point takes a dtype,
+ * contiguous, device-resident, laid out [B, H, T, D] (row-major, D fastest)
+ * unless it says otherwise.  The caller allocates every
  * output and workspace; the library allocates nothing.  Every call is
  * asynchronous on `stream` (NULL = the default stream) and returns CA_OK or an
  * error code whose text ca_last_error() returns (thread-local).
