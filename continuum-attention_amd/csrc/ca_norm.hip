@@ -14,6 +14,8 @@
 #include <hip/hip_fp16.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "ca_common.h"
 #include "ca_kernels.h"
 
@@ -88,11 +90,23 @@ __device__ __forceinline__ void store_vec(void* base, size_t i, int dtype, const
 
 // One wave per row, four rows per work group; lane l holds columns
 // VEC*(l + 64*u).  KMAX > 0: the row is read once into registers (u < KMAX,
-// C <= 64*VEC*KMAX) with every load issued before the first use; KMAX = 0:
+// C <= 64*VEC*KMAX), kChunks loads of each operand at a time; KMAX = 0:
 // any C, loops that read the row twice.  ADD: the normalised row is
 // s = x + res (res in rdtype), and s is written to sum_out (fp32).  No
 // work-group barrier: a wave past the last row exits.
-template <int VEC, int KMAX, bool ADD>
+// RT and YT are rdtype and ydtype where they are known at compile time
+// (kRuntimeDtype: not).  Memory-bound, and with the types tested at run time
+// bound by latency: each chunk's branch on the type ended in a wait, so a
+// wave had one chunk of its row in flight at a time.  Now kChunks of them are
+// (all up to C = 1024); sixteen at once took 163 instead of 118 registers and
+// with them waves ([4096, 4096] 46 against 39 us; two at once no faster).
+// Residual add in bf16, before / now, us: [512, 1024] 5.3 / 4.1, [2048, 1024]
+// 7.8 / 6.5, [8192, 1024] 16.6 / 16.6 (100 MB, 6 TB/s: resident in the last-
+// level cache), [16384, 256] 10.8 / 11.0, [2048, 2048] 12.5 / 11.5, [64, 4096]
+// 11.7 / 8.8, [4096, 4096] 38 / 39.
+constexpr int kRuntimeDtype = -1;
+constexpr int kChunks = 4;
+template <int VEC, int KMAX, bool ADD, int RT, int YT>
 __global__ __launch_bounds__(256) void ca_rmsnorm_fwd_kernel(
     const float* __restrict__ x, const void* __restrict__ res, int rdtype,
     float* __restrict__ sum_out, const float* __restrict__ w, void* __restrict__ y, int ydtype,
@@ -100,50 +114,73 @@ __global__ __launch_bounds__(256) void ca_rmsnorm_fwd_kernel(
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= N) return;
+  if constexpr (RT != kRuntimeDtype) rdtype = RT;
+  if constexpr (YT != kRuntimeDtype) ydtype = YT;
   const size_t base = (size_t)row * C;
-  // the row's values (x, or x + res) at columns c .. c+VEC-1
-  auto load_row = [&](int c, float* v) {
-    load_vec<VEC>(x, base + c, kDtypeF32, v);
-    if constexpr (ADD) {
-      float rv[VEC];
-      load_vec<VEC>(res, base + c, rdtype, rv);
-#pragma unroll
-      for (int e = 0; e < VEC; ++e) v[e] += rv[e];
-    }
-  };
   float ss = 0.f;
   if constexpr (KMAX > 0) {
-    float xv[KMAX][VEC];
+    float xv[KMAX][VEC], wv[KMAX][VEC];
+    if constexpr (KMAX == kChunks) {  // more would cost registers
 #pragma unroll
-    for (int u = 0; u < KMAX; ++u) {
-      const int c = (lane + 64 * u) * VEC;
-      if (c < C) {
-        load_row(c, xv[u]);
-        if constexpr (ADD) store_vec<VEC>(sum_out, base + c, kDtypeF32, xv[u]);
-      } else {
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) xv[u][e] = 0.f;
+      for (int u = 0; u < KMAX; ++u) {
+        const int c = (lane + 64 * u) * VEC;
+        if (c < C) load_vec<VEC>(w, c, kDtypeF32, wv[u]);
       }
     }
 #pragma unroll
-    for (int u = 0; u < KMAX; ++u)
+    for (int u0 = 0; u0 < KMAX; u0 += kChunks) {
+      float rv[ADD ? kChunks : 1][VEC];
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) ss = fmaf(xv[u][e], xv[u][e], ss);
+      for (int i = 0; i < kChunks; ++i) {
+        const int c = (lane + 64 * (u0 + i)) * VEC;
+        if (c < C) {
+          load_vec<VEC>(x, base + c, kDtypeF32, xv[u0 + i]);
+          if constexpr (ADD) load_vec<VEC>(res, base + c, rdtype, rv[i]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) {
+            xv[u0 + i][e] = 0.f;
+            if constexpr (ADD) rv[i][e] = 0.f;
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < kChunks; ++i) {
+        if constexpr (ADD) {
+          const int c = (lane + 64 * (u0 + i)) * VEC;
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) xv[u0 + i][e] += rv[i][e];
+          if (c < C) store_vec<VEC>(sum_out, base + c, kDtypeF32, xv[u0 + i]);
+        }
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) ss = fmaf(xv[u0 + i][e], xv[u0 + i][e], ss);
+      }
+      if constexpr (KMAX > kChunks) asm volatile("" ::: "memory");
+    }
     ss = wave_sum(ss);
     const float r = 1.0f / sqrtf(ss / (float)C + eps);
 #pragma unroll
     for (int u = 0; u < KMAX; ++u) {
       const int c = (lane + 64 * u) * VEC;
       if (c < C) {
-        float wv[VEC];
-        load_vec<VEC>(w, c, kDtypeF32, wv);
+        if constexpr (KMAX > kChunks) load_vec<VEC>(w, c, kDtypeF32, wv[u]);
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) wv[e] = wv[e] * xv[u][e] * r;
-        store_vec<VEC>(y, base + c, ydtype, wv);
+        for (int e = 0; e < VEC; ++e) wv[u][e] = wv[u][e] * xv[u][e] * r;
+        store_vec<VEC>(y, base + c, ydtype, wv[u]);
       }
     }
     if (lane == 0) rstd[row] = r;
   } else {
+    // the row's values (x, or x + res) at columns c .. c+VEC-1
+    auto load_row = [&](int c, float* v) {
+      load_vec<VEC>(x, base + c, kDtypeF32, v);
+      if constexpr (ADD) {
+        float rv[VEC];
+        load_vec<VEC>(res, base + c, rdtype, rv);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) v[e] += rv[e];
+      }
+    };
     for (int c = lane * VEC; c < C; c += 64 * VEC) {
       float xv[VEC];
       load_row(c, xv);
@@ -172,8 +209,14 @@ __global__ __launch_bounds__(256) void ca_rmsnorm_fwd_kernel(
 // the four rows in wave order.  KMAX as in the forward (x, dy and w of the
 // row held in registers).  ADD (x is the sum s = x + res of the forward):
 // dx += dsum (the gradient s receives from its other consumers, if any), and
-// dx is also written to dres in rdtype, the gradient of res.
-template <int VEC, int KMAX, bool ADD>
+// dx is also written to dres in rdtype, the gradient of res.  DT and RT are
+// dydtype and rdtype as in the forward; dsum is loaded with the row, not after
+// its reduction, and up to C = 1024 the sums of dy * xh stay in registers
+// (LDS only for the last sum over the waves).
+// Before / now, us, at the forward's sizes: 6.4 / 5.2, 10.5 / 8.5, 29.3 / 24.1
+// (134 MB: 5.6 TB/s), 16.7 / 14.5, 26.2 / 23.0, 15.8 / 11.9, 115 / 103.  Eight
+// waves per work group measured no better (26.5 at [8192, 1024]).
+template <int VEC, int KMAX, bool ADD, int DT, int RT>
 __global__ __launch_bounds__(256) void ca_rmsnorm_bwd_kernel(
     const void* __restrict__ dy, int dydtype, const float* __restrict__ dsum,
     const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ rstd,
@@ -181,19 +224,22 @@ __global__ __launch_bounds__(256) void ca_rmsnorm_bwd_kernel(
     int N, int C, int rows_per_block) {
   extern __shared__ float acc[];
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if constexpr (DT != kRuntimeDtype) dydtype = DT;
+  if constexpr (RT != kRuntimeDtype) rdtype = RT;
+  constexpr bool kRegSum = KMAX == kChunks;
   float* mine = acc + (size_t)wv * C;
-  for (int c = lane * VEC; c < C; c += 64 * VEC)
+  if constexpr (!kRegSum) {
+    for (int c = lane * VEC; c < C; c += 64 * VEC)
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) mine[c + e] = 0.f;
+      for (int e = 0; e < VEC; ++e) mine[c + e] = 0.f;
+  }
   const int r0 = blockIdx.x * rows_per_block;
   const int r1 = min(r0 + rows_per_block, N);
   // the gradient d of columns c .. c+VEC-1 of the row at base: stored to dx
-  // (and, with ADD, plus dsum, to dx and dres)
-  auto put = [&](size_t base, int c, float* d) {
+  // (and, with ADD, plus dsum's values e2, to dx and dres)
+  auto put = [&](size_t base, int c, float* d, const float* e2) {
     if constexpr (ADD) {
       if (dsum) {
-        float e2[VEC];
-        load_vec<VEC>(dsum, base + c, kDtypeF32, e2);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) d[e] += e2[e];
       }
@@ -202,10 +248,14 @@ __global__ __launch_bounds__(256) void ca_rmsnorm_bwd_kernel(
     store_vec<VEC>(dx, base + c, kDtypeF32, d);
   };
   if constexpr (KMAX > 0) {
-    float wt[KMAX][VEC];
+    float wt[KMAX][VEC], sum[kRegSum ? KMAX : 1][VEC];
 #pragma unroll
     for (int u = 0; u < KMAX; ++u) {
       const int c = (lane + 64 * u) * VEC;
+      if constexpr (kRegSum) {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) sum[u][e] = 0.f;
+      }
       if (c < C) {
         load_vec<VEC>(w, c, kDtypeF32, wt[u]);
       } else {
@@ -216,7 +266,7 @@ __global__ __launch_bounds__(256) void ca_rmsnorm_bwd_kernel(
     for (int row = r0 + wv; row < r1; row += 4) {
       const size_t base = (size_t)row * C;
       const float r = rstd[row];
-      float xv[KMAX][VEC], g[KMAX][VEC];
+      float xv[KMAX][VEC], g[KMAX][VEC], e2[kRegSum ? KMAX : 1][VEC];
 #pragma unroll
       for (int u = 0; u < KMAX; ++u) {
         const int c = (lane + 64 * u) * VEC;
@@ -226,6 +276,15 @@ __global__ __launch_bounds__(256) void ca_rmsnorm_bwd_kernel(
         } else {
 #pragma unroll
           for (int e = 0; e < VEC; ++e) xv[u][e] = g[u][e] = 0.f;
+        }
+      }
+      if constexpr (ADD && kRegSum) {
+        if (dsum) {
+#pragma unroll
+          for (int u = 0; u < KMAX; ++u) {
+            const int c = (lane + 64 * u) * VEC;
+            if (c < C) load_vec<VEC>(dsum, base + c, kDtypeF32, e2[u]);
+          }
         }
       }
       float s = 0.f;
@@ -243,9 +302,25 @@ __global__ __launch_bounds__(256) void ca_rmsnorm_bwd_kernel(
           for (int e = 0; e < VEC; ++e) {
             const float xh = xv[u][e] * r;
             d[e] = r * fmaf(-xh, mean, wt[u][e] * g[u][e]);
-            mine[c + e] = fmaf(g[u][e], xh, mine[c + e]);
+            if constexpr (kRegSum) sum[u][e] = fmaf(g[u][e], xh, sum[u][e]);
+            else mine[c + e] = fmaf(g[u][e], xh, mine[c + e]);
           }
-          put(base, c, d);
+          if constexpr (kRegSum) {
+            put(base, c, d, e2[u]);
+          } else {
+            if (ADD && dsum) load_vec<VEC>(dsum, base + c, kDtypeF32, e2[0]);
+            put(base, c, d, e2[0]);
+          }
+        }
+      }
+    }
+    if constexpr (kRegSum) {
+#pragma unroll
+      for (int u = 0; u < KMAX; ++u) {
+        const int c = (lane + 64 * u) * VEC;
+        if (c < C) {
+#pragma unroll
+          for (int e = 0; e < VEC; ++e) mine[c + e] = sum[u][e];
         }
       }
     }
@@ -264,7 +339,8 @@ __global__ __launch_bounds__(256) void ca_rmsnorm_bwd_kernel(
       }
       const float mean = wave_sum(s) / (float)C;
       for (int c = lane * VEC; c < C; c += 64 * VEC) {
-        float xv[VEC], wt[VEC], g[VEC], d[VEC];
+        float xv[VEC], wt[VEC], g[VEC], d[VEC], e2[VEC];
+        if (ADD && dsum) load_vec<VEC>(dsum, base + c, kDtypeF32, e2);
         load_vec<VEC>(x, base + c, kDtypeF32, xv);
         load_vec<VEC>(w, c, kDtypeF32, wt);
         load_vec<VEC>(dy, base + c, dydtype, g);
@@ -274,7 +350,7 @@ __global__ __launch_bounds__(256) void ca_rmsnorm_bwd_kernel(
           d[e] = r * fmaf(-xh, mean, wt[e] * g[e]);
           mine[c + e] = fmaf(g[e], xh, mine[c + e]);
         }
-        put(base, c, d);
+        put(base, c, d, e2);
       }
     }
   }
@@ -321,6 +397,19 @@ int rmsnorm_bwd_blocks(int N) {
 
 static bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// Calls f(T0, T1) with two element types as compile-time constants.
+template <class F>
+static void with_dtypes(int t0, int t1, F f) {
+  auto second = [&](auto a) {
+    if (t1 == kDtypeF32) f(a, std::integral_constant<int, kDtypeF32>{});
+    else if (t1 == kDtypeBF16) f(a, std::integral_constant<int, kDtypeBF16>{});
+    else f(a, std::integral_constant<int, kDtypeF16>{});
+  };
+  if (t0 == kDtypeF32) second(std::integral_constant<int, kDtypeF32>{});
+  else if (t0 == kDtypeBF16) second(std::integral_constant<int, kDtypeBF16>{});
+  else second(std::integral_constant<int, kDtypeF16>{});
+}
+
 // The 4-wide path needs C % 4 == 0 and 16-byte aligned bases (every row of
 // an fp32 tensor is then 16-byte aligned, of a 16-bit tensor 8-byte aligned).
 template <bool ADD>
@@ -329,15 +418,19 @@ static hipError_t rms_fwd(const float* x, const void* res, int rdtype, float* su
                           float eps, hipStream_t s) {
   const bool v4 = C % 4 == 0 && al16(x) && al16(w) && al16(y) && (!ADD || (al16(res) && al16(sum_out)));
   const dim3 grid((N + 3) / 4);
-  if (v4 && C <= 1024)
-    hipLaunchKernelGGL((ca_rmsnorm_fwd_kernel<4, 4, ADD>), grid, dim3(256), 0, s, x, res, rdtype,
-                       sum_out, w, y, ydtype, rstd, N, C, eps);
-  else if (v4)
-    hipLaunchKernelGGL((ca_rmsnorm_fwd_kernel<4, 16, ADD>), grid, dim3(256), 0, s, x, res, rdtype,
-                       sum_out, w, y, ydtype, rstd, N, C, eps);
+  if (!v4)
+    hipLaunchKernelGGL((ca_rmsnorm_fwd_kernel<1, 0, ADD, kRuntimeDtype, kRuntimeDtype>), grid,
+                       dim3(256), 0, s, x, res, rdtype, sum_out, w, y, ydtype, rstd, N, C, eps);
   else
-    hipLaunchKernelGGL((ca_rmsnorm_fwd_kernel<1, 0, ADD>), grid, dim3(256), 0, s, x, res, rdtype,
-                       sum_out, w, y, ydtype, rstd, N, C, eps);
+    with_dtypes(ADD ? rdtype : kDtypeF32, ydtype, [&](auto r, auto t) {
+      constexpr int RT = ADD ? decltype(r)::value : kDtypeF32, YT = decltype(t)::value;
+      if (C <= 1024)
+        hipLaunchKernelGGL((ca_rmsnorm_fwd_kernel<4, 4, ADD, RT, YT>), grid, dim3(256), 0, s, x, res,
+                           rdtype, sum_out, w, y, ydtype, rstd, N, C, eps);
+      else
+        hipLaunchKernelGGL((ca_rmsnorm_fwd_kernel<4, 16, ADD, RT, YT>), grid, dim3(256), 0, s, x, res,
+                           rdtype, sum_out, w, y, ydtype, rstd, N, C, eps);
+    });
   return hipGetLastError();
 }
 
@@ -350,15 +443,20 @@ static hipError_t rms_bwd(const void* dy, int dydtype, const float* dsum, const 
   const size_t lds = 4 * (size_t)C * sizeof(float);
   const bool v4 = C % 4 == 0 && al16(dy) && al16(x) && al16(w) && al16(dx) &&
                   (!ADD || (al16(dres) && (!dsum || al16(dsum))));
-  if (v4 && C <= 1024)
-    hipLaunchKernelGGL((ca_rmsnorm_bwd_kernel<4, 4, ADD>), dim3(nb), dim3(256), lds, s, dy, dydtype,
-                       dsum, x, w, rstd, dx, dres, rdtype, dw_part, N, C, rpb);
-  else if (v4)
-    hipLaunchKernelGGL((ca_rmsnorm_bwd_kernel<4, 16, ADD>), dim3(nb), dim3(256), lds, s, dy, dydtype,
-                       dsum, x, w, rstd, dx, dres, rdtype, dw_part, N, C, rpb);
+  if (!v4)
+    hipLaunchKernelGGL((ca_rmsnorm_bwd_kernel<1, 0, ADD, kRuntimeDtype, kRuntimeDtype>), dim3(nb),
+                       dim3(256), lds, s, dy, dydtype, dsum, x, w, rstd, dx, dres, rdtype, dw_part, N,
+                       C, rpb);
   else
-    hipLaunchKernelGGL((ca_rmsnorm_bwd_kernel<1, 0, ADD>), dim3(nb), dim3(256), lds, s, dy, dydtype,
-                       dsum, x, w, rstd, dx, dres, rdtype, dw_part, N, C, rpb);
+    with_dtypes(dydtype, ADD ? rdtype : kDtypeF32, [&](auto t, auto r) {
+      constexpr int DT = decltype(t)::value, RT = ADD ? decltype(r)::value : kDtypeF32;
+      if (C <= 1024)
+        hipLaunchKernelGGL((ca_rmsnorm_bwd_kernel<4, 4, ADD, DT, RT>), dim3(nb), dim3(256), lds, s, dy,
+                           dydtype, dsum, x, w, rstd, dx, dres, rdtype, dw_part, N, C, rpb);
+      else
+        hipLaunchKernelGGL((ca_rmsnorm_bwd_kernel<4, 16, ADD, DT, RT>), dim3(nb), dim3(256), lds, s,
+                           dy, dydtype, dsum, x, w, rstd, dx, dres, rdtype, dw_part, N, C, rpb);
+    });
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(ca_rmsnorm_dw_kernel, dim3((C + 15) / 16), dim3(256), 0, s, dw_part, dw, nb, C);
