@@ -57,6 +57,15 @@ struct Fwd {
   static constexpr int VPLANE = D * VROW;
 };
 
+// kTileSum.  Both forward kernels form a tile's V^T W^T in accumulators of its
+// own and add it to O^T with one addition per element.  Accumulated in O^T
+// itself, each of a tile's six limb products (three in bf16) rounds at the size
+// of O^T, and the error grows with the tiles summed without a break: output
+// error from float64 at [1,4,8192,64] fp32 with splits of 24 / 64 / 256 tiles
+// 2.9 / 3.8 / 5.1e-7 against 1.55 / 1.63 / 1.79e-7 with one addition per tile
+// (large scores 6.5 / 7.2 / 8.5e-7 against 6.1 / 6.2 / 6.4e-7), so that the
+// split length is free to follow the time.  It costs 16 VALU additions per tile
+// and lane: 0.5-1.5% of the fp32 forward, 3% of the bf16 one.
 // LDS row of the permuted K tile that holds tile key k (inverse of key_of_arow).
 __device__ __forceinline__ int arow_of_key(int k) {
   return (((k >> 2) & 3) << 3) | (((k >> 4) & 1) << 2) | (k & 3);
@@ -84,14 +93,12 @@ __device__ __forceinline__ float halo_dot(const float* qreg, const E* __restrict
   return acc + xhalf(acc);
 }
 
-// Waves per SIMD the register budget is set for: bf16 operands stage one
-// limb plane and take one product per k block of S, so with keys rotated
-// beforehand (no table reads) they fit four (128 VGPRs, 20 KB of LDS per
-// work group; one CA-S layer's forward 0.0708 -> 0.0689 ms), with in-kernel
-// key rotation three; other operand types two.
+// Waves per SIMD the register budget is set for (head dims 8, 16 and 32): what
+// the kernels fit without spilling.  Left to itself the compiler takes 145
+// VGPRs at D <= 16, fp32, and with them the fourth wave.
 template <int D, class E, bool ROPE>
 constexpr int fwd_waves_per_simd() {
-  return D > 64 ? 1 : std::is_same<E, __bf16>::value ? (ROPE ? 3 : 4) : 2;
+  return D <= 16 ? 4 : std::is_same<E, __bf16>::value ? (ROPE ? 3 : 4) : 3;
 }
 
 template <int D, class E, bool ROPE>
@@ -422,7 +429,13 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
       zsum += zt + r_in;
       prio_mfma_begin<!BF>();
 
-      // ---- O^T += V^T W^T: k block kb, element e = weight key 16h + 8kb + e ----
+      // ---- O^T += V^T W^T: k block kb, element e = weight key 16h + 8kb + e;
+      // the tile's product is formed from zero and added once (see kTileSum) ----
+      f32x16 part_o[P::NMB];
+#pragma unroll
+      for (int mb = 0; mb < P::NMB; ++mb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) part_o[mb][r] = 0.f;
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
         float x[8];
@@ -434,9 +447,11 @@ __global__ __launch_bounds__(256, (fwd_waves_per_simd<D, E, ROPE>())) void ca_fw
           const __bf16* vrow = &lds_vt[buf][0][(dok ? 32 * mb + q : 0) * P::VROW + 16 * h + 8 * kb];
           Limbs va = limbs_at<NL>(vrow, P::VPLANE);
           if (!dok) va = Limbs{bf16x8{}, bf16x8{}, bf16x8{}};
-          acc_o[mb] = mfma32_limbs<NL, 3>(va, wb, acc_o[mb]);
+          part_o[mb] = mfma32_limbs<NL, 3>(va, wb, part_o[mb]);
         }
       }
+#pragma unroll
+      for (int mb = 0; mb < P::NMB; ++mb) acc_o[mb] += part_o[mb];
       prio_mfma_end<!BF>();
     };
     if (wave_active && t <= wave_tmax) {
@@ -577,10 +592,12 @@ __device__ __forceinline__ float halo_dot16(const float (&qv)[Fwd16<D>::KS][8],
 }
 
 // Waves per SIMD: two work groups of eight waves per CU at D <= 64; one at
-// D = 128 (its double-buffered tiles take 116 KB of LDS).
+// D = 128 (its double-buffered tiles take 116 KB of LDS in fp32, 78 in fp16), but
+// two in bf16 (39 KB, 124 VGPRs; without the bound 145 and one work group:
+// [2,16,2048,128] with 12-tile splits 186 against 148 us).
 template <int D, class E, bool ROPE>
 constexpr int fwd16_waves_per_simd() {
-  return D > 64 ? 2 : 4;
+  return D > 64 && (ROPE || !std::is_same<E, __bf16>::value) ? 2 : 4;
 }
 
 template <int D, class E, bool ROPE>
@@ -865,22 +882,26 @@ __global__ __launch_bounds__(512, (fwd16_waves_per_simd<D, E, ROPE>())) void ca_
       wt[0] += r_in;
       zsum += zt + r_in;
 
-      // ---- O^T += V^T W^T: k = weight key 8G + e, d blocks in pairs ----
+      // ---- O^T += V^T W^T: k = weight key 8G + e, d blocks in pairs; the
+      // tile's product is formed from zero and added once (see kTileSum) ----
       const Limbs wb = split8(wt);
       prio_mfma_begin<!BF>();
 #pragma unroll
       for (int m2 = 0; m2 < P::NMB; m2 += 2) {
         Limbs va[2];
+        f32x4 part_o[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
         for (int u = 0; u < 2; ++u)
           va[u] = limbs_at<NL>(&lds_vt[buf][0][(16 * (m2 + u) + q16) * P::VROW + 8 * G4], P::VPLANE);
 #pragma unroll
         for (int st = 0; st < 6; ++st) {
           if (limb_step_used<NL, 3>(st)) {
-            acc_o[m2] = mfma16_step(st, va[0], wb, acc_o[m2]);
-            acc_o[m2 + 1] = mfma16_step(st, va[1], wb, acc_o[m2 + 1]);
+            part_o[0] = mfma16_step(st, va[0], wb, part_o[0]);
+            part_o[1] = mfma16_step(st, va[1], wb, part_o[1]);
           }
         }
+        acc_o[m2] += part_o[0];
+        acc_o[m2 + 1] += part_o[1];
       }
       prio_mfma_end<!BF>();
     };

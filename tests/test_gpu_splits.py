@@ -46,3 +46,26 @@ def test_picked_splits_match_whole_items(gpu_ca, shape, dtype, cap):
         # the gain gradient sums T^2 / 2 signed terms per slice
         tol = 5e-6 if i < 4 else 1e-4
         assert bool(((a - b).abs() <= step * b.abs() + tol * b.abs().max()).all()), i
+
+
+@pytest.mark.parametrize("T,D", [(8192, 64), (4096, 32), (4096, 8), (4096, 128)])
+def test_uncut_rows_as_accurate_as_short_splits(gpu_ca, T, D):
+    """A row's output over n tiles in one split, against 12-tile splits.  Of the
+    difference, at most half an ulp per rounding with random signs (rms 2^-24 /
+    sqrt(3) of the running sum): one rounding per tile of a sum growing like
+    the square root of the tiles (n / 2 in squares) and of Z, growing linearly
+    (n / 3), and the split side's 12 tiles and merge of n / 12 partials (6 + n /
+    24): 2^-24 sqrt(0.3 n + 2) of the output's norm, n <= T / 32."""
+    q, k, v, rho, _ = make_inputs((1, 2, T, D), 17, 1.0, [0.1, -0.1])
+    t = [x.cuda() for x in (q, k, v, rho)]
+    out = []
+    try:
+        for tiles in (12, 1 << 20):
+            gpu_ca.ops.set_split_override(tiles, 0, 0)
+            with torch.no_grad():
+                out.append(gpu_ca.continuum_attention(*t).double())
+    finally:
+        gpu_ca.ops.set_split_override()
+    rows = slice(T // 2, T)
+    err = float((out[1] - out[0])[:, :, rows].norm() / out[0][:, :, rows].norm())
+    assert err <= 2.0 ** -24 * (0.3 * T / 32 + 2) ** 0.5, err
