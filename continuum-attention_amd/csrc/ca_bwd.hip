@@ -306,7 +306,11 @@ __global__ __launch_bounds__(256, (std::is_same<E, __bf16>::value && D <= 64 ? 4
   // neighbouring keys nearly coincide the products stay small instead of
   // cancelling (|k| ~ 1 against |k_j - k_ref| ~ 1e-2 in the near-duplicate-key
   // case).  All chunks of a group use the same k_ref, so the k_ref terms
-  // cancel in the sum of the chunk partials.
+  // cancel in the sum of the chunk partials.  Zero-padded head dims take the
+  // mean of kDqRefs keys that every row of the group sees: between unrelated
+  // keys |k_j - k_ref| is sqrt(2) |k|, against the mean 1.06 |k|, and the
+  // rounding of dS is weighed by it (dQ error at [2,8,768,24], large scores,
+  // 6.8e-7 against 5.4e-7; query tiles, which take no k_ref, 7.3e-7).
   // Staging unit u: slot (key of the stage) u / C4, d = 4(u % C4)..+3; a
   // thread's units all have d chunk tid % C4, since 256 % C4 == 0.
   // rows of K (rotated here when ROPE; otherwise they arrive rotated, or
@@ -329,7 +333,19 @@ __global__ __launch_bounds__(256, (std::is_same<E, __bf16>::value && D <= 64 ? 4
   // small, matters at fp32 key spacings; bf16 keys differ by at least 2^-8
   // of their size, so the unshifted sum loses at most 2^-16 of it)
   constexpr bool BF = std::is_same<E, __bf16>::value;
-  const f32x4 kref = BF ? f32x4{0.f, 0.f, 0.f, 0.f} : k_row4(kDqRows * qg, 4 * (tid % P::C4));
+  f32x4 kref = {0.f, 0.f, 0.f, 0.f};
+  if (!BF) {
+    const int d0 = 4 * (tid % P::C4), first = kDqRows * qg;
+    if (hd != D) {
+      f32x4 r[kDqRefs];
+#pragma unroll
+      for (int u = 0; u < kDqRefs; ++u) r[u] = k_row4(u * first / (kDqRefs - 1), d0);
+      // pairwise: exact where the keys coincide
+      kref = (((r[0] + r[1]) + (r[2] + r[3])) + ((r[4] + r[5]) + (r[6] + r[7]))) * (1.0f / kDqRefs);
+    } else {
+      kref = k_row4(first, d0);
+    }
+  }
   // K rows (and RoPE table rows) through buffer resources: a stage's offsets
   // are the thread's fixed offsets plus one uniform step per stage, and rows
   // at or past T read as zeros.  Those rows become -k_ref after the shift and

@@ -999,11 +999,28 @@ __global__ __launch_bounds__(256) void ca_fwd_combine_kernel(const float* __rest
   }
 }
 
-// Head dims that run the 16x16x32 forward (the 32x32x16 kernel serves the
-// others).
-template <int D>
-constexpr bool fwd_uses_16x16() {
-  return D == 64 || D == 128;
+// The 16x16x32 forward serves D = 64 and 128, the 32x32x16 kernel the smaller
+// head dims.  At 32, where the 32x32x16 kernel is the faster one
+// ([2,16,2048,32] fp32 97 against 117 us), the 16x16x32 kernel serves the
+// zero-padded head dims 17 to 31: its scores equal the dK/dV kernel's bit for
+// bit, so that the backward's weights sum to the Z they are divided by.  With
+// large scores they otherwise do not to fp32 accuracy (dQ error at
+// [2,8,768,24] 1.2e-6, query tiles 7.3e-7).
+template <int D, class E, bool ROPE>
+static void launch_fwd_kernel(const FwdIO& io, float* part, int BH, int H, int T, int C, int G,
+                              int smax, int items, hipStream_t stream) {
+  if constexpr (D > 32 || (D == 32 && !ROPE)) {  // padded rows come without RoPE
+    if (D > 32 || io.head_dim != D) {
+      hipLaunchKernelGGL((ca_fwd16_kernel<D, E, ROPE>), dim3(items * BH), dim3(512), 0, stream,
+                         io.q, io.k, io.v, io.rope, io.log_gain, io.y, io.out, io.stats, part, BH, H,
+                         T, C, G, smax, io.head_dim);
+      return;
+    }
+  }
+  if constexpr (D <= 32)
+    hipLaunchKernelGGL((ca_fwd_kernel<D, E, ROPE>), dim3(items * BH), dim3(256), 0, stream, io.q,
+                       io.k, io.v, io.rope, io.log_gain, io.y, io.out, io.stats, part, BH, H, T, C,
+                       G, smax, io.head_dim);
 }
 
 template <int D, class E>
@@ -1014,25 +1031,10 @@ hipError_t launch_fwd(const FwdIO& io, float* part, int B, int H, int T, int C,
   const int smax = fwd_max_splits(T, C);
   const int items = fwd_num_items(T, C);
   timer_begin(kFwd, stream);
-  if constexpr (fwd_uses_16x16<D>()) {
-    if (io.rope && !io.k_rotated)
-      hipLaunchKernelGGL((ca_fwd16_kernel<D, E, true>), dim3(items * BH), dim3(512), 0, stream,
-                         io.q, io.k, io.v, io.rope, io.log_gain, io.y, io.out, io.stats, part, BH, H,
-                         T, C, G, smax, io.head_dim);
-    else
-      hipLaunchKernelGGL((ca_fwd16_kernel<D, E, false>), dim3(items * BH), dim3(512), 0, stream,
-                         io.q, io.k, io.v, io.rope, io.log_gain, io.y, io.out, io.stats, part, BH, H,
-                         T, C, G, smax, io.head_dim);
-  } else {
-    if (io.rope && !io.k_rotated)
-      hipLaunchKernelGGL((ca_fwd_kernel<D, E, true>), dim3(items * BH), dim3(256), 0, stream, io.q,
-                         io.k, io.v, io.rope, io.log_gain, io.y, io.out, io.stats, part, BH, H, T,
-                         C, G, smax, io.head_dim);
-    else
-      hipLaunchKernelGGL((ca_fwd_kernel<D, E, false>), dim3(items * BH), dim3(256), 0, stream, io.q,
-                         io.k, io.v, io.rope, io.log_gain, io.y, io.out, io.stats, part, BH, H, T,
-                         C, G, smax, io.head_dim);
-  }
+  if (io.rope && !io.k_rotated)
+    launch_fwd_kernel<D, E, true>(io, part, BH, H, T, C, G, smax, items, stream);
+  else
+    launch_fwd_kernel<D, E, false>(io, part, BH, H, T, C, G, smax, items, stream);
   timer_end(kFwd, stream);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;

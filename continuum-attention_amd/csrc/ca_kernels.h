@@ -498,6 +498,8 @@ template <class E> __host__ __device__ constexpr int q_limb_planes() { return va
 // Keys of a slice, evenly spread, whose mean serves as its typical key in the
 // gain gradient.
 constexpr int kGainRefs = 4;
+// Keys whose mean the dQ pass takes zero-padded rows' keys relative to.
+constexpr int kDqRefs = 8;
 // kDpFlip.  The matrix cores round their fp32 sums slightly downwards,
 // whatever the sign (about 2^-28 of the accumulator per dP' element,
 // measured): a bias common to a row's weight gradients, which the row's dS

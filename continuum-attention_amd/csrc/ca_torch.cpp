@@ -163,7 +163,8 @@ py::object op(py::handle qo, py::handle ko, py::handle vo, py::handle go) {
     return py::none();
   for (const Tensor* t : {&k, &v, &gain})
     if (t->device() != q.device()) return py::none();
-  const int64_t D = q.size(3), DP = D <= 128 ? ca_padded_head_dim((int)D) : 0;
+  // head dims below 8 run query tiles (ops._fused)
+  const int64_t D = q.size(3), DP = D >= 8 && D <= 128 ? ca_padded_head_dim((int)D) : 0;
   if (!DP || q.size(2) > 65536 || q.numel() / D * DP > ((int64_t)1 << 31) - 1) return py::none();
   Tensor out;
   {

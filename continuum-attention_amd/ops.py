@@ -17,9 +17,9 @@ round the output and the gradients to that type once.  ``query_tile`` is
 accepted and validated; in the reference it only bounds the memory of the
 materialised ``[BH, Qt, K]`` weights (cuda/continuum_attention.py:957), which
 the fused kernels never materialise, so it does not change their arithmetic.
-They serve head dims up to 128 (8, 16, 32, 64 and 128 directly, others on rows
-padded with zeros); larger ones run the reference's query-tile structure,
-where it does bound memory.  All ``CA_CUDA_MODE`` values select the same exact
+They serve head dims from 8 to 128 (8, 16, 32, 64 and 128 directly, others on
+rows padded with zeros); smaller and larger ones run the reference's query-tile
+structure, where it does bound memory.  All ``CA_CUDA_MODE`` values select the same exact
 fp32 path (the reference modes differ only in fp16 rounding and launch
 structure).
 
@@ -206,14 +206,17 @@ _MAX_ELEMS = (1 << 31) - 1  # and their limit on the elements of a tensor
 
 def _fused(q, k, v) -> bool:
     """Whether the fused kernels serve these tensors.  Head dims with kernels
-    of their own always go there (which reports what they refuse); others up
-    to 128, zero-padded, where the padded problem is within the kernels'
-    limits (shapes of q, k and v that differ stay with the query-tile path,
-    whose matmuls decide)."""
+    of their own always go there (which reports what they refuse); others
+    between 8 and 128, zero-padded, where the padded problem is within the
+    kernels' limits (shapes of q, k and v that differ stay with the query-tile
+    path, whose matmuls decide).  Below 8 a score is a product of so few terms
+    that query tiles round it less than the kernels (dQ and dV errors with large
+    scores, [2,8,768,4]: 6.5e-7 and 3.0e-7 against 7.4e-7 and 3.2e-7)."""
     D = q.shape[-1]
     if D in SUPPORTED_HEAD_DIMS:
         return True
-    if not 0 < D < SUPPORTED_HEAD_DIMS[-1] or k.shape != q.shape or v.shape != q.shape:
+    if (not SUPPORTED_HEAD_DIMS[0] < D < SUPPORTED_HEAD_DIMS[-1] or k.shape != q.shape
+            or v.shape != q.shape):
         return False
     padded = next(d for d in SUPPORTED_HEAD_DIMS if d > D)
     return q.shape[2] <= _MAX_T and q.numel() // D * padded <= _MAX_ELEMS
@@ -284,7 +287,7 @@ def _op_backward(q, k, v, log_gain, y, stats, dout):
 
 # ---- any head dimension: the query-tile structure over the HIP weight kernels
 #
-# Head dims above 128 (and padded problems past the kernels' limits) run the
+# Head dims below 8 and above 128 (and padded problems past the kernels' limits) run the
 # reference operator's own structure (cuda/continuum_attention.py:666-694 and
 # :707-764) on the device: per query tile, fp32 GEMMs for the scores, W.V and
 # the gradient contractions, and the HIP weight kernels (ca_weights_f32,
@@ -432,7 +435,7 @@ def continuum_attention(q, k, v, log_gain, query_tile=64):
     """Exact causal Continuum Attention (cuda/continuum_attention.py:768-783).
 
     q, k, v: ``[B, H, T, D]`` (same dtype), log_gain: ``[H]``.  On the GPU,
-    D up to 128 runs the fused kernels and larger D the query-tile structure
+    D from 8 to 128 runs the fused kernels and other D the query-tile structure
     over the HIP weight kernels (``query_tile`` rows at a time); CPU tensors
     run the float32 CPU path (``cpu.py``).
     Scores are ``exp(log_gain[h]) / sqrt(D) * q.k``; keys and values are
