@@ -103,11 +103,14 @@ __global__ __launch_bounds__(256) void ca_bwd_prep_kernel(View Qv, View Kv,
     // r = 2 L - s_ref is that mean for normally distributed scores (L - s_ref
     // is half their variance) and near it for peaked rows.  Moved by whole
     // octaves, weights and 1/Z scale exactly.
+    // The reference keys are ones the row sees: a non-finite later key leaves
+    // the row as it is.
     float sref = 0.f;
     const E* kp = view_slice<const E>(Kv, bh, H) + 8 * c;
+    const int seen = min(t, T - 1) + 1;
 #pragma unroll
     for (int k = 0; k < kGainRefs; ++k) {
-      const E* kk = kp + (long long)((long long)k * T / kGainRefs) * Kv.rstride;
+      const E* kk = kp + (long long)(k * seen / kGainRefs) * Kv.rstride;
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         const f32x4 kx = ld4(kk + 4 * u);
@@ -120,7 +123,7 @@ __global__ __launch_bounds__(256) void ca_bwd_prep_kernel(View Qv, View Kv,
     sref *= head_scale_log2(log_gain, bh % H, hd) * (1.0f / kGainRefs);
     const float lmean = m - __log2f(invz) - __log2f((float)(t + 1));
     const float n = rintf(m - (2.0f * lmean - sref)) + kShareShift;
-    if (ok && fabsf(n) < 48.f) {  // also false for rows with NaN or infinite scores
+    if (ok && fabsf(n) < 48.f) {
       m -= n;
       invz *= fast_exp2(-n);
     }

@@ -1,5 +1,6 @@
 """Zero-padded head dims against the query-tile path, which serves the other head
-dims without kernels of their own: no larger an error from the float64 oracle."""
+dims without kernels of their own: no larger an error from the float64 oracle,
+and nothing that depends on keys a row does not see."""
 import numpy as np
 import pytest
 import torch
@@ -41,3 +42,19 @@ def test_no_less_accurate_than_query_tiles(gpu_ca, D, scale):
             err[row] += [_rel2(a, b) / 3 for a, b in zip(got[:4], ref)]
     say(str(err))
     assert (err[0] <= 1.03 * err[1]).all(), err
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+def test_rows_do_not_depend_on_later_keys(gpu_ca, dtype):
+    """A NaN in a key leaves the output and dQ of the rows before its 128-query
+    group bit for bit as they are."""
+    T, D, bad = 400, 40, 300
+    q, k, v, rho, dy = make_inputs((1, 2, T, D), 8)
+    q, k, v, dy = (x.to(dtype) for x in (q, k, v, dy))
+    clean = _fused(gpu_ca, (q, k, v, rho), dy)
+    k = k.clone()
+    k[:, :, bad] = float("nan")
+    got = _fused(gpu_ca, (q, k, v, rho), dy)
+    for a, b in zip(got[:2], clean[:2]):
+        assert torch.equal(a[:, :, :256], b[:, :, :256])
+        assert bool(a[:, :, bad:].isnan().all())
