@@ -214,24 +214,94 @@ class RMSNorm(nn.Module):
         return s, self(s)
 
 
+# ---- RoPE tables, kept per shape ---------------------------------------------
+#
+# A table is built by kernels queued on the stream current at its first use and
+# then read from whichever stream asks next, so every other stream waits for the
+# event recorded behind those kernels (until they are known to have run) and is
+# noted with the allocator, which then keeps the block until that stream's queued
+# reads have run when the table is dropped.  A capture can neither wait for an
+# event from outside it nor query one: it takes only tables known to be written,
+# which are kept for good, since replays read them at any later time, and builds
+# others inside the graph, unkept, since they hold nothing before a replay.
+_TABLES_KEPT = 64
+
+
+class _Table:
+    __slots__ = ("tensors", "stream", "event", "written", "readers", "captured")
+
+    def __init__(self, tensors, stream):
+        self.tensors, self.stream = tensors, stream
+        self.event = torch.cuda.Event()
+        self.event.record(stream)
+        self.written = self.captured = False
+        self.readers = {stream.cuda_stream}
+
+    def read_on(self, stream):
+        if not self.written:
+            self.written = self.event.query()
+        if stream.cuda_stream not in self.readers:
+            for t in self.tensors:
+                t.record_stream(stream)
+            self.readers.add(stream.cuda_stream)
+        if not self.written and stream.cuda_stream != self.stream.cuda_stream:
+            stream.wait_event(self.event)
+        return self.tensors
+
+
+def _kept_table(cache, key, device, build):
+    """``build()`` (a tuple of tensors on ``device``) or its earlier result for
+    ``key``, ready for work queued on the current stream."""
+    entry = cache.get(key)
+    if device.type == "cuda":
+        if torch.cuda.is_current_stream_capturing():
+            if entry is None or not entry.written:
+                return build()
+            entry.captured = True
+            return entry.tensors
+        stream = torch.cuda.current_stream(device)
+        if entry is not None:
+            return entry.read_on(stream)
+    elif entry is not None:
+        return entry
+    with torch.inference_mode(False):  # an inference tensor could not be used in training
+        tensors = build()
+    entry = _Table(tensors, stream) if device.type == "cuda" else tensors
+    _drop_oldest(cache)
+    cache[key] = entry
+    return tensors
+
+
+def _mark_written_tables():
+    """Before a capture, with the device idle: every table kept so far can be
+    used in it."""
+    for cache in (_ROPE_CACHE, _CS_CACHE):
+        for entry in list(cache.values()):
+            if isinstance(entry, _Table) and not entry.written:
+                entry.written = entry.event.query()
+
+
+def _drop_oldest(cache):
+    if len(cache) >= _TABLES_KEPT:
+        for key, entry in list(cache.items()):
+            if not getattr(entry, "captured", False):
+                cache.pop(key, None)
+                return
+
+
 _ROPE_CACHE: dict = {}
 
 
 def _rope_tables(T, D, theta, device, dtype):
     """cos/sin of position x frequency, each frequency repeated for its pair,
     in ``dtype`` (cuda/continuum_attention.py:826-831); cached per shape."""
-    key = (T, D, float(theta), device, dtype)
-    tab = _ROPE_CACHE.get(key)
-    if tab is None:
+    def build():
         freq = 1.0 / (theta ** (torch.arange(0, D, 2, device=device, dtype=torch.float32) / D))
         phase = torch.outer(torch.arange(T, device=device, dtype=torch.float32), freq)
-        cos = phase.cos().repeat_interleave(2, -1).to(dtype)[None, None]
-        sin = phase.sin().repeat_interleave(2, -1).to(dtype)[None, None]
-        tab = (cos, sin)
-        if len(_ROPE_CACHE) > 64:
-            _ROPE_CACHE.clear()
-        _ROPE_CACHE[key] = tab
-    return tab
+        return (phase.cos().repeat_interleave(2, -1).to(dtype)[None, None],
+                phase.sin().repeat_interleave(2, -1).to(dtype)[None, None])
+
+    return _kept_table(_ROPE_CACHE, (T, D, float(theta), device, dtype), device, build)
 
 
 def _rotate_pairs(t):
@@ -256,21 +326,18 @@ def rope_cos_sin(T, D, theta, device, dtype=torch.float32):
     the operands' dtype (cuda/continuum_attention.py:828-830) and stored as
     fp32; ``theta=None`` gives the identity rotation (cos 1, sin 0, exact in
     every dtype); cached per shape and dtype."""
-    key = (T, D, None if theta is None else float(theta), device, dtype)
-    cs = _CS_CACHE.get(key)
-    if cs is None:
+    device = torch.device(device)
+
+    def build():
         if theta is None:
-            cs = torch.stack((torch.ones(T, D // 2, device=device), torch.zeros(T, D // 2, device=device)),
-                             -1).contiguous()
-        else:
-            freq = 1.0 / (theta ** (torch.arange(0, D, 2, device=device, dtype=torch.float32) / D))
-            phase = torch.outer(torch.arange(T, device=device, dtype=torch.float32), freq)
-            cs = torch.stack((phase.cos(), phase.sin()), -1)
-            cs = cs.to(dtype).float().contiguous()
-        if len(_CS_CACHE) > 64:
-            _CS_CACHE.clear()
-        _CS_CACHE[key] = cs
-    return cs
+            return (torch.stack((torch.ones(T, D // 2, device=device),
+                                 torch.zeros(T, D // 2, device=device)), -1).contiguous(),)
+        freq = 1.0 / (theta ** (torch.arange(0, D, 2, device=device, dtype=torch.float32) / D))
+        phase = torch.outer(torch.arange(T, device=device, dtype=torch.float32), freq)
+        return (torch.stack((phase.cos(), phase.sin()), -1).to(dtype).float().contiguous(),)
+
+    key = (T, D, None if theta is None else float(theta), device, dtype)
+    return _kept_table(_CS_CACHE, key, device, build)[0]
 
 
 def _aligned(x, nbytes):
@@ -706,6 +773,8 @@ class GraphedTrainStep:
                 self._forward_backward()
         torch.cuda.current_stream(dev).wait_stream(side)
         optimizer.zero_grad(set_to_none=True)
+        torch.cuda.synchronize(dev)
+        _mark_written_tables()
         self.graph = torch.cuda.CUDAGraph(keep_graph=True)
         with torch.cuda.graph(self.graph):
             self.static_loss = self._forward_backward()
