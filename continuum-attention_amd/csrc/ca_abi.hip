@@ -707,16 +707,17 @@ int run_set(const ca::BwdIO& io, int dtype, char* ws, const std::vector<ca::BwdP
 // whole backward fits, else passes over ranges of dQ groups, of every slice or
 // of sets of heads (dK, dV and dlog_gain accumulate in a fixed order).
 // kv_sums: io.dk and io.dv are the element type's gradients and the passes sum
-// dK and dV in fp32 first (the token-major backward in passes).
+// dK and dV in fp32 first (the token-major backward in passes).  first: the
+// call writes dlog_gain (else it adds to it).
 int bwd_common(const ca::BwdIO& io, int dtype, void* workspace, size_t workspace_bytes, int B,
-               int H, int T, int D, void* stream, bool kv_sums) {
+               int H, int T, int D, void* stream, bool kv_sums, bool first = true) {
   BwdPlan plan;
   if (!workspace || !plan_bwd(B, H, T, D, workspace_bytes, kv_sums, &plan))
     return fail(CA_ERR_WORKSPACE, "backward workspace of %zu bytes required, %zu given",
                 bwd_capped_bytes(B, H, T, D, kv_sums, cap_less(0)), workspace ? workspace_bytes : 0);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   char* ws = static_cast<char*>(workspace);
-  if (plan.hc == 0) return run_set(io, dtype, ws, plan.passes, true, kv_sums, B, H, T, D, s);
+  if (plan.hc == 0) return run_set(io, dtype, ws, plan.passes, first, kv_sums, B, H, T, D, s);
   const size_t esz = dtype_size(dtype);
   for (int b = 0; b < B; ++b) {
     for (int h0 = 0; h0 < H; h0 += plan.hc) {
@@ -735,7 +736,7 @@ int bwd_common(const ca::BwdIO& io, int dtype, void* workspace, size_t workspace
       sio.log_gain = io.log_gain + h0;
       sio.dlog_gain = io.dlog_gain + h0;
       const int rc = run_set(sio, dtype, ws, nh == plan.hc ? plan.passes : plan.tail_passes,
-                             b == 0, kv_sums, 1, nh, T, D, s);
+                             first && b == 0, kv_sums, 1, nh, T, D, s);
       if (rc) return rc;
     }
   }
@@ -788,19 +789,69 @@ int ca_bwd_f32(const float* q, const float* k, const float* v, const float* log_
 }  // extern "C"
 
 // ---- the operator on [B,H,T,D] tensors of any operand type and head dim -----
-// Head dims without kernels of their own run on zero-padded rows (pads at
-// the start of the workspace, the padded problem's own workspace after them).
+// Head dims without kernels of their own run on zero-padded rows: the pads of a
+// set of slices at the start of the workspace, the padded problem's own
+// workspace after them.  Where the pads of every slice would take more than
+// half of the workspace cap, the slices run as sets one after another (whole
+// batches, or heads of one batch), so that the pads stay within the cap and
+// leave the operator room for passes that fill the device.  (Pads of
+// everything took the cap from the operator: at [16,16,1180,80] fp32 they left
+// it 1 MB, 2560 passes of one head and one query group each.)
 static size_t pad_bytes(int dtype, int B, int H, int T, int DP, int tensors) {
   return tensors * align256((size_t)B * H * T * DP * dtype_size(dtype));
 }
-static size_t fwd_pads(int dtype, int B, int H, int T, int D) {
-  const int DP = ca::padded_head_dim(D);
+static size_t fwd_pads(int dtype, int B, int H, int T, int DP) {
   // q, k, v and, when the caller keeps no y, the padded fp32 output
-  return DP == D ? 0 : pad_bytes(dtype, B, H, T, DP, 3) + pad_bytes(CA_DTYPE_F32, B, H, T, DP, 1);
+  return pad_bytes(dtype, B, H, T, DP, 3) + pad_bytes(CA_DTYPE_F32, B, H, T, DP, 1);
 }
-static size_t bwd_pads(int dtype, int B, int H, int T, int D) {
-  const int DP = ca::padded_head_dim(D);
-  return DP == D ? 0 : pad_bytes(dtype, B, H, T, DP, 7);  // q, k, v, dout; dq, dk, dv
+static size_t bwd_pads(int dtype, int B, int H, int T, int DP) {
+  return pad_bytes(dtype, B, H, T, DP, 7);  // q, k, v, dout; dq, dk, dv
+}
+// nb batches of all H heads, or (nb = 1) nh heads of one batch
+struct PadSet {
+  int nb, nh;
+};
+template <class Pads>
+static PadSet pad_set_for(int B, int H, size_t budget, Pads pads) {
+  if (pads(B, H) <= budget) return PadSet{B, H};
+  auto even = [](int n, int most) { return (n + (n + most - 1) / most - 1) / ((n + most - 1) / most); };
+  const size_t batch = pads(1, H), head = pads(1, 1);
+  if (batch <= budget) return PadSet{even(B, (int)std::min<size_t>(B, budget / batch)), H};
+  return PadSet{1, even(H, (int)std::max<size_t>(1, std::min<size_t>(H, budget / head)))};
+}
+// The sets for the cap, made smaller until need(nb, nh) fits `bytes` (false:
+// not even one head does).
+template <class Pads, class Need>
+static bool pad_set_within(int B, int H, size_t bytes, Pads pads, Need need, PadSet* set) {
+  *set = pad_set_for(B, H, g_workspace_cap ? g_workspace_cap / 2 : SIZE_MAX, pads);
+  while (need(set->nb, set->nh) > bytes) {
+    if (set->nb > 1) set->nb = (set->nb + 1) / 2;
+    else if (set->nh > 1) set->nh = (set->nh + 1) / 2;
+    else return false;
+  }
+  return true;
+}
+// f(b0, h0, nb, nh) for each set, in order, until one fails
+template <class F>
+static int for_pad_sets(int B, int H, const PadSet& set, F f) {
+  for (int b = 0; b < B; b += set.nb)
+    for (int h = 0; h < H; h += set.nh) {
+      const int rc = f(b, h, std::min(set.nb, B - b), std::min(set.nh, H - h));
+      if (rc) return rc;
+    }
+  return CA_OK;
+}
+// workspace of one set's padded problem
+static size_t fwd_core_bytes(int nb, int nh, int T, int DP, size_t cap) {
+  return ca::fwd_part_floats(nb * nh, T, fwd_split(nb * nh, T, DP, true, cap), DP) * sizeof(float);
+}
+static size_t bwd_core_bytes(int dtype, int nb, int nh, int T, int DP, size_t cap) {
+  const size_t full = bwd_full_bytes(nb, nh, T, DP);
+  if (full <= cap) return full;
+  // passes: 16-bit gradients are summed over them in fp32 (as ca_bwd_qkv)
+  const bool sums = dtype != CA_DTYPE_F32;
+  const size_t need = bwd_capped_bytes(nb, nh, T, DP, sums, cap);
+  return sums ? std::min(full, need) : need;
 }
 static int check_op(const char* fn, int dtype, int B, int H, int T, int D) {
   if (dtype != CA_DTYPE_F32 && dtype != CA_DTYPE_BF16 && dtype != CA_DTYPE_F16)
@@ -843,9 +894,11 @@ int ca_padded_head_dim(int D) { return ca::padded_head_dim(D); }
 size_t ca_fwd_op_workspace_bytes(int dtype, int B, int H, int T, int D) {
   const int DP = ca::padded_head_dim(D);
   if (B <= 0 || H <= 0 || T <= 0 || !DP) return 0;
-  const size_t pads = fwd_pads(dtype, B, H, T, D);
-  return pads + ca::fwd_part_floats(B * H, T, fwd_split(B * H, T, DP, true, cap_less(pads)), DP) *
-                    sizeof(float);
+  if (DP == D) return fwd_core_bytes(B, H, T, D, cap_less(0));
+  auto pads = [&](int nb, int nh) { return fwd_pads(dtype, nb, nh, T, DP); };
+  const PadSet set = pad_set_for(B, H, g_workspace_cap ? g_workspace_cap / 2 : SIZE_MAX, pads);
+  const size_t p = pads(set.nb, set.nh);
+  return p + fwd_core_bytes(set.nb, set.nh, T, DP, cap_less(p));
 }
 
 int ca_fwd_op(const void* q, const void* k, const void* v, int dtype, const float* log_gain,
@@ -866,41 +919,45 @@ int ca_fwd_op(const void* q, const void* k, const void* v, int dtype, const floa
                  stats, D};
     return fwd_common(io, dtype, workspace, workspace_bytes, B, H, T, D, stream);
   }
-  const size_t pads = fwd_pads(dtype, B, H, T, D);
-  if (!workspace || workspace_bytes < pads)
+  auto pads = [&](int nb, int nh) { return fwd_pads(dtype, nb, nh, T, DP); };
+  PadSet set;
+  if (!pad_set_within(B, H, workspace ? workspace_bytes : 0, pads, pads, &set))
     return fail(CA_ERR_WORKSPACE, "ca_fwd_op: workspace of %zu bytes required, %zu given",
                 ca_fwd_op_workspace_bytes(dtype, B, H, T, D), workspace ? workspace_bytes : 0);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  char* ws = static_cast<char*>(workspace);
-  const size_t each = pad_bytes(dtype, B, H, T, DP, 1);
-  const long long rows = (long long)B * H * T;
-  const void* src[3] = {q, k, v};
-  hipError_t e = pad_rows(dtype, src, ws, each, 3, rows, D, DP, s);
-  if (e != hipSuccess) return fail(CA_ERR_HIP, "ca_fwd_op: pad launch: %s", hipGetErrorString(e));
-  float* yp = y ? y : reinterpret_cast<float*>(ws + 3 * each);
-  ca::FwdIO io{heads_view(ws, H, T, DP), heads_view(ws + each, H, T, DP),
-               heads_view(ws + 2 * each, H, T, DP), nullptr, false, log_gain, yp,
-               ca::View{nullptr, 0, 0, 0}, stats, D};
-  rc = fwd_common(io, dtype, ws + pads, workspace_bytes - pads, B, H, T, DP, stream);
-  if (rc || !out) return rc;
-  const char* ysrc = reinterpret_cast<const char*>(yp);
-  if (dtype == CA_DTYPE_BF16) e = unpad_rows<float, __bf16>(ysrc, 0, &out, 1, rows, D, DP, s);
-  else if (dtype == CA_DTYPE_F16) e = unpad_rows<float, _Float16>(ysrc, 0, &out, 1, rows, D, DP, s);
-  else e = unpad_rows<float, float>(ysrc, 0, &out, 1, rows, D, DP, s);
-  if (e != hipSuccess) return fail(CA_ERR_HIP, "ca_fwd_op: unpad launch: %s", hipGetErrorString(e));
-  return CA_OK;
+  const size_t esz = dtype_size(dtype);
+  return for_pad_sets(B, H, set, [&](int b0, int h0, int nb, int nh) {
+    char* ws = static_cast<char*>(workspace);
+    const size_t each = pad_bytes(dtype, nb, nh, T, DP, 1), p = pads(nb, nh);
+    const long long row0 = ((long long)b0 * H + h0) * T, rows = (long long)nb * nh * T;
+    auto at = [&](const void* t) { return static_cast<const char*>(t) + row0 * D * esz; };
+    const void* src[3] = {at(q), at(k), at(v)};
+    hipError_t e = pad_rows(dtype, src, ws, each, 3, rows, D, DP, s);
+    if (e != hipSuccess) return fail(CA_ERR_HIP, "ca_fwd_op: pad launch: %s", hipGetErrorString(e));
+    float* yp = y ? y + row0 * DP : reinterpret_cast<float*>(ws + 3 * each);
+    ca::FwdIO io{heads_view(ws, nh, T, DP), heads_view(ws + each, nh, T, DP),
+                 heads_view(ws + 2 * each, nh, T, DP), nullptr, false, log_gain + h0, yp,
+                 ca::View{nullptr, 0, 0, 0}, stats + 2 * row0, D};
+    const int rc = fwd_common(io, dtype, ws + p, workspace_bytes - p, nb, nh, T, DP, stream);
+    if (rc || !out) return rc;
+    void* dst = const_cast<char*>(at(out));
+    const char* ysrc = reinterpret_cast<const char*>(yp);
+    if (dtype == CA_DTYPE_BF16) e = unpad_rows<float, __bf16>(ysrc, 0, &dst, 1, rows, D, DP, s);
+    else if (dtype == CA_DTYPE_F16) e = unpad_rows<float, _Float16>(ysrc, 0, &dst, 1, rows, D, DP, s);
+    else e = unpad_rows<float, float>(ysrc, 0, &dst, 1, rows, D, DP, s);
+    if (e != hipSuccess) return fail(CA_ERR_HIP, "ca_fwd_op: unpad launch: %s", hipGetErrorString(e));
+    return (int)CA_OK;
+  });
 }
 
 size_t ca_bwd_op_workspace_bytes(int dtype, int B, int H, int T, int D) {
   const int DP = ca::padded_head_dim(D);
   if (B <= 0 || H <= 0 || T <= 0 || !DP) return 0;
-  const size_t pads = bwd_pads(dtype, B, H, T, D), cap = cap_less(pads);
-  const size_t full = bwd_full_bytes(B, H, T, DP);
-  if (full <= cap) return pads + full;
-  // passes: 16-bit gradients are summed over them in fp32 (as ca_bwd_qkv)
-  const bool sums = dtype != CA_DTYPE_F32;
-  const size_t need = bwd_capped_bytes(B, H, T, DP, sums, cap);
-  return pads + (sums ? std::min(full, need) : need);
+  if (DP == D) return bwd_core_bytes(dtype, B, H, T, D, cap_less(0));
+  auto pads = [&](int nb, int nh) { return bwd_pads(dtype, nb, nh, T, DP); };
+  const PadSet set = pad_set_for(B, H, g_workspace_cap ? g_workspace_cap / 2 : SIZE_MAX, pads);
+  const size_t p = pads(set.nb, set.nh);
+  return p + bwd_core_bytes(dtype, set.nb, set.nh, T, DP, cap_less(p));
 }
 
 int ca_bwd_op(const void* q, const void* k, const void* v, int dtype, const float* log_gain,
@@ -916,39 +973,52 @@ int ca_bwd_op(const void* q, const void* k, const void* v, int dtype, const floa
     if (!aligned_to(p, a)) return fail(CA_ERR_INVALID, "ca_bwd_op: tensors must be %zu-byte aligned", a);
   if (!aligned16(y)) return fail(CA_ERR_INVALID, "ca_bwd_op: y must be 16-byte aligned");
   const int DP = ca::padded_head_dim(D);
-  const size_t pads = bwd_pads(dtype, B, H, T, D);
-  if (!workspace || workspace_bytes < pads)
+  const size_t bytes = workspace ? workspace_bytes : 0;
+  // the backward of the slices whose tensors (rows of DP columns) are given
+  auto run = [&](const void* const (&in)[4], void* const (&grads)[3], int b0, int h0, int nb, int nh,
+                 char* ws, size_t core) {
+    const long long row0 = ((long long)b0 * H + h0) * T;
+    ca::BwdIO io{heads_view(in[0], nh, T, DP), heads_view(in[1], nh, T, DP),
+                 heads_view(in[2], nh, T, DP), nullptr, false, log_gain + h0, y + row0 * DP,
+                 stats + 2 * row0, heads_view(in[3], nh, T, DP), heads_view(grads[0], nh, T, DP),
+                 heads_view(grads[1], nh, T, DP), heads_view(grads[2], nh, T, DP), dlog_gain + h0};
+    io.head_dim = D;
+    const bool sums = dtype != CA_DTYPE_F32 && core < bwd_full_bytes(nb, nh, T, DP);
+    return bwd_common(io, dtype, ws, core, nb, nh, T, DP, stream, sums, b0 == 0);
+  };
+  if (DP == D)
+    return run({q, k, v, dout}, {dq, dk, dv}, 0, 0, B, H, static_cast<char*>(workspace), bytes);
+  auto pads = [&](int nb, int nh) { return bwd_pads(dtype, nb, nh, T, DP); };
+  auto need = [&](int nb, int nh) {  // what one pass takes if that fits, else the least
+    const size_t p = pads(nb, nh), full = p + bwd_full_bytes(nb, nh, T, DP);
+    return full <= bytes ? full : p + bwd_core_bytes(dtype, nb, nh, T, DP, 1);
+  };
+  PadSet set;
+  if (!pad_set_within(B, H, bytes, pads, need, &set))
     return fail(CA_ERR_WORKSPACE, "ca_bwd_op: workspace of %zu bytes required, %zu given",
-                ca_bwd_op_workspace_bytes(dtype, B, H, T, D), workspace ? workspace_bytes : 0);
+                ca_bwd_op_workspace_bytes(dtype, B, H, T, D), bytes);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  char* ws = static_cast<char*>(workspace);
-  const size_t each = DP == D ? 0 : pad_bytes(dtype, B, H, T, DP, 1);
-  const long long rows = (long long)B * H * T;
-  const void* in[4] = {q, k, v, dout};
-  void* grads[3] = {dq, dk, dv};
-  const void *pin[4], *pgrad[3];
-  hipError_t e;
-  for (int i = 0; i < 4; ++i) pin[i] = DP == D ? in[i] : ws + i * each;
-  for (int i = 0; i < 3; ++i) pgrad[i] = DP == D ? grads[i] : ws + (4 + i) * each;
-  if (DP != D) {
-    e = pad_rows(dtype, in, ws, each, 4, rows, D, DP, s);
+  const size_t esz = dtype_size(dtype);
+  return for_pad_sets(B, H, set, [&](int b0, int h0, int nb, int nh) {
+    char* ws = static_cast<char*>(workspace);
+    const size_t each = pad_bytes(dtype, nb, nh, T, DP, 1), p = pads(nb, nh);
+    const long long off = ((long long)b0 * H + h0) * T * D * (long long)esz, rows = (long long)nb * nh * T;
+    const void* src[4] = {q, k, v, dout};
+    void* dst[3] = {dq, dk, dv};
+    for (const void*& t : src) t = static_cast<const char*>(t) + off;
+    for (void*& t : dst) t = static_cast<char*>(t) + off;
+    hipError_t e = pad_rows(dtype, src, ws, each, 4, rows, D, DP, s);
     if (e != hipSuccess) return fail(CA_ERR_HIP, "ca_bwd_op: pad launch: %s", hipGetErrorString(e));
-  }
-  ca::BwdIO io{heads_view(pin[0], H, T, DP), heads_view(pin[1], H, T, DP),
-               heads_view(pin[2], H, T, DP), nullptr, false, log_gain, y, stats,
-               heads_view(pin[3], H, T, DP), heads_view(pgrad[0], H, T, DP),
-               heads_view(pgrad[1], H, T, DP), heads_view(pgrad[2], H, T, DP), dlog_gain};
-  io.head_dim = D;
-  const size_t core = workspace_bytes - pads;
-  const bool sums = dtype != CA_DTYPE_F32 && core < bwd_full_bytes(B, H, T, DP);
-  rc = bwd_common(io, dtype, ws + pads, core, B, H, T, DP, stream, sums);
-  if (rc || DP == D) return rc;
-  const char* gsrc = ws + 4 * each;
-  if (dtype == CA_DTYPE_BF16) e = unpad_rows<__bf16, __bf16>(gsrc, each, grads, 3, rows, D, DP, s);
-  else if (dtype == CA_DTYPE_F16) e = unpad_rows<_Float16, _Float16>(gsrc, each, grads, 3, rows, D, DP, s);
-  else e = unpad_rows<float, float>(gsrc, each, grads, 3, rows, D, DP, s);
-  if (e != hipSuccess) return fail(CA_ERR_HIP, "ca_bwd_op: unpad launch: %s", hipGetErrorString(e));
-  return CA_OK;
+    char* g = ws + 4 * each;
+    const int rc = run({ws, ws + each, ws + 2 * each, ws + 3 * each}, {g, g + each, g + 2 * each}, b0,
+                       h0, nb, nh, ws + p, bytes - p);
+    if (rc) return rc;
+    if (dtype == CA_DTYPE_BF16) e = unpad_rows<__bf16, __bf16>(g, each, dst, 3, rows, D, DP, s);
+    else if (dtype == CA_DTYPE_F16) e = unpad_rows<_Float16, _Float16>(g, each, dst, 3, rows, D, DP, s);
+    else e = unpad_rows<float, float>(g, each, dst, 3, rows, D, DP, s);
+    if (e != hipSuccess) return fail(CA_ERR_HIP, "ca_bwd_op: unpad launch: %s", hipGetErrorString(e));
+    return (int)CA_OK;
+  });
 }
 
 static int check_qkv(const char* fn, int dtype, const void* qkv, const float* rope_cs,

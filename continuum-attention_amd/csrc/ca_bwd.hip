@@ -622,10 +622,12 @@ __global__ __launch_bounds__(256) void ca_unpad_kernel(UnpadSet<S, E> set, long 
       ++row;
     }
   }
-  if (i0 + 4 <= n)
+  // a set of slices inside a tensor (odd T and D) may start anywhere
+  const bool wide = (reinterpret_cast<uintptr_t>(dst) & (4 * sizeof(E) - 1)) == 0;
+  if (wide && i0 + 4 <= n)
     st4(dst + i0, v);
   else
-    for (int e = 0; i0 + e < n; ++e) st1(dst + i0 + e, v[e]);
+    for (int e = 0; e < 4 && i0 + e < n; ++e) st1(dst + i0 + e, v[e]);
 }
 
 template <class E>

@@ -99,7 +99,9 @@ enum { CA_DTYPE_F32 = 0, CA_DTYPE_BF16 = 1, CA_DTYPE_F16 = 2 };
  * are and write the output and gradients rounded once to that type; scores,
  * weights and sums are fp32.  Head dims other than 8, 16, 32, 64 and 128 run
  * on rows padded with zeros in the workspace to the next of them
- * (ca_padded_head_dim; 0: not supported); scores keep 1/sqrt(D).
+ * (ca_padded_head_dim; 0: not supported), where those rows would take more than
+ * half of the workspace cap as sets of slices one after another; scores keep
+ * 1/sqrt(D).
  * Forward: out [B,H,T,D] (dtype) and the fp32 output y
  * [B,H,T,ca_padded_head_dim(D)] that ca_bwd_op reads.  Either may be NULL: out
  * when y is the result (fp32, unpadded D), y when no backward follows.

@@ -300,3 +300,23 @@ def test_workspace_size_caches_follow_the_cap_and_splits(ca):
     finally:
         ops.set_split_override(0, 0, 0)
         ops.set_workspace_cap(prev)
+
+
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+def test_padded_workspaces_within_the_cap(ca, dtype):
+    """Zero-padded head dims: pads and workspace together stay within the cap, and
+    the pads leave the operator at least half of it or its whole need, at sizes
+    around those where the pads of every slice reach it."""
+    lib = ca.native.load()
+    cap = lib.ca_workspace_cap()
+    for B, H, D, DP in ((16, 16, 80, 128), (64, 16, 72, 128), (3, 64, 40, 64), (1, 128, 24, 32),
+                        (256, 4, 9, 16)):
+        for T in (64, 500, 1024, 1160, 1180, 2048, 4100):
+            if B * H * T * DP >= 1 << 31:
+                continue
+            fwd = lib.ca_fwd_op_workspace_bytes(dtype, B, H, T, D)
+            bwd = lib.ca_bwd_op_workspace_bytes(dtype, B, H, T, D)
+            assert 0 < fwd <= cap and 0 < bwd <= cap, (B, H, T, D, fwd, bwd)
+            pads = 7 * B * H * T * DP * (4 if dtype == 0 else 2)
+            if pads > cap // 2:  # in sets, near the cap and not in slivers
+                assert bwd > cap // 3, (B, H, T, D, bwd)

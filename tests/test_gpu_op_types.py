@@ -118,3 +118,33 @@ def test_wide_head_dims_match_oracle(gpu_ca, D, T):
     assert rel(y.cpu(), O.ca_forward(*n)[0]) <= OUT_TOL
     for a, b in zip(grads, O.ca_backward(*n, dy.numpy())):
         assert rel(a.cpu(), b) <= GRAD_TOL
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(3, 2, 300, 80), (1, 5, 201, 9)])
+def test_padded_head_dims_in_sets(gpu_ca, dtype, shape):
+    """Pads of everything above half of a lowered cap: sets of batches or heads
+    one after another, each in one pass or (the smaller cap) several, and slices
+    that start at odd addresses.  Each set is the operator on its slices, so the
+    results differ by the order of the passes' sums alone."""
+    B, H, T, D = shape
+    q, k, v, rho, dy = make_inputs(shape, 21, 1.0, [0.1 * h for h in range(H)])
+    q, k, v, dy = (x.to(dtype) for x in (q, k, v, dy))
+    y, grads = _typed(gpu_ca, q, k, v, rho, dy)
+    lib = gpu_ca.native.load()
+    code = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}[dtype]
+    full = lib.ca_bwd_op_workspace_bytes(code, B, H, T, D)
+    prev = gpu_ca.ops.workspace_cap()
+    step = 0.0 if dtype == torch.float32 else 2 * HALF_ULP[dtype]
+    for part in (2, 4):
+        say(f"[case] {shape} {dtype} cap 1/{part} of {full}")
+        try:
+            gpu_ca.ops.set_workspace_cap(full // part)
+            assert lib.ca_bwd_op_workspace_bytes(code, B, H, T, D) <= full // part
+            y2, grads2 = _typed(gpu_ca, q, k, v, rho, dy)
+        finally:
+            gpu_ca.ops.set_workspace_cap(prev)
+        for a, b in zip((y, *grads[:3]), (y2, *grads2[:3])):
+            a, b = a.float(), b.float()
+            assert bool(((a - b).abs() <= step * b.abs() + 5e-6 * b.abs().max()).all())
+        assert rel(grads2[3].cpu(), grads[3].cpu()) < 1e-5
