@@ -150,6 +150,7 @@ def torch_ext():
         spec = importlib.util.spec_from_file_location("_ca_torch", TORCH_EXT_PATH)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
+        module.set_error(CAError)
         _ext = module
     return _ext
 

@@ -23,6 +23,7 @@
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
@@ -34,11 +35,19 @@ using at::Tensor;
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
 
+PyObject* ca_error = nullptr;  // _native.CAError (set at load, kept for good)
+
+// The errors of _native.check, from any thread.
 void check(int rc) {
   if (rc == CA_OK) return;
   const std::string msg = std::string("continuum-attention_amd: ") + ca_last_error();
   if (rc == CA_ERR_INVALID || rc == CA_ERR_UNSUPPORTED) TORCH_CHECK_VALUE(false, msg);
-  TORCH_CHECK(false, msg);
+  py::gil_scoped_acquire gil;
+  const py::object error = py::reinterpret_borrow<py::object>(ca_error)(rc, msg);
+  PyErr_SetObject(ca_error, error.ptr());
+  python_error e;  // autograd carries it from its threads to the caller
+  e.persist();
+  throw std::move(e);
 }
 
 int dtype_code(at::ScalarType t) {
@@ -407,6 +416,8 @@ py::object weights(py::handle so) {
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("set_error", [](py::object cls) { ca_error = cls.release().ptr(); });
+  m.def("check", &check, py::call_guard<py::gil_scoped_release>());
   m.def("op", &op);
   m.def("rope_attention", &rope_attention);
   m.def("rmsnorm", &rmsnorm);

@@ -320,3 +320,17 @@ def test_padded_workspaces_within_the_cap(ca, dtype):
             pads = 7 * B * H * T * DP * (4 if dtype == 0 else 2)
             if pads > cap // 2:  # in sets, near the cap and not in slivers
                 assert bwd > cap // 3, (B, H, T, D, bwd)
+
+
+def test_native_functions_raise_the_librarys_errors(ca):
+    """A failed call inside the native autograd functions raises what the Python
+    ones raise (_native.check)."""
+    ext, native = ca.native.torch_ext(), ca.native
+    assert ext.check(native.CA_OK) is None
+    for rc in (native.CA_ERR_INVALID, native.CA_ERR_UNSUPPORTED):
+        with pytest.raises(ValueError):
+            ext.check(rc)
+    for rc in (native.CA_ERR_HIP, native.CA_ERR_WORKSPACE):
+        with pytest.raises(native.CAError) as e:
+            ext.check(rc)
+        assert e.value.code == rc and "continuum-attention_amd: " in str(e.value)
