@@ -101,6 +101,13 @@ Tensor workspace(size_t bytes, const Tensor& like) {
 void first_order_only(const char* what) {
   TORCH_CHECK(!at::GradMode::is_enabled(), what);
 }
+// Saved tensors come back from saved-tensor hooks, from wherever those put them.
+void on_one_gpu(const char* what, std::initializer_list<const Tensor*> ts) {
+  const c10::Device device = (*ts.begin())->device();
+  for (const Tensor* t : ts)
+    TORCH_CHECK(t->is_cuda() && t->device() == device, what,
+                ": all tensors must be on the same GPU");
+}
 constexpr const char* kOpFirstOrder = "CA Volta analytic kernel supports first-order gradients only";
 
 // ---- the operator --------------------------------------------------------------
@@ -141,8 +148,7 @@ struct OpFunction : torch::autograd::Function<OpFunction> {
     const Tensor q = operand(saved[0], dt), k = operand(saved[1], dt), v = operand(saved[2], dt);
     const Tensor gain = operand(saved[3], at::kFloat), y = operand(saved[4], at::kFloat),
                  stats = operand(saved[5], at::kFloat), dy = operand(grads[0], dt);
-    for (const Tensor* t : {&k, &v, &gain, &y, &stats, &dy})
-      TORCH_CHECK(t->device() == q.device(), "continuum_attention: all tensors must be on the same device");
+    on_one_gpu("continuum_attention", {&q, &k, &v, &gain, &y, &stats, &dy});
     const c10::DeviceGuard guard(q.device());
     const int B = q.size(0), H = q.size(1), T = q.size(2), D = q.size(3);
     const int code = dtype_code(dt);
@@ -213,8 +219,7 @@ struct RopeFunction : torch::autograd::Function<RopeFunction> {
     const Tensor qkv = operand(saved[0], dt), gain = operand(saved[1], at::kFloat),
                  y = operand(saved[2], at::kFloat), stats = operand(saved[3], at::kFloat),
                  dy = operand(grads[0], dt);
-    for (const Tensor* t : {&gain, &y, &stats, &dy})
-      TORCH_CHECK(t->device() == qkv.device(), "continuum attention: all tensors must be on the same device");
+    on_one_gpu("continuum attention", {&qkv, &gain, &y, &stats, &dy});
     const c10::DeviceGuard guard(qkv.device());
     const int H = ctx->saved_data["heads"].toInt();
     const int B = qkv.size(0), T = qkv.size(1), D = qkv.size(2) / 3 / H;
@@ -283,6 +288,7 @@ struct NormFunction : torch::autograd::Function<NormFunction> {
     const variable_list saved = ctx->get_saved_variables();
     const Tensor x = operand(saved[0], at::kFloat), w = operand(saved[1], at::kFloat),
                  rstd = operand(saved[2], at::kFloat), g = norm_operand(grads[0]);
+    on_one_gpu("RMSNorm", {&x, &w, &rstd, &g});
     const c10::DeviceGuard guard(x.device());
     const int C = x.size(-1), N = x.numel() / C;
     Tensor dx = empty(x.sizes(), x, at::kFloat), dw = empty(w.sizes(), x, at::kFloat);
@@ -324,6 +330,7 @@ struct AddNormFunction : torch::autograd::Function<AddNormFunction> {
     const Tensor g = grads[1].defined() ? norm_operand(grads[1]) : at::zeros_like(s);
     Tensor gs;
     if (grads[0].defined()) gs = operand(grads[0], at::kFloat);
+    on_one_gpu("add + RMSNorm", {&s, &w, &rstd, &g, gs.defined() ? &gs : &g});
     Tensor dx = empty(s.sizes(), s, at::kFloat), dres = empty(s.sizes(), s, rd);
     Tensor dw = empty(w.sizes(), s, at::kFloat);
     const size_t bytes = ca_rmsnorm_bwd_workspace_bytes(N, C);
@@ -390,6 +397,8 @@ struct WeightsFunction : torch::autograd::Function<WeightsFunction> {
     first_order_only("continuous_attention_weights on the GPU supports first-order gradients only");
     const Tensor s = operand(ctx->get_saved_variables()[0], at::kFloat),
                  g = operand(grads[0], at::kFloat);
+    on_one_gpu("continuous_attention_weights", {&s, &g});
+    TORCH_CHECK_VALUE(g.sizes() == s.sizes(), "grad_weights shape ", g.sizes(), " != scores shape ", s.sizes());
     const c10::DeviceGuard guard(s.device());
     const int T = s.size(-1), N = s.numel() / ((int64_t)T * T);
     Tensor ds = empty(s.sizes(), s, at::kFloat);

@@ -26,7 +26,7 @@ from torch import nn
 from torch.nn import functional as F
 
 from . import _native
-from .ops import (SUPPORTED_HEAD_DIMS, _UNLIMITED_MODES, _bwd_qkv_workspace_bytes,
+from .ops import (SUPPORTED_HEAD_DIMS, _UNLIMITED_MODES, _bwd_qkv_workspace_bytes, _check_device,
                   _fwd_qkv_workspace_bytes, _mode, check_mode_limits, continuum_attention)
 
 _DTYPE_CODE = {torch.float32: _native.CA_DTYPE_F32, torch.bfloat16: _native.CA_DTYPE_BF16,
@@ -87,6 +87,7 @@ class _RMSNormFn(torch.autograd.Function):
         if torch.is_grad_enabled():
             raise RuntimeError("the fused RMSNorm supports first-order gradients only")
         xc, w, rstd = ctx.saved_tensors
+        _check_device(xc, w, rstd, gy)  # saved-tensor hooks may have moved them
         lib = _native.load()
         C = xc.shape[-1]
         N = xc.numel() // C
@@ -141,6 +142,7 @@ class _AddRMSNormFn(torch.autograd.Function):
         if torch.is_grad_enabled():
             raise RuntimeError("the fused add + RMSNorm supports first-order gradients only")
         s, w, rstd = ctx.saved_tensors
+        _check_device(s, w, rstd, *(t for t in (gs, gy) if t is not None))
         lib = _native.load()
         C = s.shape[-1]
         N = s.numel() // C
@@ -399,6 +401,7 @@ class _RopeContinuumAttention(torch.autograd.Function):
         if torch.is_grad_enabled():
             raise RuntimeError("CA Volta analytic kernel supports first-order gradients only")
         x, gain, y, stats = ctx.saved_tensors
+        _check_device(x, gain, y, stats, gout)
         cs = ctx.cs
         Bsz, T, heads, D = ctx.shape
         lib = _native.load()

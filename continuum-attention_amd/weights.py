@@ -82,6 +82,8 @@ def ca_weights_backward(scores: torch.Tensor, grad_weights: torch.Tensor, start:
     if start < 0 or start + Q > K:
         raise ValueError(f"ca_weights_backward: queries {start}..{start + Q - 1} need K >= {start + Q}, "
                          f"got K={K}")
+    if grad_weights.device != scores.device:
+        raise RuntimeError("ca_weights_backward: all tensors must be on the same device")
     lib = _native.load()
     s = _f32c(scores)
     gw = _f32c(grad_weights)

@@ -173,3 +173,25 @@ def test_threads_and_streams(gpu_ca):
         t.join()
     for a, b in zip(alone, got):
         assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("name", ["op_f32", "op_f16_padded", "rope_bf16", "norm_f32",
+                                  "norm_bf16_unused_sum", "weights"])
+def test_saved_tensors_left_on_the_cpu_are_refused(gpu_ca, name, native, monkeypatch):
+    """Saved-tensor hooks that do not bring the tensors back: an error, no kernel."""
+    run = CASES[name](gpu_ca)
+    if not native:
+        monkeypatch.setattr(gpu_ca.native, "torch_ext", _NoneExt)
+    for moved in (lambda n: True, lambda n: n == 1):  # every tensor, then the second alone
+        count = []
+
+        def unpack(t, moved=moved, count=count):
+            count.append(1)
+            return t.cpu() if moved(len(count) - 1) else t
+
+        if name == "weights" and not moved(0):
+            continue  # one saved tensor
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            with pytest.raises(RuntimeError, match="same|ROCm GPU|CUDA"):
+                run()
