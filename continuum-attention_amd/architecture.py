@@ -205,7 +205,7 @@ class _SwiGLUFn(torch.autograd.Function):
         lib = _native.load()
         H = uc.shape[-1] // 2
         N = uc.numel() // (2 * H)
-        g = dh.float().contiguous()
+        g = dh.float().resolve_neg().contiguous()
         if g.data_ptr() % 16:
             g = g.clone()
         du = torch.empty_like(uc)

@@ -83,9 +83,10 @@ bool grads_needed(std::initializer_list<const Tensor*> ts) {
   return false;
 }
 
-// A tensor as the kernels read it (a saved or incoming one may be a view).
+// A tensor as the kernels read it (a saved or incoming one may be a view, of
+// negated values too).
 Tensor operand(Tensor t, at::ScalarType dtype) {
-  t = t.detach();
+  t = t.detach().resolve_neg();
   if (t.scalar_type() != dtype) t = t.to(dtype);
   t = t.contiguous();
   return aligned(t) ? t : t.clone();

@@ -71,7 +71,7 @@ class _RMSNormFn(torch.autograd.Function):
         C = x.shape[-1]
         N = x.numel() // C
         xc = _aligned(x.detach(), 16)
-        w = weight.detach().contiguous()
+        w = _aligned(weight.detach(), 4)
         y = torch.empty(x.shape, device=x.device, dtype=out_dtype)
         rstd = torch.empty(N, device=x.device, dtype=torch.float32)
         stream = _native.stream_handle(x.device)
@@ -91,7 +91,7 @@ class _RMSNormFn(torch.autograd.Function):
         lib = _native.load()
         C = xc.shape[-1]
         N = xc.numel() // C
-        g = gy.contiguous()
+        g = _aligned(gy, 4)
         if g.dtype not in _DTYPE_CODE:
             g = g.float()
         dx = torch.empty_like(xc)
@@ -122,7 +122,7 @@ class _AddRMSNormFn(torch.autograd.Function):
         N = x.numel() // C
         xc = _aligned(x.detach(), 16)
         rc = _aligned(res.detach(), 16)
-        w = weight.detach().contiguous()
+        w = _aligned(weight.detach(), 4)
         s = torch.empty(x.shape, device=x.device, dtype=torch.float32)
         y = torch.empty(x.shape, device=x.device, dtype=out_dtype)
         rstd = torch.empty(N, device=x.device, dtype=torch.float32)
@@ -146,10 +146,10 @@ class _AddRMSNormFn(torch.autograd.Function):
         lib = _native.load()
         C = s.shape[-1]
         N = s.numel() // C
-        g = torch.zeros_like(s) if gy is None else gy.contiguous()
+        g = torch.zeros_like(s) if gy is None else _aligned(gy, 4)
         if g.dtype not in _DTYPE_CODE:
             g = g.float()
-        gsum = None if gs is None else gs.float().contiguous()
+        gsum = None if gs is None else _aligned(gs.float(), 4)
         dx = torch.empty_like(s)
         dres = torch.empty(s.shape, device=s.device, dtype=ctx.res_dtype)
         dw = torch.empty_like(w)
@@ -343,7 +343,7 @@ def rope_cos_sin(T, D, theta, device, dtype=torch.float32):
 
 
 def _aligned(x, nbytes):
-    x = x.contiguous()
+    x = x.resolve_neg().contiguous()
     return x if x.data_ptr() % nbytes == 0 else x.clone()
 
 
@@ -379,7 +379,7 @@ class _RopeContinuumAttention(torch.autograd.Function):
         dev, dt = qkv.device, _DTYPE_CODE[qkv.dtype]
         x = _aligned(qkv.detach(), 16)
         cs = rope_cos_sin(T, D, theta, dev, qkv.dtype) if theta is not None else None
-        gain = log_gain.detach().float().contiguous()
+        gain = _aligned(log_gain.detach().float(), 4)
         y = torch.empty(Bsz, heads, T, D, device=dev, dtype=torch.float32)
         out = torch.empty(Bsz, T, C, device=dev, dtype=qkv.dtype)
         stats = torch.empty(Bsz * heads * T, 2, device=dev, dtype=torch.float32)

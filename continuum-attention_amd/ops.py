@@ -67,7 +67,7 @@ def check_mode_limits(mode: str, is_cuda: bool, q_dtype: torch.dtype, v_dtype: t
 
 
 def _as_f32(x: torch.Tensor) -> torch.Tensor:
-    x = x.detach()
+    x = x.detach().resolve_neg()  # a view of negated values holds them unnegated
     if x.dtype != torch.float32:
         x = x.float()
     x = x.contiguous()
@@ -223,7 +223,7 @@ def _fused(q, k, v) -> bool:
 
 
 def _operand(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
-    x = x.detach()
+    x = x.detach().resolve_neg()
     if x.dtype != dtype:
         x = x.to(dtype)
     x = x.contiguous()

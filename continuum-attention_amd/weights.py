@@ -28,7 +28,7 @@ from . import cpu as _cpu
 
 
 def _f32c(x: torch.Tensor) -> torch.Tensor:
-    x = x.detach()
+    x = x.detach().resolve_neg()
     if x.dtype != torch.float32:
         x = x.float()
     return x.contiguous()

@@ -195,3 +195,39 @@ def test_saved_tensors_left_on_the_cpu_are_refused(gpu_ca, name, native, monkeyp
         with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
             with pytest.raises(RuntimeError, match="same|ROCm GPU|CUDA"):
                 run()
+
+
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_views_of_negated_values(gpu_ca, dtype, native, monkeypatch):
+    """Tensors and gradients with the negative bit set (torch.conj and imag make
+    them) are read as their values."""
+    if not native:
+        monkeypatch.setattr(gpu_ca.native, "torch_ext", _NoneExt)
+    g = torch.Generator().manual_seed(4)
+    q, k, v, dy = (torch.randn(1, 2, 70, 40, generator=g).to(dtype).cuda() for _ in range(4))
+    gain = torch.zeros(2, device="cuda")
+    norm = gpu_ca.decoder.RMSNorm(40).cuda()
+    x, s = q[0].float(), torch.randn(2, 70, 70, generator=g).cuda()
+    flip = torch._neg_view
+
+    def run(neg):
+        def arg(t):
+            return (flip(-t) if neg else t.clone()).requires_grad_()
+
+        out = []
+        for f, args, grad in (
+                (lambda *a: gpu_ca.continuum_attention(*a, gain), (q, k, v), dy),
+                (lambda a: gpu_ca.decoder.rope_continuum_attention(a, gain, 1e4, 2),
+                 (torch.cat([q[0, :, :, :32].reshape(1, 70, 64)] * 3, -1),),
+                 dy[0, :, :, :32].reshape(1, 70, 64)),
+                (norm, (x,), dy[0].float()),
+                (lambda a, b: norm.add_and_norm(a, b)[1], (x, q[0]), dy[0].float()),
+                (gpu_ca.continuous_attention_weights, (s,), s.flip(0))):
+            leaves = [arg(t) for t in args]
+            y = f(*leaves)
+            out += [y.detach(), *torch.autograd.grad(y, leaves, flip(-grad) if neg else grad)]
+        return out
+
+    for a, b in zip(run(True), run(False)):
+        assert torch.equal(a, b)
