@@ -41,7 +41,7 @@ from torch.nn import functional as F
 from . import _native
 from .decoder import RMSNorm as _DecoderRMSNorm
 from .decoder import token_embedding as _token_embedding
-from .decoder import rope_continuum_attention
+from .decoder import _GAIN_CACHE, _kept_table, rope_continuum_attention
 from .ops import SUPPORTED_HEAD_DIMS, continuum_attention
 from .cpu import _C_J0, _C_RIGHT, _SERIES_BELOW, _series
 from .weights import continuous_attention_weights
@@ -155,12 +155,8 @@ class CausalAttention(nn.Module):
             return self.log_qk_gain
         g = math.log(1.0 / self.fixed_tau) if self.variant in ("B", "P") else 0.0
         # a constant: kept per (device, value), not rebuilt every step
-        cache = self.__dict__.setdefault("_gain_cache", {})
-        key = (device, self.heads, g)
-        t = cache.get(key)
-        if t is None:
-            t = cache[key] = torch.full((self.heads,), g, device=device, dtype=torch.float32)
-        return t
+        return _kept_table(_GAIN_CACHE, (device, self.heads, g), device, lambda: (
+            torch.full((self.heads,), g, device=device, dtype=torch.float32),))[0]
 
     def forward(self, x):
         Bsz, T, _ = x.shape

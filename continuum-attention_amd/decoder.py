@@ -216,7 +216,7 @@ class RMSNorm(nn.Module):
         return s, self(s)
 
 
-# ---- RoPE tables, kept per shape ---------------------------------------------
+# ---- RoPE tables, kept per shape, and other constants --------------------------
 #
 # A table is built by kernels queued on the stream current at its first use and
 # then read from whichever stream asks next, so every other stream waits for the
@@ -277,7 +277,7 @@ def _kept_table(cache, key, device, build):
 def _mark_written_tables():
     """Before a capture, with the device idle: every table kept so far can be
     used in it."""
-    for cache in (_ROPE_CACHE, _CS_CACHE):
+    for cache in (_ROPE_CACHE, _CS_CACHE, _GAIN_CACHE):
         for entry in list(cache.values()):
             if isinstance(entry, _Table) and not entry.written:
                 entry.written = entry.event.query()
@@ -292,6 +292,7 @@ def _drop_oldest(cache):
 
 
 _ROPE_CACHE: dict = {}
+_GAIN_CACHE: dict = {}  # constant log-gains (architecture.py)
 
 
 def _rope_tables(T, D, theta, device, dtype):

@@ -151,3 +151,17 @@ def test_graph_replays_with_a_kept_table(gpu_ca, warm):
         torch.cuda.synchronize()
         assert torch.equal(out, call())
         del junk
+
+
+def test_constant_gains_are_kept_the_same_way(ca, monkeypatch):
+    """TinyLM's constant log-gain: one tensor per (device, value) through
+    _kept_table, none on the module (which stays copyable)."""
+    import copy
+    A = ca.architecture
+    seen = []
+    monkeypatch.setattr(A, "_kept_table", lambda *a: seen.append(a[0]) or ca.decoder._kept_table(*a))
+    attn = types.SimpleNamespace(variant="B", fixed_tau=0.5, heads=3)
+    gain = A.CausalAttention._log_gain(attn, torch.device("cpu"))
+    assert seen[0] is ca.decoder._GAIN_CACHE and gain.shape == (3,)
+    assert A.CausalAttention._log_gain(attn, torch.device("cpu")) is gain
+    assert set(vars(copy.deepcopy(attn))) == {"variant", "fixed_tau", "heads"}
