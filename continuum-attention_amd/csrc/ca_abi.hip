@@ -80,58 +80,105 @@ int device_cus() {
 // another launch's tail, reads back.  The length is picked by estimated time:
 // the items are dealt out in dispatch order, each to the slot that is free
 // first, and
-//   time = step_us (ideal + kTail (last slot's end - ideal)) + partials + launch
-// with ideal the slots' mean load.  kTail < 1: near the end fewer work groups
-// share a CU and each runs faster.  Against sweeps of every length on the
-// device the estimate picks the measured best or a length within 2% of it.
-// Before (thresholds on the number of items) / now, time per fwd+bwd:
-//   [1,16,2048,64] bf16 layer 239 / 228 us
-//   [4,16,1001,64] bf16 228 / 214 us   [2,16,2048,64] bf16 407 / 395 us
-//   [8,16,2048,64] bf16 1605 / 1500 us [1,16,8192,64] fp32 3730 / 3635 us
+//   time = step_us (ideal + tail (last slot's end - ideal)) + partials + launch
+// with ideal the slots' mean load.  tail < 1: near the end fewer work groups
+// share a CU and each runs faster.
+// engines > 1: where one work group fills a CU (the forward at D = 128), which
+// slot is free matters.  Work groups go to the eight XCDs in turn, and in each
+// to its shader engines in turn and in order: one whose engine is full holds up
+// those behind it.  The times show it (us, against the steps that dealing to
+// engines and dealing to any free slot predict, [1,16,2048,128] fp32):
+//   tiles      12      16      20      24      32      48    whole
+//   time      143     168     141     160     203     153     191
+//   engines    40      51      42      50      66      49      65
+//   any slot   40      47      42      50      38      49      65
+// The forward's constants (in steps) are fitted to its times at every length, at
+// 24 shapes [1..16, 2..24, 400..8192] of each head dim in fp32, bf16 and fp16:
+// the picked length takes on average 3.3% (D <= 32), 0.9% (64) and 1.2% (128) more
+// time than the best one, at most 20%, 8% and 16%.  One set of constants for
+// all head dims (tail 0.6, one step of overhead) was 5%, 2.6% and 3.6% off on
+// average and up to 29%, 24% and 45%: [1,16,2048,128] fp32 203 us against 141,
+// [2,16,2048,8] 119 against 93, [2,8,768,64] 31.6 against 25.2.  The length must
+// not depend on the operand type: the types' outputs are compared bit for bit.
+// Against thresholds on the number of items, before the estimates, fwd+bwd:
+//   [4,16,1001,64] bf16 228 / 214 us   [8,16,2048,64] bf16 1605 / 1500 us
 //   [1,8,1537,128] fp32 209 / 180 us   [2,8,768,80] fp32 164 / 144 us
-//   [2,16,2048,64] fp32 510-516 / 512-517 us, [4,16,512,64] fp32 116 / 118 us
-// The forward's length must not depend on the operand type: the types'
-// outputs are compared bit for bit.
 struct SplitModel {
   int resident;      // work groups the device holds at once
   int overhead;      // an item's prologue and epilogue, in steps
+  double tail;       // see above
   double step_us;    // one step of one item with the device full
   double part_us;    // device time per partial item, written and read back
   double launch_us;  // extra launch when anything is split
+  int engines = 1;   // shader engines per XCD that work groups are dealt to in order
 };
-constexpr double kTail = 0.6;
-// From this many rounds of whole groups on the tail is under 2% of the time
-// and nothing is cut; it also bounds the host's work per estimate.
+constexpr int kXcds = 8;
+// From this many rounds of whole groups on nothing is cut: the tail is under 2%
+// of the time (the forward's longest groups come first: from 4 rounds on whole
+// groups measured best); it also bounds the host's work per estimate.
 constexpr int kSplitRounds = 64;
-inline bool many_rounds(const SplitModel& m, int groups, int BH) {
-  return (long long)groups * BH >= (long long)kSplitRounds * m.resident;
+constexpr int kFwdSplitRounds = 8;
+inline bool many_rounds(const SplitModel& m, int groups, int BH, int rounds = kSplitRounds) {
+  return (long long)groups * BH >= (long long)rounds * m.resident;
 }
+
+// Work-group slots and when each comes free, in steps.
+struct Slots {
+  std::vector<int> free_at = std::vector<int>(64, 0);  // slots that become free at each step
+  size_t lo = 0;
+  explicit Slots(int n) { free_at[0] = n; }
+  size_t first_free() {
+    while (free_at[lo] == 0) ++lo;
+    return lo;
+  }
+  // n of the slots first_free() counts run until `end`
+  void take(int n, size_t end) {
+    free_at[lo] -= n;
+    if (end >= free_at.size()) free_at.resize(2 * end, 0);
+    free_at[end] += n;
+  }
+};
 
 // items(f) calls f(length) for each item of a slice in dispatch order; every
 // item is launched for all BH slices.
 template <class Items>
 double split_cost(const SplitModel& m, int BH, int part_items, Items items) {
-  std::vector<int> free_at(64, 0);  // slots that become free at each step
-  free_at[0] = m.resident;
-  size_t lo = 0;
-  int last = 0;
+  size_t last = 0;
   double total = 0;
-  items([&](int len) {
-    const int t = len + m.overhead;
-    total += (double)t * BH;
-    for (int need = BH; need > 0;) {
-      while (free_at[lo] == 0) ++lo;
-      const int n = std::min(need, free_at[lo]);
-      free_at[lo] -= n;
-      const size_t end = lo + t;
-      if (end >= free_at.size()) free_at.resize(2 * end, 0);
-      free_at[end] += n;
-      last = std::max(last, (int)end);
-      need -= n;
-    }
-  });
-  const double ideal = total / m.resident;
-  return m.step_us * (ideal + kTail * std::max(0.0, last - ideal)) +
+  if (m.engines > 1) {  // one XCD's share of the work groups, in order
+    const int each = std::max(1, m.resident / (kXcds * m.engines));
+    std::vector<Slots> engine(m.engines, Slots(each));
+    size_t now = 0;
+    long long n = 0, dealt = 0;
+    items([&](int len) {
+      const int t = len + m.overhead;
+      const long long share = (n + BH + kXcds - 1) / kXcds - (n + kXcds - 1) / kXcds;
+      n += BH;
+      total += (double)t * share;
+      for (long long i = 0; i < share; ++i) {
+        Slots& e = engine[dealt++ % m.engines];
+        now = std::max(now, e.first_free());
+        e.take(1, now + t);
+        last = std::max(last, now + t);
+      }
+    });
+    total /= (double)each * m.engines;
+  } else {
+    Slots slots(m.resident);
+    items([&](int len) {
+      const int t = len + m.overhead;
+      total += (double)t * BH;
+      for (int need = BH; need > 0;) {
+        const size_t at = slots.first_free(), end = at + t;
+        const int n = std::min(need, slots.free_at[at]);
+        slots.take(n, end);
+        last = std::max(last, end);
+        need -= n;
+      }
+    });
+    total /= m.resident;
+  }
+  return m.step_us * (total + m.tail * std::max(0.0, last - total)) +
          (part_items ? m.part_us * part_items * BH + m.launch_us : 0.0);
 }
 
@@ -187,9 +234,10 @@ int fwd_split(int BH, int T, int D, bool for_sizing, size_t bytes = SIZE_MAX) {
   if (for_sizing || C >= max_tiles) return C;
   const int cus = device_cus();
   if (!cus) return C;
-  // D <= 64: two work groups per CU
-  const SplitModel m{D > 64 ? cus : 2 * cus, 1, D > 64 ? 4.1 : 2.0 + 2.3 * D / 64, 0.017 * D / 64, 4.0};
-  if (many_rounds(m, G, BH)) return max_tiles;
+  const SplitModel m = D > 64   ? SplitModel{cus, 0, 0.7, 1.0, 0.012, 1.0, 4}
+                       : D > 32 ? SplitModel{2 * cus, 3, 0.176, 1.0, 0.00042, 1.46}
+                                : SplitModel{4 * cus, 0, 0.5, 1.0, 0.001, 0.0};
+  if (many_rounds(m, G, BH, kFwdSplitRounds)) return max_tiles;
   return cached_split(SplitKey{0, BH, T, D, 0, 0, m.resident, C}, [&] {
     int best = max_tiles;
     double cost = 1e30;
@@ -219,7 +267,7 @@ ca::DqSplit dq_split_for(int BH, int T, int D, const ca::BwdPass& p, bool for_si
   if (!cus) return sized;
   const int whole = ca::num_q_tiles(T);
   // three work groups per CU, two at D = 128
-  const SplitModel m{D > 64 ? 2 * cus : 3 * cus, 1, 3.2 * std::max(D, 32) / 64, 0.016 * D / 64, 4.5};
+  const SplitModel m{D > 64 ? 2 * cus : 3 * cus, 1, 0.6, 3.2 * std::max(D, 32) / 64, 0.016 * D / 64, 4.5};
   if (many_rounds(m, p.g1 - p.g0, BH)) return ca::dq_split_chunk(T, p, whole);
   const int chunk = cached_split(SplitKey{1, BH, T, D, p.g0, p.g1, m.resident, sized.part_items}, [&] {
     int best = whole;
@@ -252,7 +300,7 @@ ca::DkdvSplit dkdv_split_for(int BH, int D, int dtype, const ca::BwdPass& p, boo
   const bool bf16 = dtype == CA_DTYPE_BF16;
   const int whole = p.qb - p.qa;
   // work groups per CU: dkdv_waves_per_simd (four waves each)
-  const SplitModel m{cus * (D > 64 ? 2 : bf16 ? 4 : 3), 2, D > 64 ? 6.9 : 1.9 + 2.9 * D / 64,
+  const SplitModel m{cus * (D > 64 ? 2 : bf16 ? 4 : 3), 2, 0.6, D > 64 ? 6.9 : 1.9 + 2.9 * D / 64,
                      0.02 * D / 64, 0.0};
   if (many_rounds(m, p.kv_groups, BH)) return ca::dkdv_split_chunk(p, whole);
   const int chunk = cached_split(SplitKey{2 + bf16, BH, p.kv_groups, D, p.qa, p.qb, m.resident,
