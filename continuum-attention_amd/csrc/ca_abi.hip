@@ -297,13 +297,14 @@ ca::DkdvSplit dkdv_split_for(int BH, int D, int dtype, const ca::BwdPass& p, boo
   const ca::DkdvSplit sized = ca::dkdv_split(BH, p, kDqSplitBound);
   const int cus = for_sizing ? 0 : device_cus();
   if (!cus) return sized;
-  const bool bf16 = dtype == CA_DTYPE_BF16;
   const int whole = p.qb - p.qa;
-  // work groups per CU: dkdv_waves_per_simd (four waves each)
-  const SplitModel m{cus * (D > 64 ? 2 : bf16 ? 4 : 3), 2, 0.6, D > 64 ? 6.9 : 1.9 + 2.9 * D / 64,
-                     0.02 * D / 64, 0.0};
+  // work groups of four waves: as many per CU as waves per SIMD
+  const int planes = dtype == CA_DTYPE_BF16 ? ca::q_limb_planes<__bf16>()
+                     : dtype == CA_DTYPE_F16 ? ca::q_limb_planes<_Float16>() : ca::q_limb_planes<float>();
+  const SplitModel m{cus * ca::dkdv_waves_per_simd(D, planes), 2, 0.6,
+                     D > 64 ? 6.9 : 1.9 + 2.9 * D / 64, 0.02 * D / 64, 0.0};
   if (many_rounds(m, p.kv_groups, BH)) return ca::dkdv_split_chunk(p, whole);
-  const int chunk = cached_split(SplitKey{2 + bf16, BH, p.kv_groups, D, p.qa, p.qb, m.resident,
+  const int chunk = cached_split(SplitKey{2, BH, p.kv_groups, D, p.qa, p.qb, m.resident,
                                           sized.part_items}, [&] {
     int best = whole;
     double cost = 1e30;

@@ -32,12 +32,12 @@ struct Bwd {
   static constexpr int CPT = (CHUNKS + 255) / 256;
 };
 
-// Waves per SIMD the register budget is set for, and whether the query tile
-// is single-buffered (SB): one staged tile and no register prefetch across
-// the tile's work.  SB issues the next tile's loads when its own products are
-// issued, waits at the barrier for the other waves, then stores: the load
-// latency overlaps the barrier wait and the other resident work groups' work,
-// and the registers and LDS it saves hold another wave per SIMD.
+// Whether the query tile is single-buffered (SB; D >= 32): one staged tile and
+// no register prefetch across the tile's work.  SB issues the next tile's loads
+// when its own products are issued, waits at the barrier for the other waves,
+// then stores: the load latency overlaps the barrier wait and the other resident
+// work groups' work, and the registers and LDS it saves hold another wave per
+// SIMD (dkdv_waves_per_simd).
 //   D = 128: SB, two waves (254 VGPRs, 56 KB; double-buffered 307 and 111 KB
 //     held one): [2,16,2048,128] fp32 757 -> 521 us, [1,8,1537,128] 146 -> 113.
 //   D = 32 and 64, fp32 and fp16: SB, three waves (168 VGPRs, 31 KB at 64)
@@ -50,16 +50,7 @@ struct Bwd {
 constexpr bool kDkdvDescending = true;
 
 template <int D, class E, bool SB>
-constexpr int dkdv_waves_per_simd() {
-  return D > 64 ? 2 : q_limb_planes<E>() == 1 ? 4 : SB ? 3 : 2;
-}
-template <int D, class E>
-constexpr bool dkdv_has_single_buffer() {
-  return D >= 32;
-}
-
-template <int D, class E, bool SB>
-__global__ __launch_bounds__(256, (dkdv_waves_per_simd<D, E, SB>())) void ca_bwd_dkdv_kernel(
+__global__ __launch_bounds__(256, dkdv_waves_per_simd(D, q_limb_planes<E>())) void ca_bwd_dkdv_kernel(
     View Kv, View Vv, const float* __restrict__ rope, const float* __restrict__ rope_k,
     const __bf16* __restrict__ limbs,
     const float* __restrict__ qstat, const float* __restrict__ log_gain, View dKv, View dVv,
@@ -514,7 +505,7 @@ template <int D, class E>
 hipError_t launch_bwd_dkdv(const BwdIO& io, const BwdWork& ws, const BwdPass& pass,
                            const DkdvSplit& kvs, int BH, int H, int T, hipStream_t stream) {
   // the single-buffered variant wherever it is built
-  auto kernel = ca_bwd_dkdv_kernel<D, E, dkdv_has_single_buffer<D, E>()>;
+  auto kernel = ca_bwd_dkdv_kernel<D, E, (D >= 32)>;
   hipLaunchKernelGGL(kernel, dim3(kvs.items * BH), dim3(256), 0, stream, io.k,
                      io.v, io.rope, io.k_rotated ? nullptr : io.rope, ws.limbs, ws.qstat,
                      io.log_gain, io.dk, io.dv, ws.dsbuf,

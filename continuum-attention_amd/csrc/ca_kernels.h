@@ -495,6 +495,13 @@ __host__ __device__ inline int bwd_pass_tiles(const BwdPass& p) { return p.qb - 
 // the reference rounds it; value_limbs of them), then the three dY/Z limbs.
 // Workspaces are sized for six planes.
 template <class E> __host__ __device__ constexpr int q_limb_planes() { return value_limbs<E>(); }
+// The dK/dV kernel's waves per SIMD, by head dim and q_limb_planes: what its
+// registers are bounded for and what its split lengths count on.  bf16 (fewer
+// limb registers), and fp16 at D < 32, fit four (128 VGPRs); other operands
+// three (168); D = 128 two.
+__host__ __device__ constexpr int dkdv_waves_per_simd(int D, int planes) {
+  return D > 64 ? 2 : planes == 1 || (planes == 2 && D < 32) ? 4 : 3;
+}
 // Keys of a slice, evenly spread, whose mean serves as its typical key in the
 // gain gradient.
 constexpr int kGainRefs = 4;
