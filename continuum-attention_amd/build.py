@@ -130,13 +130,13 @@ def build(verbose: bool = False, extra_flags=None) -> str:
             if verbose and out.strip():
                 print(out, flush=True)
             objs.append(obj)
-        ext.result()
     tmp = LIB + ".tmp"
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}{res.stderr}")
     os.replace(tmp, LIB)
+    ext.result()  # the C library stands also where g++ or torch's headers are missing
     link_torch_ext(ext_obj, verbose)
     return LIB
 

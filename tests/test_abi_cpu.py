@@ -334,3 +334,27 @@ def test_native_functions_raise_the_librarys_errors(ca):
         with pytest.raises(native.CAError) as e:
             ext.check(rc)
         assert e.value.code == rc and "continuum-attention_amd: " in str(e.value)
+
+
+def test_c_library_is_built_without_the_torch_binding(monkeypatch, tmp_path):
+    """Where the torch binding cannot be compiled the build says so, after
+    writing the C library, which needs hipcc alone."""
+    import importlib.util
+    import shutil
+    spec = importlib.util.spec_from_file_location(
+        "ca_build", os.path.join(ROOT, "continuum-attention_amd", "build.py"))
+    b = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(b)
+    if shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"):
+        pytest.skip("no hipcc")
+
+    def no_headers(obj, verbose):
+        raise RuntimeError("g++ on ca_torch.cpp failed")
+
+    monkeypatch.setattr(b, "compile_torch_ext", no_headers)
+    monkeypatch.setattr(b, "SOURCES", ["ca_swiglu.hip"])
+    monkeypatch.setattr(b, "HERE", str(tmp_path))
+    monkeypatch.setattr(b, "LIB", str(tmp_path / "lib.so"))
+    with pytest.raises(RuntimeError, match="ca_torch.cpp"):
+        b.build()
+    assert (tmp_path / "lib.so").exists()
