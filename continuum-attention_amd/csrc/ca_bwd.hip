@@ -14,12 +14,13 @@
 //   ca_bwd_dkdv     (ca_bwd_dkdv.hip) one work group per (slice, 56 keys); wave w owns 14 keys
 //                   (16 MFMA slots).  The 4 waves walk the query tiles
 //                   together: each 32-query tile of Q and dY/Z limbs is staged
-//                   once in LDS (double-buffered) and read by every wave both
+//                   once in LDS (double-buffered below D = 32) and read by every wave both
 //                   row-wise (S = Q K^T, dP' = (dY/Z) V^T) and transposed
 //                   (dV^T += (dY/Z)^T W, dK^T += Q^T dS) with
 //                   ds_read_b64_tr_b16.  K and V of the wave's slots stay in
 //                   registers as bf16 limbs for the whole launch.  All four
-//                   products are bf16x6 on v_mfma_f32_16x16x32_bf16.  dS of
+//                   products are limb products (six for fp32 values, fewer
+//                   with 16-bit Q, K or V) on v_mfma_f32_16x16x32_bf16.  dS of
 //                   the owned keys is also spilled, one 32-query column per
 //                   (query tile, key), for the dQ pass.
 //                   Each item also forms its gain partial
@@ -35,10 +36,11 @@
 // Score-tile layout in ca_bwd_dkdv: the 16x16 result of S / dP' puts slot j
 // (key 14*kb - 1 + j) in lane j of each 16-lane row and queries 4*(l/16) + r
 // in its registers, so the two neighbours of a segment sit in adjacent lanes
-// of one DPP row (row_shr / row_shl).  p = 2^(s - m) stays unnormalised and
-// dY arrives pre-scaled by 1/Z, so the weight gradient g = dY.v/Z - Dl/Z comes
-// straight out of the MFMA (its accumulator starts at -Dl/Z) and dV = W^T dY
-// is formed as w^T (dY/Z) with no per-row scaling in the kernel.
+// of one DPP row (row_shr / row_shl).  p = 2^(s - m - kShareShift) stays
+// unnormalised and dY arrives pre-scaled by 1/Z, so the weight gradient
+// g = dY.v/Z - Dl/Z comes straight out of the MFMA (its accumulator starts at
+// +Dl/Z and changes sign halfway, see kDpFlip) and dV = W^T dY is formed as
+// w^T (dY/Z) with no per-row scaling in the kernel.
 #include <type_traits>
 
 #include "ca_common.h"

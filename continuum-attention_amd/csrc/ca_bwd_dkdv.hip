@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256, dkdv_waves_per_simd(D, q_limb_planes<E>())) vo
   }
 
   // ---- query-tile staging (all waves), one tile ahead ----
-  // Tile qt of the pass is one contiguous block of six limb planes [32][D]
+  // Tile qt of the pass is one contiguous block of P::PLANES limb planes [32][D]
   // (rows past T are zero) and 32 row statistics: thread tid copies 16-byte
   // chunks tid + 256u of the block, so the only per-tile address work is the
   // uniform block base.

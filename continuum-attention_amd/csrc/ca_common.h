@@ -3,9 +3,9 @@
 // Segment math
 // ------------
 // A segment joins two adjacent keys (left l, right r) of one query row.  The
-// kernels keep scores in log2 units relative to the row shift m (q is
-// pre-scaled by c_h*log2(e) and -m rides in the MFMA accumulator), so the
-// endpoint weights are p = 2^s and the signed natural difference is
+// kernels keep scores in log2 units relative to the row shift m (one fused
+// multiply-add after the product: s = c_h log2(e) q.k - m), so the endpoint
+// weights are p = 2^s and the signed natural difference is
 // x = (s_r - s_l) * ln2.  With J_n(x) = int_0^1 u^n e^{x u} du the
 // reference's segment terms (architecture.py:32-62,91-96;
 // analytic_reference.py:12-75, there written with shifted moments of |x|) are
@@ -29,8 +29,11 @@
 // serves both shares.  The polynomial coefficients are fitted (weighted least
 // squares with Lawson reweighting toward minimax relative error) on
 // [-0.5, 0.5] with quadratic E and O: max relative error 1.7e-7 (J1) and
-// 2.2e-7 (J2) in exact arithmetic, about float32 resolution.  tests/test_device_math.py re-checks these
-// constants and formulas in float32 against the float64 oracle.
+// 2.2e-7 (J2) in exact arithmetic, about float32 resolution.  These one-sided
+// forms serve the three-pass row kernel; the fused kernels and the register row
+// kernel use the symmetric forms further below.  tests/test_device_math.py and
+// tests/test_device_math_symmetric.py re-check the constants and formulas in
+// float32 against the float64 oracle.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -490,7 +493,7 @@ __device__ __forceinline__ void seg_shares_grad_x(float x, float pl, float pr, f
 // For |h| < kHalfSeriesT the quotients cancel; there dp = S tanh h gives
 // d = dp C(h^2) with the even function C(y) = (coth h - 1/h) / h, and from it
 // a = S - h d and b = a C: one quadratic polynomial (minimax relative error
-// 1.3e-7 on the range) serves all three.  20 VALU instructions per segment
+// 1.5e-7 on the range) serves all three.  20 VALU instructions per segment
 // for L and R and 27 with the gradients (against 21 and 36 for the one-sided
 // closed forms above), and half their rounding error: the series stays
 // accurate to a larger |h|, so the quotients start where they cancel less.

@@ -166,7 +166,11 @@ __global__ __launch_bounds__(256) void ca_weights_rows_kernel(
 // rows 16-byte misaligned (K = 1023) 42.6 -> 34.3 and 53.9 -> 40.2 us.  Rows
 // of at most kRowShort keys, which would leave three quarters of the lanes
 // idle, stay with the three-pass kernel (one key per lane; at 256 matrices of
-// [64, 64] backward 12.2 against 14.1 us), and so do rows past 2048 keys.
+// [64, 64] backward 12.2 against 14.1 us), and so do rows past 2048 keys.  From
+// 65 keys on, where the three-pass kernel needs a second step, this one is the
+// faster: 2^26 scores in rows of 65 keys 391 / 489 -> 374 / 481 us (three-pass /
+// this one, forward / backward), 96 keys 310 / 389 -> 265 / 322, 128 keys
+// 296 / 391 -> 208 / 255, 2048 keys 176 / 241 -> 76 / 114.
 constexpr int kRowRegChunk = 256;
 constexpr int kRowShort = 64;
 template <bool kBwd, int NC, bool VEC>
