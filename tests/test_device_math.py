@@ -1,6 +1,7 @@
-"""Pins the HIP kernels' segment math on the CPU.
+"""Pins the one-sided segment math of the three-pass row kernel on the CPU (the
+symmetric form of the other kernels: tests/test_device_math_symmetric.py).
 
-The device functions seg_shares / seg_shares_grad (csrc/ca_common.h) are
+The device functions seg_shares_x / seg_shares_grad_x (csrc/ca_common.h) are
 re-evaluated here in float32 numpy, with the polynomial constants parsed from
 the header itself, and compared with the float64 oracle's segment terms
 (oracle/ca_oracle.py: shifted moments, analytic_reference.py:12-75).  A wrong
