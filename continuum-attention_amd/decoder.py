@@ -256,7 +256,11 @@ def _kept_table(cache, key, device, build):
     ``key``, ready for work queued on the current stream."""
     entry = cache.get(key)
     if device.type == "cuda":
-        if torch.cuda.is_current_stream_capturing():
+        capturing = torch.cuda.is_current_stream_capturing()
+        if (entry is not None and entry.written and not capturing
+                and _native.stream_handle(device) in entry.readers):
+            return entry.tensors
+        if capturing:
             if entry is None or not entry.written:
                 return build()
             entry.captured = True

@@ -32,6 +32,7 @@ def fake(ca, monkeypatch):
     st = types.SimpleNamespace(stream=_Stream(1), capturing=False, noted=[], event=_Event)
     monkeypatch.setattr(_Event, "done", False)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: st.stream)
+    monkeypatch.setattr(ca.native, "stream_handle", lambda device: st.stream.cuda_stream)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: st.capturing)
     monkeypatch.setattr(torch.cuda, "Event", _Event)
     monkeypatch.setattr(torch.Tensor, "record_stream",
