@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the Continuum Attention operator on one MI355X.
 
-Workload (BASELINE.json configs[1]): the isolated CA operator at
+Workload: the isolated CA operator at
 [B,H,T,D] = [2,16,2048,64] fp32, forward + backward, causal full context,
 Q,K,V ~ N(0,1) with the op's own 1/sqrt(64) scale, log_gain = 0 (tau = 1),
 upstream grad ~ N(0,1), seed 0.  One "step" is one forward + backward of the

@@ -28,7 +28,7 @@ HIPCC_FLAGS = [
     "-fPIC",
     "-ffp-contract=fast",
     # packed fp32 VALU forms are disabled: some of them have returned wrong
-    # results on this GPU pool with no error
+    # results on this GPU with no error
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     # keep MFMA accumulators in VGPRs: the dK/dV kernel otherwise shuffles
     # loop-carried tiles between AGPRs every iteration (~100 moves per tile)

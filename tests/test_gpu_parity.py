@@ -143,9 +143,9 @@ def test_head_dims(gpu_ca, D):
                                              (4, 33, 7, torch.float32), (128, 1, 64, torch.float32),
                                              (128, 130, 37, torch.bfloat16)])
 def test_any_head_dim_query_tiles(gpu_ca, D, T, tile, dtype):
-    """Head dims without fused kernels (80, 96, 48, 24, 4) run the
-    reference's query-tile structure on the device (fp32 GEMMs + the HIP
-    weight kernels); D = 128 runs the fused kernels.  Outputs and all four
+    """Head dims without kernels of their own: 80, 96, 48 and 24 run the fused
+    kernels on zero-padded rows, 4 the reference's query-tile structure on the
+    device (fp32 GEMMs + the HIP weight kernels); D = 128 runs the fused kernels.  Outputs and all four
     gradients against the oracle, across tile boundaries and a tile that does
     not divide T, nonzero gains, and bf16 inputs."""
     say(f"[case] any head dim D={D} T={T} query_tile={tile} {dtype}")
